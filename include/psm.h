@@ -102,6 +102,7 @@ typedef struct psm_sigma {
 #define PSM_SCAN_TEAM 0x100
 #define PSM_SCAN_HALF 0x200
 #define PSM_SCAN_QUAD 0x400
+#define PSM_SCAN_ROW 0x800
 #define PSM_SCAN_TOP_SHIFT 16
 #define PSM_SCAN_TOP_MASK 0xff0000
 
@@ -123,17 +124,21 @@ typedef struct psm_problem {
    * once per recomputation; the caller zeroes it. */
   float fallback_ratio;
   /* bits 0-7: scan items folded per lane (0: the PSM_SCAN_K environment
-   * variable, else 2 with team-cooperative upper levels and 4 without);
-   * PSM_SCAN_TEAM: levels above the first run team-cooperative kernels
+   * variable, else 2 with 16-lane upper levels and 4 without);
+   * PSM_SCAN_TEAM: levels above the first run 16 lanes per combination
    * (square-root form, float / double); with bits 0-7 clear they do so by
    * default, unless the PSM_SCAN_TEAM environment variable is 0;
    * PSM_SCAN_HALF: level 0 of the scan runs 32-lane workgroups (square-root
    * form, float / double): twice the workgroups, half the LDS each, one
    * scan-over-lanes step less;
-   * PSM_SCAN_QUAD: level 0 of the scan runs quad-cooperative kernels (four
-   * lanes per combination, 64 or, with PSM_SCAN_HALF, 32 quads per
-   * workgroup; square-root form, float / double): the level layout is the
-   * same, each combination's chain of dependent operations about a third;
+   * PSM_SCAN_QUAD: level 0 of the scan runs four lanes per combination, 64 or,
+   * with PSM_SCAN_HALF, 32 combinations per workgroup (square-root form,
+   * float / double): the level layout is the same, each combination's chain
+   * of dependent operations about a third;
+   * PSM_SCAN_ROW: level 0 of the scan runs 16 lanes per combination, 16
+   * combinations per workgroup (square-root form, float / double; it takes
+   * precedence over PSM_SCAN_QUAD and PSM_SCAN_HALF): the shortest chain, for
+   * the few items of a short sequence;
    * bits 16-23 (PSM_SCAN_TOP_MASK): a level whose items fit one workgroup
    * with at most this many items per lane is the top level (values below the
    * fan-in, 0 included, mean the fan-in) */
@@ -414,7 +419,8 @@ int psm_math_check(int64_t n, const double* x, double* out_rcp, double* out_sqrt
  * schedules whose workspace fits workspace_bytes: first chunk in {2, 4, 8, 16,
  * 32} states per lane x scan fan-in scan_k in {2, 4, 8}, with and without
  * PSM_SCAN_TEAM and PSM_SCAN_HALF, and with PSM_SCAN_TEAM | PSM_SCAN_QUAD
- * with and without PSM_SCAN_HALF (square-root form in float / double); then
+ * with and without PSM_SCAN_HALF, and with PSM_SCAN_TEAM | PSM_SCAN_ROW at
+ * fan-in 1 and 2 (square-root form in float / double); then
  * the chunks at 5/8 .. 7/4 of the best chunk (those that are not powers of
  * two, at most 64) with the three best scan_k values.  Returns the fastest in
  * *best_chunk / *best_scan_k (and its time per pass in *best_ms, may be

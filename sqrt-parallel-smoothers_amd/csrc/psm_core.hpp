@@ -60,7 +60,17 @@ struct SAgg {
 };
 
 // ---------------------------------------------------------------- SoA load / store
-// Component q of item i lives at base[q * stride + i].
+// Component q of item i lives at base[q * stride + i].  The workspace's buffers
+// hold their items in blocks of kBlk positions, the NQ components of a block one
+// after the other (blk): one component of 64 consecutive positions is 64
+// consecutive words, the components of an item lie within one block (a few KB
+// apart at fixed offsets, which fit the instructions' immediate offsets, instead
+// of one far-away stream each), and kBlk is the component stride.
+constexpr int kBlk = 64;
+template <int NQ, typename R>
+PSM_DEV R* blk(R* base, int64_t pos) {
+  return base + (pos >> 6) * (int64_t)(NQ * kBlk) + (pos & 63);
+}
 template <typename R, int N>
 PSM_DEV void ld(const R* __restrict__ base, int64_t stride, int64_t i, int& q, R (&v)[N]) {
 #pragma unroll
@@ -108,55 +118,61 @@ PSM_DEV void ld_tri(const R* __restrict__ base, int64_t stride, int64_t i, int& 
 }
 
 template <bool SYM, typename R, int NX, int NY>
-PSM_DEV void load_trans(const R* base, int64_t stride, int64_t i, Step<R, NX, NY>& s) {
+PSM_DEV void load_trans(const R* base, int64_t pos, Step<R, NX, NY>& s) {
+  const R* p = blk<Step<R, NX, NY>::NQ>(base, pos);
   int q = 0;
-  ld(base, stride, i, q, s.F);
-  ld_tri<SYM>(base, stride, i, q, s.cq);
-  ld(base, stride, i, q, s.bt);
+  ld(p, kBlk, 0, q, s.F);
+  ld_tri<SYM>(p, kBlk, 0, q, s.cq);
+  ld(p, kBlk, 0, q, s.bt);
 }
 template <bool SYM, typename R, int NX, int NY>
-PSM_DEV void load_obs(const R* base, int64_t stride, int64_t i, Step<R, NX, NY>& s) {
+PSM_DEV void load_obs(const R* base, int64_t pos, Step<R, NX, NY>& s) {
+  const R* p = blk<Step<R, NX, NY>::NQ>(base, pos);
   int q = Step<R, NX, NY>::NTRANS;
-  ld(base, stride, i, q, s.H);
-  ld_tri<SYM>(base, stride, i, q, s.cr);
-  ld(base, stride, i, q, s.c);
+  ld(p, kBlk, 0, q, s.H);
+  ld_tri<SYM>(p, kBlk, 0, q, s.cr);
+  ld(p, kBlk, 0, q, s.c);
 }
 
 template <typename R, int NX>
-PSM_DEV void load_agg(const R* base, int64_t stride, int64_t i, FAgg<R, NX>& a) {
+PSM_DEV void load_agg(const R* base, int64_t pos, FAgg<R, NX>& a) {
+  const R* p = blk<FAgg<R, NX>::NQ>(base, pos);
   int q = 0;
-  ld(base, stride, i, q, a.A);
-  ld(base, stride, i, q, a.b);
-  ld(base, stride, i, q, a.U);
-  ld(base, stride, i, q, a.eta);
-  ld(base, stride, i, q, a.Z);
-  a.flag = (int)base[(int64_t)q * stride + i];
+  ld(p, kBlk, 0, q, a.A);
+  ld(p, kBlk, 0, q, a.b);
+  ld(p, kBlk, 0, q, a.U);
+  ld(p, kBlk, 0, q, a.eta);
+  ld(p, kBlk, 0, q, a.Z);
+  a.flag = (int)p[q * kBlk];
 }
 template <typename R, int NX>
-PSM_DEV void store_agg(R* base, int64_t stride, int64_t i, const FAgg<R, NX>& a) {
+PSM_DEV void store_agg(R* base, int64_t pos, const FAgg<R, NX>& a) {
+  R* p = blk<FAgg<R, NX>::NQ>(base, pos);
   int q = 0;
-  st(base, stride, i, q, a.A);
-  st(base, stride, i, q, a.b);
-  st(base, stride, i, q, a.U);
-  st(base, stride, i, q, a.eta);
-  st(base, stride, i, q, a.Z);
-  base[(int64_t)q * stride + i] = R(a.flag);
+  st(p, kBlk, 0, q, a.A);
+  st(p, kBlk, 0, q, a.b);
+  st(p, kBlk, 0, q, a.U);
+  st(p, kBlk, 0, q, a.eta);
+  st(p, kBlk, 0, q, a.Z);
+  p[q * kBlk] = R(a.flag);
 }
 template <typename R, int NX>
-PSM_DEV void load_agg(const R* base, int64_t stride, int64_t i, SAgg<R, NX>& a) {
+PSM_DEV void load_agg(const R* base, int64_t pos, SAgg<R, NX>& a) {
+  const R* p = blk<SAgg<R, NX>::NQ>(base, pos);
   int q = 0;
-  ld(base, stride, i, q, a.g);
-  ld(base, stride, i, q, a.E);
-  ld(base, stride, i, q, a.D);
-  a.flag = (int)base[(int64_t)q * stride + i];
+  ld(p, kBlk, 0, q, a.g);
+  ld(p, kBlk, 0, q, a.E);
+  ld(p, kBlk, 0, q, a.D);
+  a.flag = (int)p[q * kBlk];
 }
 template <typename R, int NX>
-PSM_DEV void store_agg(R* base, int64_t stride, int64_t i, const SAgg<R, NX>& a) {
+PSM_DEV void store_agg(R* base, int64_t pos, const SAgg<R, NX>& a) {
+  R* p = blk<SAgg<R, NX>::NQ>(base, pos);
   int q = 0;
-  st(base, stride, i, q, a.g);
-  st(base, stride, i, q, a.E);
-  st(base, stride, i, q, a.D);
-  base[(int64_t)q * stride + i] = R(a.flag);
+  st(p, kBlk, 0, q, a.g);
+  st(p, kBlk, 0, q, a.E);
+  st(p, kBlk, 0, q, a.D);
+  p[q * kBlk] = R(a.flag);
 }
 
 template <typename A> struct Agg_nx;
@@ -194,50 +210,62 @@ PSM_DEV void copy_agg(const SAgg<R, NX>& s, SAgg<R, NX>& d) {
 // Square-root form
 // ============================================================================
 
+// Predicted factor and the update's array.  M = tria([F U | chol Q]) in its
+// first NX columns; then the rows [chol R | H M; 0 | M] reduced at their first
+// NY pivots: P[:NY][:NY] = chol S, P[NY:][:NY] = K chol S, and P[NY:][NY:] a
+// square root of the updated covariance, triangularised last.  The pivots touch
+// the columns that can be non-zero only (chol Q and M are lower triangular).
+template <typename R, int NX, int NY>
+PSM_DEV void sqrt_update_array(const Step<R, NX, NY>& s, const R (&U)[NX][NX],
+                               R (&P)[NY + NX][NY + NX]) {
+  R M[NX][2 * NX];
+#pragma unroll
+  for (int i = 0; i < NX; ++i)
+#pragma unroll
+    for (int j = 0; j < NX; ++j) {
+      R acc = s.F[i][j] * U[j][j];
+#pragma unroll
+      for (int k = j + 1; k < NX; ++k) acc = fma(s.F[i][k], U[k][j], acc);
+      M[i][j] = acc;
+      M[i][NX + j] = s.cq[i][j];
+    }
+  tria_lower_inplace<NX>(M);
+#pragma unroll
+  for (int i = 0; i < NY; ++i) {
+#pragma unroll
+    for (int j = 0; j < NY; ++j) P[i][j] = s.cr[i][j];
+#pragma unroll
+    for (int j = 0; j < NX; ++j) {
+      R acc = s.H[i][j] * M[j][j];
+#pragma unroll
+      for (int k = j + 1; k < NX; ++k) acc = fma(s.H[i][k], M[k][j], acc);
+      P[i][NY + j] = acc;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NX; ++i) {
+#pragma unroll
+    for (int j = 0; j < NY; ++j) P[NY + i][j] = R(0);
+#pragma unroll
+    for (int j = 0; j < NX; ++j) P[NY + i][NY + j] = M[i][j];
+  }
+  tria_inplace<R, NY + NX, NY + NX>(P);
+}
+
 // Predict + update of a distribution (m, L) with one step (sequential sqrt
-// Kalman filter, parsmooth/sequential/_filtering.py:80-108).  Returns the
-// log-likelihood increment (FP64) of parsmooth/_utils.py:152-160 evaluated at
-// the innovation factor, which is what parsmooth/parallel/_filtering.py:149-154
-// computes from the filtered state of the previous step.
+// Kalman filter, parsmooth/sequential/_filtering.py:80-108).  L is lower
+// triangular.  Returns the log-likelihood increment (FP64) of
+// parsmooth/_utils.py:152-160 evaluated at the innovation factor, which is what
+// parsmooth/parallel/_filtering.py:149-154 computes from the filtered state of
+// the previous step.
 template <typename R, int NX, int NY>
 PSM_DEV typename AccOf<R>::type sqrt_kf_step(const Step<R, NX, NY>& s, const R (&y)[NY], R (&m)[NX], R (&L)[NX][NX]) {
   R m1[NX];
   mv(s.F, m, m1);
 #pragma unroll
   for (int i = 0; i < NX; ++i) m1[i] += s.bt[i];
-  R M[NX][2 * NX];
-#pragma unroll
-  for (int i = 0; i < NX; ++i)
-#pragma unroll
-    for (int j = 0; j < NX; ++j) {
-      R acc = R(0);
-#pragma unroll
-      for (int k = 0; k < NX; ++k) acc = fma(s.F[i][k], L[k][j], acc);
-      M[i][j] = acc;
-      M[i][NX + j] = s.cq[i][j];
-    }
-  tria_inplace<R, NX, 2 * NX>(M);
-  R P[NY + NX][NX + NY];
-#pragma unroll
-  for (int i = 0; i < NY; ++i) {
-#pragma unroll
-    for (int j = 0; j < NX; ++j) {
-      R acc = R(0);
-#pragma unroll
-      for (int k = 0; k < NX; ++k) acc = fma(s.H[i][k], M[k][j], acc);
-      P[i][j] = acc;
-    }
-#pragma unroll
-    for (int j = 0; j < NY; ++j) P[i][NX + j] = s.cr[i][j];
-  }
-#pragma unroll
-  for (int i = 0; i < NX; ++i) {
-#pragma unroll
-    for (int j = 0; j < NX; ++j) P[NY + i][j] = M[i][j];
-#pragma unroll
-    for (int j = 0; j < NY; ++j) P[NY + i][NX + j] = R(0);
-  }
-  tria_inplace<R, NY + NX, NX + NY>(P);
+  R P[NY + NX][NY + NX];
+  sqrt_update_array(s, L, P);
   // innovation v = y - H m1 - c ; w = P11^{-1} v
   R w[NY];
   using Acc = typename AccOf<R>::type;
@@ -268,7 +296,7 @@ PSM_DEV typename AccOf<R>::type sqrt_kf_step(const Step<R, NX, NY>& s, const R (
 // Absorb one more step into a filter aggregate: agg <- agg (+) element(step).
 // Same conditional + likelihood algebra as the operator, specialised to a
 // right operand that is a single step, which needs no 2nx x 2nx
-// triangularisation.
+// triangularisation.  a.U and a.Z are lower triangular.
 template <typename R, int NX, int NY>
 PSM_DEV void sqrt_absorb(FAgg<R, NX>& a, const Step<R, NX, NY>& s, const R (&y)[NY]) {
   // predict: A1 = F A, b1 = F b + bt, U1 = tria([F U | cq])
@@ -277,39 +305,8 @@ PSM_DEV void sqrt_absorb(FAgg<R, NX>& a, const Step<R, NX, NY>& s, const R (&y)[
   mv(s.F, a.b, b1);
 #pragma unroll
   for (int i = 0; i < NX; ++i) b1[i] += s.bt[i];
-  R M[NX][2 * NX];
-#pragma unroll
-  for (int i = 0; i < NX; ++i)
-#pragma unroll
-    for (int j = 0; j < NX; ++j) {
-      R acc = R(0);
-#pragma unroll
-      for (int k = 0; k < NX; ++k) acc = fma(s.F[i][k], a.U[k][j], acc);
-      M[i][j] = acc;
-      M[i][NX + j] = s.cq[i][j];
-    }
-  tria_inplace<R, NX, 2 * NX>(M);
-  R P[NY + NX][NX + NY];
-#pragma unroll
-  for (int i = 0; i < NY; ++i) {
-#pragma unroll
-    for (int j = 0; j < NX; ++j) {
-      R acc = R(0);
-#pragma unroll
-      for (int k = 0; k < NX; ++k) acc = fma(s.H[i][k], M[k][j], acc);
-      P[i][j] = acc;
-    }
-#pragma unroll
-    for (int j = 0; j < NY; ++j) P[i][NX + j] = s.cr[i][j];
-  }
-#pragma unroll
-  for (int i = 0; i < NX; ++i) {
-#pragma unroll
-    for (int j = 0; j < NX; ++j) P[NY + i][j] = M[i][j];
-#pragma unroll
-    for (int j = 0; j < NY; ++j) P[NY + i][NX + j] = R(0);
-  }
-  tria_inplace<R, NY + NX, NX + NY>(P);
+  R P[NY + NX][NY + NX];
+  sqrt_update_array(s, a.U, P);
   // w = P11^{-1} (y - H b1 - c), G = P11^{-1} H A1
   R w[NY], G[NY][NX];
 #pragma unroll
@@ -331,7 +328,7 @@ PSM_DEV void sqrt_absorb(FAgg<R, NX>& a, const Step<R, NX, NY>& s, const R (&y)[
       G[i][col] = h * inv;
     }
   }
-  // A = A1 - P21 G ; b = b1 + P21 w ; U = P22 ; eta += G^T w ; Z = tria([Z | G^T])
+  // A = A1 - P21 G ; b = b1 + P21 w ; U = P22 ; eta += G^T w
 #pragma unroll
   for (int i = 0; i < NX; ++i) {
     R bb = b1[i];
@@ -352,128 +349,177 @@ PSM_DEV void sqrt_absorb(FAgg<R, NX>& a, const Step<R, NX, NY>& s, const R (&y)[
     for (int j = 0; j < NY; ++j) e = fma(G[j][i], w[j], e);
     a.eta[i] = e;
   }
-  R Zc[NX][NX + NY];
+  // Z = tria([G^T | Z]): row i starts with its G column and ends at Z's
+  // diagonal, so pivot i works on column i of Z and the NY columns of G^T
 #pragma unroll
   for (int i = 0; i < NX; ++i) {
+    R x[1 + NY];
+    x[0] = a.Z[i][i];
 #pragma unroll
-    for (int j = 0; j < NX; ++j) Zc[i][j] = a.Z[i][j];
+    for (int j = 0; j < NY; ++j) x[1 + j] = G[j][i];
+    const Pivot<R> pv = make_pivot(x[0], pivot_norm2<1 + NY, 0>(x, 0));
+    a.Z[i][i] = pv.nrm;
 #pragma unroll
-    for (int j = 0; j < NY; ++j) Zc[i][NX + j] = G[j][i];
+    for (int k = i + 1; k < NX; ++k) {
+      R m[1 + NY];
+      m[0] = a.Z[k][i];
+#pragma unroll
+      for (int j = 0; j < NY; ++j) m[1 + j] = G[j][k];
+      pivot_apply<1 + NY, 0>(pv, x, m, 0);
+      a.Z[k][i] = m[0];
+#pragma unroll
+      for (int j = 0; j < NY; ++j) G[j][k] = m[1 + j];
+    }
   }
-  tria_inplace<R, NX, NX + NY>(Zc);
-#pragma unroll
-  for (int i = 0; i < NX; ++i)
-#pragma unroll
-    for (int j = 0; j < NX; ++j) a.Z[i][j] = Zc[i][j];
 }
 
-// Full filtering operator out = e1 (+) e2 (parsmooth/parallel/_operators.py:43-77),
-// written with M1 = U1 Xi11^{-T} and P = I - M1 Xi21^T:
-//   A = A2 P A1, b = A2 P (b1 + U1 U1^T eta2) + b2, U = tria([A2 M1 | U2]),
-//   eta = A1^T P^T (eta2 - Z2 Z2^T b1) + eta1, Z = tria([A1^T Xi22 | Z1]).
-// out may alias e2 but not e1.
+// The filtering operator as one array of rows (parsmooth/parallel/_operators.py:43-77
+// in blocks).  With W = U1^T Z2 and w = eta2 - Z2 (Z2^T b1), an orthogonal Q that
+// makes [W | I] Q = [X | 0] (n pivots) takes
+//     [A1^T Z2 |    0   ] Q = [V^T | Y]
+//     [   0    | A2 U1  ] Q = [ S  | .]
+//     [   0    | w^T U1 ] Q = [r^T | .]
+// and the combination is
+//     A = A2 A1 - S V,              b   = A2 b1 + b2 + S r,
+//     U = tria([S | U2]),           eta = A1^T w + eta1 - V^T r,
+//     Z = tria([Y | Z1]).
+// X X^T = I + W W^T is the operator's Xi11 Xi11^T, S = A2 U1 X^-T its A2 M1,
+// Y Y^T its A1^T Xi22 Xi22^T A1: the same blocks without the second half of the
+// 2n x 2n triangularisation (any square root of Xi22 Xi22^T serves in Z), without
+// the solve for M1 and without forming P.  w is formed first: eta2 and Z2 Z2^T b1
+// are large beside their difference when b1 is, and carrying them through the
+// pivots apart costs FP32 half a digit of the mean.  Every row stays zero right
+// of column n + i until pivot i, so a pivot works on n + 1 columns.
+//
+// FilterArray holds the reduced pivot rows: row i as it was at its pivot, and
+// the pivot's scalars; reflect() takes any row [a | b] through Q.
 template <typename R, int NX>
-PSM_DEV void sqrt_combine_core(const FAgg<R, NX>& e1, const FAgg<R, NX>& e2, FAgg<R, NX>& out) {
-  R X[2 * NX][2 * NX];
-  // [[U1^T Z2, I], [Z2, 0]]
+struct FilterArray {
+  R x[NX][2 * NX];
+  Pivot<R> pv[NX];
+  // x[:, :NX] = W on entry
+  PSM_DEV void reduce() {
 #pragma unroll
-  for (int i = 0; i < NX; ++i)
+    for (int i = 0; i < NX; ++i)
 #pragma unroll
-    for (int j = 0; j < NX; ++j) {
-      R acc = R(0);
+      for (int j = 0; j < NX; ++j) x[i][NX + j] = (i == j) ? R(1) : R(0);
 #pragma unroll
-      for (int k = 0; k < NX; ++k) acc = fma(e1.U[k][i], e2.Z[k][j], acc);
-      X[i][j] = acc;
-      X[i][NX + j] = (i == j) ? R(1) : R(0);
-      X[NX + i][j] = e2.Z[i][j];
-      X[NX + i][NX + j] = R(0);
+    for (int i = 0; i < NX; ++i) {
+      pv[i] = make_pivot(x[i][i], pivot_norm2<NX, NX>(x[i], i));
+#pragma unroll
+      for (int k = i + 1; k < NX; ++k) pivot_apply<NX, NX>(pv[i], x[i], x[k], i);
     }
-  tria_inplace<R, 2 * NX, 2 * NX>(X);
-  // M1 = U1 Xi11^{-T}  (rows of U1 solved against Xi11^T from the right)
-  R M1[NX][NX];
+  }
+  PSM_DEV void reflect(R (&row)[2 * NX]) const {
+#pragma unroll
+    for (int i = 0; i < NX; ++i) pivot_apply<NX, NX>(pv[i], x[i], row, i);
+  }
+};
+
+// w = eta2 - Z2 (Z2^T b1)
+template <typename R, int NX>
+PSM_DEV void innovation(const R (&b1)[NX], const R (&eta2)[NX], const R (&Z2)[NX][NX], R (&w)[NX]) {
+  R t[NX];
 #pragma unroll
   for (int j = 0; j < NX; ++j) {
-    const R inv = rcp_(X[j][j]);
+    t[j] = Z2[j][j] * b1[j];
 #pragma unroll
-    for (int r = 0; r < NX; ++r) {
-      R s = e1.U[r][j];
-#pragma unroll
-      for (int k = 0; k < j; ++k) s = fma(-M1[r][k], X[j][k], s);
-      M1[r][j] = s * inv;
-    }
+    for (int k = j + 1; k < NX; ++k) t[j] = fma(Z2[k][j], b1[k], t[j]);
   }
-  // P = I - M1 Xi21^T
-  R Pm[NX][NX];
-#pragma unroll
-  for (int i = 0; i < NX; ++i)
-#pragma unroll
-    for (int j = 0; j < NX; ++j) {
-      R acc = (i == j) ? R(1) : R(0);
-#pragma unroll
-      for (int k = 0; k < NX; ++k) acc = fma(-M1[i][k], X[NX + j][k], acc);
-      Pm[i][j] = acc;
-    }
-  // v = b1 + U1 (U1^T eta2) ; w = eta2 - Z2 (Z2^T b1)
-  R t1[NX], t2[NX], v[NX], w[NX];
-  mTv(e1.U, e2.eta, t1);
-  mTv(e2.Z, e1.b, t2);
 #pragma unroll
   for (int i = 0; i < NX; ++i) {
-    R a1 = e1.b[i], a2 = e2.eta[i];
+    w[i] = eta2[i];
 #pragma unroll
-    for (int k = 0; k < NX; ++k) {
-      a1 = fma(e1.U[i][k], t1[k], a1);
-      a2 = fma(-e2.Z[i][k], t2[k], a2);
-    }
-    v[i] = a1;
-    w[i] = a2;
+    for (int k = 0; k <= i; ++k) w[i] = fma(-Z2[i][k], t[k], w[i]);
   }
-  // PA1 = P A1, Pv = P v, PTw = P^T w
-  R PA1[NX][NX], Pv[NX], PTw[NX];
-  mm(Pm, e1.A, PA1);
-  mv(Pm, v, Pv);
-  mTv(Pm, w, PTw);
-  // eta = A1^T PTw + eta1
-  R eta[NX];
+}
+// [0 | w^T U1]
+template <typename R, int NX>
+PSM_DEV void innovation_row(const R (&U1)[NX][NX], const R (&w)[NX], R (&row)[2 * NX]) {
 #pragma unroll
-  for (int i = 0; i < NX; ++i) {
-    R acc = e1.eta[i];
+  for (int j = 0; j < NX; ++j) {
+    R acc = U1[j][j] * w[j];
 #pragma unroll
-    for (int k = 0; k < NX; ++k) acc = fma(e1.A[k][i], PTw[k], acc);
-    eta[i] = acc;
+    for (int k = j + 1; k < NX; ++k) acc = fma(U1[k][j], w[k], acc);
+    row[j] = R(0);
+    row[NX + j] = acc;
   }
-  // Z = tria([A1^T Xi22 | Z1])
-  R Zc[NX][2 * NX];
+}
+
+// out = e1 (+) e2; U and Z of both operands lower triangular.  out may alias e2
+// but not e1.
+template <typename R, int NX>
+PSM_DEV void sqrt_combine_core(const FAgg<R, NX>& e1, const FAgg<R, NX>& e2, FAgg<R, NX>& out) {
+  FilterArray<R, NX> q;
 #pragma unroll
   for (int i = 0; i < NX; ++i)
 #pragma unroll
     for (int j = 0; j < NX; ++j) {
       R acc = R(0);
 #pragma unroll
-      for (int k = j; k < NX; ++k) acc = fma(e1.A[k][i], X[NX + k][NX + j], acc);
-      Zc[i][j] = acc;
+      for (int k = (i > j ? i : j); k < NX; ++k) acc = fma(e1.U[k][i], e2.Z[k][j], acc);
+      q.x[i][j] = acc;
+    }
+  q.reduce();
+  R w[NX], r[2 * NX];
+  innovation(e1.b, e2.eta, e2.Z, w);
+  innovation_row(e1.U, w, r);
+  q.reflect(r);
+  R Zc[NX][2 * NX], Vt[NX][NX], eta[NX];
+#pragma unroll
+  for (int i = 0; i < NX; ++i) {
+    R row[2 * NX];
+    R h = e1.eta[i];
+#pragma unroll
+    for (int j = 0; j < NX; ++j) {
+      R acc = R(0);
+#pragma unroll
+      for (int k = j; k < NX; ++k) acc = fma(e1.A[k][i], e2.Z[k][j], acc);
+      row[j] = acc;
+      row[NX + j] = R(0);
+      h = fma(e1.A[j][i], w[j], h);
+    }
+    q.reflect(row);
+#pragma unroll
+    for (int j = 0; j < NX; ++j) {
+      Vt[i][j] = row[j];
+      Zc[i][j] = row[NX + j];
       Zc[i][NX + j] = e1.Z[i][j];
+      h = fma(-row[j], r[j], h);
     }
-  // U = tria([A2 M1 | U2])
-  R Uc[NX][2 * NX];
+    eta[i] = h;
+  }
+  tria_lower_inplace<NX>(Zc);
+  R Uc[NX][2 * NX], A[NX][NX], b[NX];
 #pragma unroll
-  for (int i = 0; i < NX; ++i)
+  for (int i = 0; i < NX; ++i) {
+    R row[2 * NX];
+    R bb = e2.b[i];
 #pragma unroll
     for (int j = 0; j < NX; ++j) {
       R acc = R(0);
 #pragma unroll
-      for (int k = 0; k < NX; ++k) acc = fma(e2.A[i][k], M1[k][j], acc);
-      Uc[i][j] = acc;
-      Uc[i][NX + j] = e2.U[i][j];
+      for (int k = j; k < NX; ++k) acc = fma(e2.A[i][k], e1.U[k][j], acc);
+      row[j] = R(0);
+      row[NX + j] = acc;
+      bb = fma(e2.A[i][j], e1.b[j], bb);
     }
-  // A = A2 PA1 ; b = A2 Pv + b2
-  R A[NX][NX], b[NX];
-  mm(e2.A, PA1, A);
-  mv(e2.A, Pv, b);
+    q.reflect(row);
 #pragma unroll
-  for (int i = 0; i < NX; ++i) b[i] += e2.b[i];
-  tria_inplace<R, NX, 2 * NX>(Uc);
-  tria_inplace<R, NX, 2 * NX>(Zc);
+    for (int j = 0; j < NX; ++j) {
+      R acc = R(0);
+#pragma unroll
+      for (int k = 0; k < NX; ++k) acc = fma(e2.A[i][k], e1.A[k][j], acc);
+#pragma unroll
+      for (int k = 0; k < NX; ++k) acc = fma(-row[k], Vt[j][k], acc);
+      A[i][j] = acc;
+      Uc[i][j] = row[j];
+      Uc[i][NX + j] = e2.U[i][j];
+      bb = fma(row[j], r[j], bb);
+    }
+    b[i] = bb;
+  }
+  tria_lower_inplace<NX>(Uc);
 #pragma unroll
   for (int i = 0; i < NX; ++i) {
     out.b[i] = b[i];
@@ -497,39 +543,8 @@ PSM_DEV void sqrt_filter_element(const Step<R, NX, NY>& s, const R (&m)[NX], con
   mv(s.F, m, m1);
 #pragma unroll
   for (int i = 0; i < NX; ++i) m1[i] += s.bt[i];
-  R M[NX][2 * NX];
-#pragma unroll
-  for (int i = 0; i < NX; ++i)
-#pragma unroll
-    for (int j = 0; j < NX; ++j) {
-      R acc = R(0);
-#pragma unroll
-      for (int k = 0; k < NX; ++k) acc = fma(s.F[i][k], L[k][j], acc);
-      M[i][j] = acc;
-      M[i][NX + j] = s.cq[i][j];
-    }
-  tria_inplace<R, NX, 2 * NX>(M);
-  R P[NY + NX][NX + NY];
-#pragma unroll
-  for (int i = 0; i < NY; ++i) {
-#pragma unroll
-    for (int j = 0; j < NX; ++j) {
-      R acc = R(0);
-#pragma unroll
-      for (int k = 0; k < NX; ++k) acc = fma(s.H[i][k], M[k][j], acc);
-      P[i][j] = acc;
-    }
-#pragma unroll
-    for (int j = 0; j < NY; ++j) P[i][NX + j] = s.cr[i][j];
-  }
-#pragma unroll
-  for (int i = 0; i < NX; ++i) {
-#pragma unroll
-    for (int j = 0; j < NX; ++j) P[NY + i][j] = M[i][j];
-#pragma unroll
-    for (int j = 0; j < NY; ++j) P[NY + i][NX + j] = R(0);
-  }
-  tria_inplace<R, NY + NX, NX + NY>(P);
+  R P[NY + NX][NY + NX];
+  sqrt_update_array(s, L, P);
   R HF[NY][NX];
   mm(s.H, s.F, HF);
   // G = P11^{-1} HF ; w1 = P11^{-1}(y - H m1 - c) ; w2 = P11^{-1}(y - H bt - c)
@@ -603,15 +618,23 @@ PSM_DEV void sqrt_smoother_element(const R (&F)[NX][NX], const R (&cq)[NX][NX], 
   for (int i = 0; i < NX; ++i)
 #pragma unroll
     for (int j = 0; j < NX; ++j) {
-      R acc = R(0);
+      R acc = F[i][j] * L[j][j];
 #pragma unroll
-      for (int k = 0; k < NX; ++k) acc = fma(F[i][k], L[k][j], acc);
+      for (int k = j + 1; k < NX; ++k) acc = fma(F[i][k], L[k][j], acc);
       X[i][j] = acc;
       X[i][NX + j] = cq[i][j];
       X[NX + i][j] = L[i][j];
       X[NX + i][NX + j] = R(0);
     }
-  tria_inplace<R, 2 * NX, 2 * NX>(X);
+  // the pivots of [F L | cq] work on the n + 1 columns that can be non-zero;
+  // what they leave right of column n in the lower rows is then triangularised
+  tria_pivots<NX, NX, NX>(X);
+  R D[NX][NX];
+#pragma unroll
+  for (int i = 0; i < NX; ++i)
+#pragma unroll
+    for (int j = 0; j < NX; ++j) D[i][j] = X[NX + i][NX + j];
+  tria_inplace<R, NX, NX>(D);
   // E = Phi21 Phi11^{-1}: E Phi11 = Phi21, solved column by column from the right
 #pragma unroll
   for (int jj = 0; jj < NX; ++jj) {
@@ -636,7 +659,7 @@ PSM_DEV void sqrt_smoother_element(const R (&F)[NX][NX], const R (&cq)[NX][NX], 
     for (int k = 0; k < NX; ++k) acc = fma(-out.E[i][k], p[k], acc);
     out.g[i] = acc;
 #pragma unroll
-    for (int j = 0; j < NX; ++j) out.D[i][j] = X[NX + i][NX + j];
+    for (int j = 0; j < NX; ++j) out.D[i][j] = D[i][j];
   }
   out.flag = FLAG_NORMAL;
 }
@@ -659,7 +682,7 @@ PSM_DEV void sqrt_smoother_combine_core(const SAgg<R, NX>& e1, SAgg<R, NX>& e2) 
       M[i][j] = acc;
       M[i][NX + j] = e2.D[i][j];
     }
-  tria_inplace<R, NX, 2 * NX>(M);
+  tria_lower_inplace<NX>(M);
 #pragma unroll
   for (int i = 0; i < NX; ++i) {
     e2.g[i] += g[i];
@@ -682,13 +705,13 @@ PSM_DEV void sqrt_smoother_apply(const SAgg<R, NX>& e, R (&m)[NX], R (&Ds)[NX][N
   for (int i = 0; i < NX; ++i)
 #pragma unroll
     for (int j = 0; j < NX; ++j) {
-      R acc = R(0);
+      R acc = e.E[i][j] * Ds[j][j];
 #pragma unroll
-      for (int k = 0; k < NX; ++k) acc = fma(e.E[i][k], Ds[k][j], acc);
+      for (int k = j + 1; k < NX; ++k) acc = fma(e.E[i][k], Ds[k][j], acc);
       M[i][j] = acc;
       M[i][NX + j] = e.D[i][j];
     }
-  tria_inplace<R, NX, 2 * NX>(M);
+  tria_lower_inplace<NX>(M);
 #pragma unroll
   for (int i = 0; i < NX; ++i) {
     m[i] = g[i] + e.g[i];

@@ -45,7 +45,7 @@ struct ScanLevel {
   int64_t n;      // items at this level
   int K;          // items per lane
   int64_t nwg;    // workgroups
-  int64_t stride; // padded item count (component stride of the interleaved layout)
+  int64_t stride; // padded item count
   int wg;         // lanes (or teams) per scan workgroup at this level
   size_t off_in;  // byte offsets in the workspace
   size_t off_out;
@@ -53,15 +53,15 @@ struct ScanLevel {
 
 struct Plan {
   int64_t M = 0;
-  int64_t Mp = 0;  // padded state count (component stride of the per-state buffers)
+  int64_t Mp = 0;  // padded state count of the per-state buffers
   int chunk = 0;
   int wg = 0;      // scan workgroup size
-  bool team = false;  // team-cooperative kernels above level 0
-  bool quad = false;  // quad-cooperative level-0 up-sweep
+  bool team = false;  // 16 lanes per combination above level 0
+  int lanes0 = 1;     // lanes per combination at level 0
   int64_t nchunks = 0;
   int nlevels = 0;
   ScanLevel lv[16];
-  size_t off_lin = 0, off_ell = 0, off_selem = 0, off_guard = 0, off_traj = 0, total = 0;
+  size_t off_lin = 0, off_ell = 0, off_selem = 0, off_guard = 0, off_traj = 0, off_ref = 0, total = 0;
 };
 
 // Per-workgroup flag words of the guarded second launches of the FP32
@@ -92,6 +92,10 @@ inline int default_chunk(int64_t M) {
   return c < 4 ? 4 : (c > 16 ? 16 : (int)c);
 }
 
+inline int resolve_chunk(const psm_problem_t* p) {
+  return p->chunk > 0 ? p->chunk : env_int("PSM_CHUNK", default_chunk(p->n_states), 1, 4096);
+}
+
 // wg: lanes per workgroup of level 0 (one lane per combination); wgu: lanes or
 // teams per workgroup of the levels above.
 inline Plan make_plan(const psm_problem_t* p, size_t rsize, int nlin, int nqf, int nqs,
@@ -100,7 +104,7 @@ inline Plan make_plan(const psm_problem_t* p, size_t rsize, int nlin, int nqf, i
   if (wgu <= 0) wgu = wg;
   Plan pl;
   pl.M = p->n_states;
-  pl.chunk = p->chunk > 0 ? p->chunk : env_int("PSM_CHUNK", default_chunk(pl.M), 1, 4096);
+  pl.chunk = resolve_chunk(p);
   pl.nchunks = (pl.M + pl.chunk - 1) / pl.chunk;
   pl.Mp = state_stride(pl.M, pl.chunk);
   pl.wg = wg;
@@ -134,7 +138,7 @@ inline Plan make_plan(const psm_problem_t* p, size_t rsize, int nlin, int nqf, i
       s.nwg = (n + (int64_t)wg_l * kmax - 1) / ((int64_t)wg_l * kmax);
     }
     const int64_t blk = (int64_t)wg_l * s.K;
-    s.stride = (n + blk - 1) / blk * blk;
+    s.stride = ((n + blk - 1) / blk * blk + kBlk - 1) / kBlk * kBlk;
     s.off_in = off;
     off = align_up(off + (size_t)nq * s.stride * rsize);
     s.off_out = off;
@@ -208,7 +212,7 @@ struct OpsTable {
                       const void*, const void*, const void*, void*, void*, hipStream_t);
   // the launch schedule a problem resolves to (environment defaults applied),
   // packed: chunk | level-0 fan-in << 16 | levels << 24 | team << 32 |
-  // level-0 workgroup size << 33 | quad level 0 << 49; a captured launch
+  // level-0 workgroup size << 33 | lanes per level-0 combination << 49; a captured launch
   // sequence is valid only for the same signature
   uint64_t (*plan_signature)(const psm_problem_t*);
   // reverse-mode adjoint (square-root form, float / double primal)
@@ -230,11 +234,12 @@ struct Impl {
 
   using Acc = typename AccOf<R>::type;
   // Level 0 of a scan (the chunk aggregates: many items) runs one lane per
-  // combination with WG lanes per workgroup.  The square-root form in float /
-  // double runs the levels above (few items, a latency chain) with the
-  // team-cooperative kernels, kTeamVL teams per workgroup, when scan_k has the
-  // PSM_SCAN_TEAM bit, or by default (scan_k without a fan-in; the
-  // PSM_SCAN_TEAM environment variable set to 0 turns the default off).
+  // combination with WG lanes per workgroup, or four (PSM_SCAN_QUAD) or sixteen
+  // (PSM_SCAN_ROW).  The square-root form in float / double runs the levels above
+  // (few items, a latency chain) with 16 lanes per combination, kRowVL
+  // combinations per workgroup, when scan_k has the PSM_SCAN_TEAM bit, or by
+  // default (scan_k without a fan-in; the PSM_SCAN_TEAM environment variable
+  // set to 0 turns the default off).
   static constexpr bool TEAM = SQRT && (std::is_same<R, float>::value ||
                                         std::is_same<R, double>::value);
   static constexpr int WG = scan_wg<FA, R>() < scan_wg<SA, R>() ? scan_wg<FA, R>() : scan_wg<SA, R>();
@@ -245,17 +250,49 @@ struct Impl {
     return env_int("PSM_SCAN_TEAM", 1) != 0;
   }
 
+  // Lanes per combination at level 0 and the fan-in when scan_k asks for none.
+  // A scan of n items is a chain of about log2 n combinations, whatever the
+  // schedule, so few items take the kernel with the shortest one: 16 lanes, which
+  // needs 16 n lanes (nx = 5, FP64: 2.3 us a combination against about 4 with four
+  // lanes and 9 with one).  Up to 4096 items its three levels of 16 groups hold
+  // them all without a fold (T = 4096, 10 iterations at chunk 4: 1.82 ms, 2.04 with
+  // fan-in 2, 2.11 with four lanes, 2.45 with one); up to 20,000 the fan-in of 2
+  // saves a level (T = 65,536, 4 iterations: 1.26 ms at both, 1.52 with one lane);
+  // beyond, four lanes (T = 131,072: 1.59 ms against 1.67 and 1.89; the ragged
+  // batches of 0.5 to 17 million states are 6 to 18 % faster than with one lane),
+  // 32 groups per workgroup so that three workgroups share a CU's LDS.
+  struct Level0 {
+    int lanes, wg, k;
+  };
+  static Level0 default_level0(int64_t nchunks) {
+    if (nchunks <= 4096) return Level0{16, kRowVL, 1};
+    if (nchunks <= 20000) return Level0{16, kRowVL, 2};
+    return Level0{4, WG / 2, 2};
+  }
+
   static Plan plan(const psm_problem_t* p) {
     const bool team = TEAM && team_requested(p);
     const bool half = TEAM && (p->scan_k & PSM_SCAN_HALF) != 0;
-    Plan pl = make_plan(p, sizeof(R), NLIN, FA::NQ, SA::NQ, sizeof(Acc), half ? WG / 2 : WG,
-                        team ? kTeamVL : WG, team ? 2 : 4);
+    Level0 l0{1, half ? WG / 2 : WG, team ? 2 : 4};
+    if (TEAM && (p->scan_k & PSM_SCAN_ROW)) {
+      l0.lanes = 16;
+      l0.wg = kRowVL;
+    } else if (TEAM && (p->scan_k & PSM_SCAN_QUAD)) {
+      l0.lanes = 4;
+    } else if (team && (p->scan_k & ~PSM_SCAN_TOP_MASK) == 0) {
+      const int c = resolve_chunk(p);
+      l0 = default_level0((p->n_states + c - 1) / c);
+    }
+    Plan pl = make_plan(p, sizeof(R), NLIN, FA::NQ, SA::NQ, sizeof(Acc), l0.wg, team ? kRowVL : WG, l0.k);
     pl.team = team;
-    pl.quad = TEAM && (p->scan_k & PSM_SCAN_QUAD) != 0;
+    pl.lanes0 = l0.lanes;
     // one state-interleaved trajectory (mean and factor per state) for launch
     // sequences that pass trajectories between their own passes
     pl.off_traj = pl.total;
-    pl.total = align_up(pl.total + (size_t)(NX + NX * NX) * pl.Mp * sizeof(R));
+    pl.total = align_up(pl.total + (size_t)kTrajWords<!SQRT, NX> * pl.Mp * sizeof(R));
+    // the nominal means of the centred passes
+    pl.off_ref = pl.total;
+    if (kCentred<R, SQRT>) pl.total = align_up(pl.total + (size_t)NX * pl.Mp * sizeof(R));
     return pl;
   }
 
@@ -268,7 +305,7 @@ struct Impl {
     sig |= (uint64_t)(pl.nlevels & 0xff) << 24;
     sig |= (uint64_t)(pl.team ? 1 : 0) << 32;
     sig |= (uint64_t)(pl.lv[0].wg & 0xffff) << 33;
-    sig |= (uint64_t)(pl.quad ? 1 : 0) << 49;
+    sig |= (uint64_t)(pl.lanes0 & 31) << 49;
     for (int l = 1; l < pl.nlevels; ++l) sig = sig * 1099511628211ull + (uint64_t)pl.lv[l].K;
     return sig;
   }
@@ -405,100 +442,60 @@ struct Impl {
   }
 
   // Exclusive scan of the level-0 items (chunk aggregates, already in scan
-  // order in the interleaved layout).  The level-0 down-sweep is left to the
-  // apply kernel (level0_prefix): *final_off receives the level-0 prefixes
-  // within each workgroup and *upper_off the complete level-1 prefixes
-  // (SIZE_MAX with a single level, whose prefixes are already complete).
+  // order in the interleaved layout): each level leaves its items' prefixes within
+  // their workgroups, which the apply kernel joins (enter_chunk).  lv receives
+  // the levels; rev0: the smoother's reversed level 0.
   template <typename Agg>
-  static int run_scan(const Plan& pl, char* ws, const Fallback& fb, Guards& g, hipStream_t st,
-                      size_t* final_off, size_t* upper_off) {
+  static int run_scan(const Plan& pl, char* ws, const Fallback& fb, Guards& g, hipStream_t st, int rev0,
+                      ScanLevels<R>* lv) {
     constexpr bool filt = std::is_same<Agg, FA>::value;
+    lv->n = pl.nlevels;
     for (int l = 0; l < pl.nlevels; ++l) {
       const ScanLevel& s = pl.lv[l];
       R* in = (R*)(ws + s.off_in);
       R* out = (R*)(ws + s.off_out);
+      lv->prefix[l] = out;
+      lv->span[l] = l == 0 ? 1u : lv->span[l - 1] * (uint32_t)(pl.lv[l - 1].K * pl.lv[l - 1].wg);
+      lv->map[l] = level_map(pl, l, l == 0 ? rev0 : 0);
       const bool top = l + 1 == pl.nlevels;
       R* tot = top ? nullptr : (R*)(ws + pl.lv[l + 1].off_in);
       const LevelMap tm = top ? LevelMap{0, 0, 1, WG, 0} : level_map(pl, l + 1, 0);
       TimedScope ts_(l == 0 ? (filt ? "k_fscan_up_l0" : "k_sscan_up_l0")
                             : (filt ? "k_fscan_up" : "k_sscan_up"), st);
-      // wavefronts per workgroup of the kernel this level runs
-      const int64_t wpw = (TEAM && l > 0 && pl.team) ? TeamCfg<Agg, R>::WGT / 64
-                          : (TEAM && l == 0 && pl.quad) ? (s.wg * kQuadLanes + 63) / 64
-                                                        : (s.wg + 63) / 64;
-      launch_fb(fb, g, (unsigned)s.nwg, s.nwg * wpw, [&](auto f) {
+      // lanes per combination of the kernel this level runs
+      const int lanes = !TEAM ? 1 : (l == 0 ? pl.lanes0 : (pl.team ? 16 : 1));
+      launch_fb(fb, g, (unsigned)s.nwg, s.nwg * ((s.wg * lanes + 63) / 64), [&](auto f) {
         using F = decltype(f);
-        bool launched = false;
+        auto coop = [&](auto gl, auto vl) {
+          constexpr int G = decltype(gl)::value, VL = decltype(vl)::value;
+          hipLaunchKernelGGL((k_scan_up_coop<Agg, R, G, VL, F>), dim3((unsigned)s.nwg), dim3(VL * G), 0, st,
+                             (const R*)in, level_map(pl, l, 0), out, tot, tm, f);
+        };
+        auto lane = [&](auto vl) {
+          constexpr int VL = decltype(vl)::value;
+          hipLaunchKernelGGL((k_scan_up<Agg, R, SQRT, VL, F>), dim3((unsigned)s.nwg), dim3(VL), 0, st,
+                             (const R*)in, level_map(pl, l, 0), out, tot, tm, f);
+        };
+        using I = std::integral_constant<int, WG>;
         if constexpr (TEAM) {
-          if (l > 0 && pl.team) {
-            hipLaunchKernelGGL((k_scan_up_team<Agg, R, F>), dim3((unsigned)s.nwg),
-                               dim3(TeamCfg<Agg, R>::WGT), 0, st, (const R*)in, level_map(pl, l, 0),
-                               out, tot, tm, f);
-            launched = true;
+          using H = std::integral_constant<int, WG / 2>;
+          if (lanes == 16) {
+            coop(std::integral_constant<int, 16>{}, std::integral_constant<int, kRowVL>{});
+          } else if (lanes == 4) {
+            if (s.wg == WG / 2) coop(std::integral_constant<int, 4>{}, H{});
+            else coop(std::integral_constant<int, 4>{}, I{});
+          } else if (s.wg == WG / 2) {
+            lane(H{});
+          } else {
+            lane(I{});
           }
+        } else {
+          lane(I{});
         }
-        if constexpr (TEAM) {
-          if (l == 0 && pl.quad) {
-            if (s.wg == WG / 2)
-              hipLaunchKernelGGL((k_scan_up_quad<Agg, R, WG / 2, F>), dim3((unsigned)s.nwg),
-                                 dim3(WG / 2 * kQuadLanes), 0, st, (const R*)in,
-                                 level_map(pl, l, 0), out, tot, tm, f);
-            else
-              hipLaunchKernelGGL((k_scan_up_quad<Agg, R, WG, F>), dim3((unsigned)s.nwg),
-                                 dim3(WG * kQuadLanes), 0, st, (const R*)in, level_map(pl, l, 0),
-                                 out, tot, tm, f);
-            launched = true;
-          }
-        }
-        if constexpr (TEAM) {
-          if (!launched && s.wg == WG / 2) {  // half-wave level 0
-            hipLaunchKernelGGL((k_scan_up<Agg, R, SQRT, WG / 2, F>), dim3((unsigned)s.nwg), dim3(WG / 2),
-                               0, st, (const R*)in, level_map(pl, l, 0), out, tot, tm, f);
-            launched = true;
-          }
-        }
-        if (!launched)
-          hipLaunchKernelGGL((k_scan_up<Agg, R, SQRT, WG, F>), dim3((unsigned)s.nwg), dim3(WG), 0,
-                             st, (const R*)in, level_map(pl, l, 0), out, tot, tm, f);
       });
       int rc = hip_check("k_scan_up");
       if (rc) return rc;
     }
-    // complete prefixes of level l >= 1 land in lv[l].in (free once the up-sweep is done)
-    for (int l = pl.nlevels - 2; l >= 1; --l) {
-      const ScanLevel& s = pl.lv[l];
-      const size_t upper_off =
-          (l + 1 == pl.nlevels - 1) ? pl.lv[l + 1].off_out : pl.lv[l + 1].off_in;
-      TimedScope ts_(filt ? "k_fscan_down" : "k_sscan_down", st);
-      const int64_t dwaves = (TEAM && l > 0 && pl.team)
-                                 ? s.nwg * s.K * (TeamCfg<Agg, R>::WGT / 64)
-                                 : (int64_t)grid_for(s.nwg * s.K * s.wg, WG) * ((WG + 63) / 64);
-      launch_fb(fb, g, std::max((unsigned)(s.nwg * s.K), grid_for(s.nwg * s.K * s.wg, WG)), dwaves,
-                [&](auto f) {
-        using F = decltype(f);
-        bool launched = false;
-        if constexpr (TEAM) {
-          if (l > 0 && pl.team) {
-            hipLaunchKernelGGL((k_scan_down_team<Agg, R, F>), dim3((unsigned)(s.nwg * s.K)),
-                               dim3(TeamCfg<Agg, R>::WGT), 0, st, (const R*)(ws + s.off_out),
-                               level_map(pl, l, 0), (const R*)(ws + upper_off),
-                               level_map(pl, l + 1, 0), (R*)(ws + s.off_in), f);
-            launched = true;
-          }
-        }
-        if (!launched)
-          hipLaunchKernelGGL((k_scan_down<Agg, R, SQRT, WG, F>),
-                             dim3((unsigned)grid_for(s.nwg * s.K * s.wg, WG)), dim3(WG), 0,
-                             st, (const R*)(ws + s.off_out), level_map(pl, l, 0),
-                             (const R*)(ws + upper_off), level_map(pl, l + 1, 0),
-                             (R*)(ws + s.off_in), f);
-      });
-      int rc = hip_check("k_scan_down");
-      if (rc) return rc;
-    }
-    *final_off = pl.lv[0].off_out;
-    *upper_off = pl.nlevels == 1 ? SIZE_MAX
-                                 : (pl.nlevels == 2 ? pl.lv[1].off_out : pl.lv[1].off_in);
     return PSM_OK;
   }
 
@@ -518,7 +515,7 @@ struct Impl {
     launch_fb(fb, g, grid_for(pl.Mp, kLaneWG), grid_for(pl.Mp, kLaneWG), [&](auto f) {
       hipLaunchKernelGGL((k_linearize_states<R, NX, NY, SQRT, decltype(f)>), dim3(grid_for(pl.Mp, kLaneWG)),
                          dim3(kLaneWG), 0, st, pl.M, pl.Mp, pl.chunk, trv, obv, ob ? 1 : 0, sv, use,
-                         (const R*)nm, (const R*)nL, inter, (R*)(ws + pl.off_lin), f);
+                         (const R*)nm, (const R*)nL, inter, (R*)(ws + pl.off_lin), (R*)(ws + pl.off_ref), f);
     });
     return hip_check("k_linearize_states");
   }
@@ -552,24 +549,21 @@ struct Impl {
     launch_fb(fb, g, grid_for(pl.nchunks, kLaneWG), grid_for(pl.nchunks, kLaneWG), [&](auto f) {
       hipLaunchKernelGGL((k_filter_reduce<R, NX, NY, SQRT, decltype(f)>), dim3(grid_for(pl.nchunks, kLaneWG)),
                          dim3(kLaneWG), 0, st, pl.M, pl.Mp, pl.chunk, pl.nchunks, p->state_offsets,
-                         p->n_seq, lin, (const R*)ys, (const R*)m0, (const R*)L0,
+                         p->n_seq, lin, (const R*)ys, (const R*)m0, (const R*)L0, (const R*)(ws + pl.off_ref),
                          (R*)(ws + pl.lv[0].off_in), level_map(pl, 0, 0), f);
     });
     }
     if ((rc = hip_check("k_filter_reduce"))) return rc;
-    size_t pre_off = 0, up_off = 0;
-    if ((rc = run_scan<FA>(pl, ws, fb, g, st, &pre_off, &up_off))) return rc;
+    ScanLevels<R> lv;
+    if ((rc = run_scan<FA>(pl, ws, fb, g, st, 0, &lv))) return rc;
     Acc* ell_state = ell ? (Acc*)(ws + pl.off_ell) : nullptr;
     {
     TimedScope ts_("k_filter_apply", st);
     launch_fb(fb, g, grid_for(pl.nchunks, kLaneWG), grid_for(pl.nchunks, kLaneWG), [&](auto f) {
       hipLaunchKernelGGL((k_filter_apply<R, NX, NY, SQRT, decltype(f)>), dim3(grid_for(pl.nchunks, kLaneWG)),
                          dim3(kLaneWG), 0, st, pl.M, pl.Mp, pl.chunk, pl.nchunks, p->state_offsets,
-                         p->n_seq, lin, (const R*)ys, (const R*)m0, (const R*)L0,
-                         (const R*)(ws + pre_off), level_map(pl, 0, 0),
-                         up_off == SIZE_MAX ? nullptr : (const R*)(ws + up_off),
-                         pl.nlevels > 1 ? level_map(pl, 1, 0) : level_map(pl, 0, 0),
-                         (R*)(ws + pl.lv[0].off_in), (R*)om, (R*)oL, om_inter, ell_state, f);
+                         p->n_seq, lin, (const R*)ys, (const R*)m0, (const R*)L0, (const R*)(ws + pl.off_ref),
+                         lv, (R*)om, (R*)oL, om_inter, ell_state, f);
     });
     }
     if ((rc = hip_check("k_filter_apply"))) return rc;
@@ -609,22 +603,19 @@ struct Impl {
       hipLaunchKernelGGL((k_smoother_reduce<R, NX, NY, SQRT, decltype(f)>),
                          dim3(grid_for(pl.nchunks, kLaneWG)), dim3(kLaneWG), 0, st, pl.M, pl.Mp, pl.chunk,
                          pl.nchunks, p->state_offsets, p->n_seq, (const R*)(ws + pl.off_lin), (const R*)fm,
-                         (const R*)fL, fm_inter, (R*)(ws + pl.off_selem), (R*)(ws + pl.lv[0].off_in),
+                         (const R*)fL, fm_inter, (const R*)(ws + pl.off_ref), (R*)(ws + pl.off_selem), (R*)(ws + pl.lv[0].off_in),
                          level_map(pl, 0, 1), f);
     });
     }
     if ((rc = hip_check("k_smoother_reduce"))) return rc;
-    size_t pre_off = 0, up_off = 0;
-    if ((rc = run_scan<SA>(pl, ws, fb, g, st, &pre_off, &up_off))) return rc;
+    ScanLevels<R> lv;
+    if ((rc = run_scan<SA>(pl, ws, fb, g, st, 1, &lv))) return rc;
     {
       TimedScope ts_("k_smoother_apply", st);
       launch_fb(fb, g, grid_for(pl.nchunks, kLaneWG), grid_for(pl.nchunks, kLaneWG), [&](auto f) {
         hipLaunchKernelGGL((k_smoother_apply<R, NX, SQRT, decltype(f)>), dim3(grid_for(pl.nchunks, kLaneWG)),
                            dim3(kLaneWG), 0, st, pl.M, pl.Mp, pl.chunk, pl.nchunks,
-                           (const R*)(ws + pl.off_selem), (const R*)(ws + pre_off),
-                           level_map(pl, 0, 1), up_off == SIZE_MAX ? nullptr : (const R*)(ws + up_off),
-                           pl.nlevels > 1 ? level_map(pl, 1, 0) : level_map(pl, 0, 0),
-                           (R*)(ws + pl.lv[0].off_in), (R*)om, (R*)oL, om_inter, f);
+                           (const R*)(ws + pl.off_selem), lv, (const R*)(ws + pl.off_ref), (R*)om, (R*)oL, om_inter, f);
       });
     }
     return hip_check("k_smoother_apply");
@@ -672,7 +663,7 @@ struct Impl {
       hipLaunchKernelGGL((k_smoother_reduce<R, NX, NY, SQRT, decltype(f)>), dim3(grid_for(pl.nchunks, kLaneWG)),
                          dim3(kLaneWG), 0, st, pl.M, pl.Mp, pl.chunk, pl.nchunks, p->state_offsets,
                          p->n_seq, (const R*)(ws + pl.off_lin), (const R*)fm, (const R*)fL, 0,
-                         (R*)(ws + pl.off_selem), (R*)(ws + pl.lv[0].off_in), level_map(pl, 0, 1), f);
+                         (const R*)(ws + pl.off_ref), (R*)(ws + pl.off_selem), (R*)(ws + pl.lv[0].off_in), level_map(pl, 0, 1), f);
     });
     if ((rc = hip_check("k_smoother_reduce"))) return rc;
     const int64_t lanes = sp.nch * S;
@@ -686,7 +677,7 @@ struct Impl {
     if ((rc = hip_check("k_sample_bounds"))) return rc;
     hipLaunchKernelGGL((k_sample_apply<R, NX, SQRT>), dim3(grid_for(lanes, kLaneWG)), dim3(kLaneWG),
                        0, st, pl.M, pl.Mp, pl.chunk, sp.Cs, sp.nch, S, (const R*)(ws + pl.off_selem),
-                       (const R*)eps, (const R*)(ws + sp.off_xb), (R*)out);
+                       (const R*)eps, (const R*)(ws + sp.off_xb), (const R*)(ws + pl.off_ref), (R*)out);
     return hip_check("k_sample_apply");
   }
 

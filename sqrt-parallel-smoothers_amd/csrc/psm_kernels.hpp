@@ -6,10 +6,9 @@
 //  * Caller-visible trajectories are array-of-structs, exactly the shapes of the
 //    reference: mean (n_states, nx), chol/cov (n_states, nx, nx).
 //  * Internal per-state buffers (linearized model, smoother elements) and the
-//    scan items are struct-of-arrays, component q of an item at
-//    base[q * stride + position], with positions interleaved (StateMap,
-//    LevelMap) so that the items a wave works on in one step are consecutive
-//    words.
+//    scan items are struct-of-arrays within blocks of 64 positions (blk), with
+//    positions interleaved (StateMap, LevelMap) so that the items a wave works
+//    on in one step are consecutive words.
 //
 // One filter pass over a ragged batch (all sequences concatenated, n_states
 // states) is
@@ -17,14 +16,14 @@
 //                           linearized at the nominal state
 //   2. k_filter_reduce      one lane per chunk of C states: the chunk aggregate
 //                           by absorbing its steps one by one
-//   3. k_scan_up/k_scan_down exclusive scan of the chunk aggregates with the
+//   3. k_scan_up            exclusive scan of the chunk aggregates with the
 //                           full filtering operator (Kogge-Stone inside a
 //                           workgroup, recursive across workgroups; no
-//                           level-0 down-sweep, see 4)
-//   4. k_filter_apply       one lane per chunk: joins the chunk's level-0
-//                           prefix with its workgroup's prefix, then runs the
-//                           sequential square-root Kalman filter from that
-//                           incoming filtered state, writing the filtered
+//                           down-sweep, see 4)
+//   4. k_filter_apply       one lane per chunk: takes the prior through the
+//                           chunk's prefixes of every scan level, then runs
+//                           the sequential square-root Kalman filter from
+//                           that incoming filtered state, writing the filtered
 //                           states and the per-step log-likelihood terms
 // and the smoother pass mirrors it backwards in time (elements, reverse scan,
 // application).  Because the first state of every sequence carries its prior
@@ -38,8 +37,7 @@
 
 #include "psm_core.hpp"
 #include "psm_scan_mem.hpp"
-#include "psm_team.hpp"
-#include "psm_quad.hpp"
+#include "psm_coop.hpp"
 
 namespace psm {
 
@@ -48,9 +46,10 @@ constexpr int kScanWG = 64;     // one wave per scan workgroup
 // LDS buffers of 64 aggregates would not fit the 160 KB of LDS (tangent types).
 template <typename Agg, typename R>
 constexpr int scan_wg() {
-  return (3 * Agg::NQ * 64 * (int)sizeof(R) <= 150 * 1024) ? 64 : 32;
+  return (3 * odd_words(Agg::NQ) * 64 * (int)sizeof(R) <= 150 * 1024) ? 64 : 32;
 }
 constexpr int kLaneWG = 64;     // workgroup size of the lane-per-item kernels
+constexpr int kRowVL = 16;      // groups of 16 lanes per workgroup of the cooperative scans
 
 // Positions in the internal struct-of-arrays buffers.  The lane-per-chunk
 // kernels run 64 consecutive chunks in one wave and step through their C
@@ -60,10 +59,10 @@ constexpr int kLaneWG = 64;     // workgroup size of the lane-per-item kernels
 // full-line load instead of a C-strided gather).
 struct StateMap {
   int C;
+  PSM_DEV int64_t at(int64_t c, int64_t k) const { return (c >> 6) * ((int64_t)C << 6) + (k << 6) + (c & 63); }
   PSM_DEV int64_t operator()(int64_t i) const {
     const int64_t c = i / C;
-    const int64_t k = i - c * C;
-    return (c >> 6) * ((int64_t)C << 6) + (k << 6) + (c & 63);
+    return at(c, i - c * C);
   }
 };
 inline int64_t state_stride(int64_t M, int C) {
@@ -82,13 +81,16 @@ struct LevelMap {
   int K;
   int WG;
   int rev;
+  // (item counts fit 32 bits: 2^31 chunk aggregates would not fit the memory)
   PSM_DEV int64_t at(int64_t p) const {
-    const int64_t blk = (int64_t)K * WG;
-    const int64_t b = p / blk;
-    const int64_t r = p - b * blk;
-    const int64_t l = r / K;
-    return b * blk + (r - l * K) * WG + l;
+    const uint32_t span = (uint32_t)K * (uint32_t)WG;
+    const uint32_t b = (uint32_t)p / span;
+    const uint32_t r = (uint32_t)p - b * span;
+    const uint32_t l = r / (uint32_t)K;
+    return (int64_t)b * span + (r - l * K) * WG + l;
   }
+  // fold step j of lane t of workgroup b
+  PSM_DEV int64_t at(int64_t b, int t, int j) const { return (b * K + j) * WG + t; }
   PSM_DEV int64_t pos(int64_t c) const { return at(rev ? n - 1 - c : c); }
 };
 
@@ -129,32 +131,35 @@ PSM_DEV void st_aos(R* __restrict__ p, int64_t i, const R (&v)[M][N]) {
 // Trajectories (a mean and a factor per state) come in two layouts: the API's
 // array-of-structs (state i at m + i NX, L + i NX^2; inter == 0), or, inside a
 // launch sequence that owns them, the state-interleaved layout of the
-// workspace (inter != 0: component q of state i at m[q Mp + pos], pos its
-// interleaved position, means first, then a factor's lower triangle or a
-// covariance in full (SYM), so that a launch sequence and the host loop over
-// the same passes agree bit for bit), which lane-per-chunk kernels read and
-// write coalesced.
+// workspace (inter != 0: blocked at the state's interleaved position pos, means
+// first, then a factor's lower triangle or a covariance in full (SYM), so that a
+// launch sequence and the host loop over the same passes agree bit for bit),
+// which lane-per-chunk kernels read and write coalesced.
+template <bool SYM, int NX>
+constexpr int kTrajWords = NX + (SYM ? NX * NX : NX * (NX + 1) / 2);
 template <bool SYM, typename R, int NX>
-PSM_DEV void traj_load(const R* __restrict__ m_, const R* __restrict__ L_, int inter, int64_t Mp,
+PSM_DEV void traj_load(const R* __restrict__ m_, const R* __restrict__ L_, int inter,
                        int64_t i, int64_t pos, R (&m)[NX], R (&L)[NX][NX]) {
   if (inter) {
+    const R* p = blk<kTrajWords<SYM, NX>>(m_, pos);
     int q = 0;
-    ld(m_, Mp, pos, q, m);
-    if constexpr (SYM) ld(m_, Mp, pos, q, L);
-    else ld_tri<false>(m_, Mp, pos, q, L);
+    ld(p, kBlk, 0, q, m);
+    if constexpr (SYM) ld(p, kBlk, 0, q, L);
+    else ld_tri<false>(p, kBlk, 0, q, L);
   } else {
     ld_aos(m_, i, m);
     ld_aos(L_, i, L);
   }
 }
 template <bool SYM, typename R, int NX>
-PSM_DEV void traj_store(R* __restrict__ m_, R* __restrict__ L_, int inter, int64_t Mp, int64_t i,
+PSM_DEV void traj_store(R* __restrict__ m_, R* __restrict__ L_, int inter, int64_t i,
                         int64_t pos, const R (&m)[NX], const R (&L)[NX][NX]) {
   if (inter) {
+    R* p = blk<kTrajWords<SYM, NX>>(m_, pos);
     int q = 0;
-    st(m_, Mp, pos, q, m);
-    if constexpr (SYM) st(m_, Mp, pos, q, L);
-    else st_tri(m_, Mp, pos, q, L);
+    st(p, kBlk, 0, q, m);
+    if constexpr (SYM) st(p, kBlk, 0, q, L);
+    else st_tri(p, kBlk, 0, q, L);
   } else {
     st_aos(m_, i, m);
     st_aos(L_, i, L);
@@ -281,25 +286,69 @@ PSM_DEV void linearize_point_w(const ModelView<R>& md, const SigmaView<R>& sp, i
   }
 }
 
+// Centred states of the FP32 square-root passes.  Between the linearization and
+// the output every mean is a difference from the nominal mean of its state:
+// x_k = n_k + d_k turns x_{k+1} = F x_k + b into d_{k+1} = F d_k + b', b' = b + F n_k
+// - n_{k+1}, and y = H x + c into y = H d + c', c' = c + H n_k (formed in FP64, where
+// n_k, n_{k+1} and F are exact).  The rounding of an aggregate's A (about 1 on
+// its diagonal, so 6e-8 a step, adding up along a sequence) multiplies d, of the
+// size of the posterior's spread, and not x, a position of 10 to 1000: the
+// smoothed means of a T = 16,385 pass were 1.5e-5 of their norm off a 64-bit
+// recursion, and are 1.8e-6 with this.  ref holds n_k (blocked at the states'
+// interleaved positions, NX words).  Trajectories hold n + d in either layout, so that a
+// launch sequence and the host loop over the same passes agree bit for bit.
+template <typename R, bool SQRT>
+constexpr bool kCentred = SQRT && std::is_same<R, float>::value;
+
+// b <- b + F m - next
+template <typename R, int NO, int NI>
+PSM_DEV void centre(const R (&F)[NO][NI], const R (&m)[NI], const R (&next)[NO], R (&b)[NO]) {
+#pragma unroll
+  for (int a = 0; a < NO; ++a) {
+    double s = (double)b[a] - (double)next[a];
+#pragma unroll
+    for (int k = 0; k < NI; ++k) s = fma((double)F[a][k], (double)m[k], s);
+    b[a] = (R)s;
+  }
+}
+// m -/+ the nominal mean at interleaved position pos
+template <typename R, int NX>
+PSM_DEV void to_centred(const R* __restrict__ ref, int64_t pos, R (&m)[NX]) {
+  R n[NX];
+  int q = 0;
+  ld(blk<NX>(ref, pos), kBlk, 0, q, n);
+#pragma unroll
+  for (int a = 0; a < NX; ++a) m[a] -= n[a];
+}
+template <typename R, int NX>
+PSM_DEV void from_centred(const R* __restrict__ ref, int64_t pos, R (&m)[NX]) {
+  R n[NX];
+  int q = 0;
+  ld(blk<NX>(ref, pos), kBlk, 0, q, n);
+#pragma unroll
+  for (int a = 0; a < NX; ++a) m[a] += n[a];
+}
+
 // Thread t fills position t of the state-interleaved buffer (coalesced stores);
 // its state is the inverse of StateMap.
 template <typename R, int NX, int NY, bool SQRT, typename FB = Fallback>
 __global__ __launch_bounds__(kLaneWG) void k_linearize_states(
     int64_t M, int64_t Mp, int C, ModelView<R> tr, ModelView<R> ob, int do_obs, SigmaView<R> sp,
     int use_sigma, const R* __restrict__ nom_m, const R* __restrict__ nom_L, int nom_inter,
-    R* __restrict__ lin, FB fb) {
+    R* __restrict__ lin, R* __restrict__ ref, FB fb) {
   if (fb.skip()) return;
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= Mp) return;
   const int64_t g = (int64_t)C << 6;
-  const int64_t blk = t / g;
-  const int64_t r = t - blk * g;
-  const int64_t i = ((blk << 6) + (r & 63)) * C + (r >> 6);
+  const int64_t gb = t / g;
+  const int64_t r = t - gb * g;
+  const int64_t i = ((gb << 6) + (r & 63)) * C + (r >> 6);
   if (i >= M) return;
   tr.row = i;
   ob.row = i;
   R m[NX], L[NX][NX];
-  traj_load<!SQRT, R, NX>(nom_m, nom_L, nom_inter, Mp, i, t, m, L);
+  traj_load<!SQRT, R, NX>(nom_m, nom_L, nom_inter, i, t, m, L);
+  R* lp = blk<Step<R, NX, NY>::NQ>(lin, t);
   // FP32: the regression's increments wait in LDS for its residual pass
   PointCache<R> pc{nullptr, 0, 0};
   if constexpr (std::is_same<R, float>::value) {
@@ -309,20 +358,41 @@ __global__ __launch_bounds__(kLaneWG) void k_linearize_states(
   {
     R F[NX][NX], Cq[NX][NX], b[NX];
     linearize_point_w<R, NX, NX, SQRT>(tr, sp, use_sigma, m, L, F, Cq, b, fb, pc);
+    if constexpr (kCentred<R, SQRT>) {
+      R next[NX];
+      copy(m, next);
+      if (i + 1 < M) {
+        if (nom_inter) {
+          // the next slot of this chunk, or the first of the next
+          const int64_t pos = (r >> 6) + 1 < C ? t + 64 : StateMap{C}(i + 1);
+          int q = 0;
+          ld(blk<kTrajWords<!SQRT, NX>>(nom_m, pos), kBlk, 0, q, next);
+        } else {
+          ld_aos(nom_m, i + 1, next);
+        }
+      }
+      int q = 0;
+      st(blk<NX>(ref, t), kBlk, 0, q, m);
+      centre(F, m, next, b);
+    }
     int q = 0;
-    st(lin, Mp, t, q, F);
+    st(lp, kBlk, 0, q, F);
     if constexpr (SQRT) lower_factor(Cq);
-    st_tri(lin, Mp, t, q, Cq);
-    st(lin, Mp, t, q, b);
+    st_tri(lp, kBlk, 0, q, Cq);
+    st(lp, kBlk, 0, q, b);
   }
   if (do_obs) {
     R H[NY][NX], Cr[NY][NY], c[NY];
     linearize_point_w<R, NX, NY, SQRT>(ob, sp, use_sigma, m, L, H, Cr, c, fb);
+    if constexpr (kCentred<R, SQRT>) {
+      const R zero[NY] = {};
+      centre(H, m, zero, c);
+    }
     int q = Step<R, NX, NY>::NTRANS;
-    st(lin, Mp, t, q, H);
+    st(lp, kBlk, 0, q, H);
     if constexpr (SQRT) lower_factor(Cr);
-    st_tri(lin, Mp, t, q, Cr);
-    st(lin, Mp, t, q, c);
+    st_tri(lp, kBlk, 0, q, Cr);
+    st(lp, kBlk, 0, q, c);
   }
 }
 
@@ -333,7 +403,7 @@ template <typename R, int NX, int NY, bool SQRT, typename FB = Fallback>
 __global__ __launch_bounds__(kLaneWG) void k_filter_reduce(
     int64_t M, int64_t Mp, int chunk, int64_t nchunks, const int64_t* __restrict__ soff, int nseq,
     const R* __restrict__ lin, const R* __restrict__ ys, const R* __restrict__ m0,
-    const R* __restrict__ L0, R* __restrict__ agg, LevelMap lm, FB fb) {
+    const R* __restrict__ L0, const R* __restrict__ ref, R* __restrict__ agg, LevelMap lm, FB fb) {
   if (fb.skip()) return;
   const StateMap sm{chunk};
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -348,20 +418,22 @@ __global__ __launch_bounds__(kLaneWG) void k_filter_reduce(
     if (i == soff[s]) {
       set_zero(a.A);
       ld_aos(m0, s, a.b);
+      if constexpr (kCentred<R, SQRT>) to_centred(ref, sm.at(c, i - i0), a.b);
       ld_aos(L0, s, a.U);
+      if constexpr (SQRT) lower_factor(a.U);
       set_zero(a.eta);
       set_zero(a.Z);
       a.flag = FLAG_HEAD;
     } else {
       Step<R, NX, NY> st_;
-      load_trans<!SQRT>(lin, Mp, sm(i - 1), st_);
-      load_obs<!SQRT>(lin, Mp, sm(i), st_);
+      load_trans<!SQRT>(lin, i > i0 ? sm.at(c, i - i0 - 1) : sm.at(c - 1, chunk - 1), st_);
+      load_obs<!SQRT>(lin, sm.at(c, i - i0), st_);
       R y[NY];
       ld_aos(ys, i - s - 1, y);
       absorb_fb<R, NX, NY, SQRT>(a, st_, y, fb);
     }
   }
-  store_agg(agg, lm.stride, lm.pos(c), a);
+  store_agg(agg, lm.pos(c), a);
 }
 
 // ============================================================================
@@ -391,16 +463,17 @@ __global__ __launch_bounds__(WG) void k_scan_up(const R* __restrict__ in, LevelM
   const int K = lm.K;
   const int64_t n = lm.n;
   auto slot = [&](int buf, int lane) { return V{lds + buf * NQ * WG, (int64_t)WG, (int64_t)lane}; };
-  R* inm = const_cast<R*>(in);
   const V stage = slot(2, t);
   const int64_t base = ((int64_t)blockIdx.x * WG + t) * K;
+  auto view = [&](const R* p, int64_t pos) { return V{blk<NQ>(const_cast<R*>(p), pos), kBlk, 0}; };
+  auto item = [&](int j) { return view(in, lm.at(blockIdx.x, t, j)); };
   int cur = 0;
-  if (base < n) view_copy(V{inm, lm.stride, lm.at(base)}, slot(0, t));
+  if (base < n) view_copy(item(0), slot(0, t));
   else view_identity(slot(0, t));
   for (int j = 1; j < K; ++j) {
     const int64_t p = base + j;
     if (p >= n) break;
-    view_copy(V{inm, lm.stride, lm.at(p)}, stage);
+    view_copy(item(j), stage);
     combine_mem_fb<R, NX, SQRT>(slot(cur, t), stage, slot(1 - cur, t), fb);
     cur = 1 - cur;
   }
@@ -414,7 +487,7 @@ __global__ __launch_bounds__(WG) void k_scan_up(const R* __restrict__ in, LevelM
   }
   __syncthreads();
   if (t == WG - 1 && totals != nullptr)
-    view_copy(slot(cur, t), V{totals, tm.stride, tm.at((int64_t)blockIdx.x)});
+    view_copy(slot(cur, t), view(totals, tm.at((int64_t)blockIdx.x)));
   // running exclusive prefix in this lane's slot of the other buffer; once
   // every lane has read its predecessor's inclusive prefix, slot(cur, t) is
   // free for the next running prefix
@@ -426,12 +499,11 @@ __global__ __launch_bounds__(WG) void k_scan_up(const R* __restrict__ in, LevelM
   for (int j = 0; j < K; ++j) {
     const int64_t p = base + j;
     if (p >= n) break;
-    const int64_t item = lm.at(p);
-    view_copy(run, V{out_excl, lm.stride, item});
+    view_copy(run, view(out_excl, lm.at(blockIdx.x, t, j)));
     // the running prefix after the lane's last item is its inclusive total,
     // which the scan over the lanes already produced
     if (j + 1 == K || p + 1 == n) break;
-    view_copy(V{inm, lm.stride, item}, stage);
+    view_copy(item(j), stage);
     combine_mem_fb<R, NX, SQRT>(run, stage, tmp, fb);
     const V x = run;
     run = tmp;
@@ -439,239 +511,135 @@ __global__ __launch_bounds__(WG) void k_scan_up(const R* __restrict__ in, LevelM
   }
 }
 
-// dst[p] <- upper[w] (+) out_excl[p] (workgroup w > 0; w == 0 copies): the
-// complete exclusive prefixes, written out of place so the operands stay
-// intact for the FP64 fallback.  upper holds the complete exclusive prefixes of
-// the next level (um).  The combinations are independent, so every thread
-// takes one storage position q of the level (consecutive threads, consecutive
-// positions) and recovers its scan position p and workgroup w from q.
-template <typename Agg, typename R, bool SQRT, int WG = scan_wg<Agg, R>(), typename FB = Fallback>
-__global__ __launch_bounds__(WG) void k_scan_down(const R* __restrict__ out_excl, LevelMap lm,
-                                                  const R* __restrict__ upper, LevelMap um,
-                                                  R* __restrict__ dst, FB fb) {
-  if (fb.skip()) return;
-  using V = typename ViewOf<Agg>::type;
-  constexpr int NX = Agg_nx<Agg>::value;
-  const int64_t q = (int64_t)blockIdx.x * WG + threadIdx.x;
-  const int64_t span = (int64_t)lm.K * lm.WG;
-  const int64_t w = q / span;
-  const int64_t r = q - w * span;
-  const int64_t p = w * span + (r % lm.WG) * lm.K + r / lm.WG;
-  if (p >= lm.n) return;
-  const V e{const_cast<R*>(out_excl), lm.stride, q};
-  const V o{dst, lm.stride, q};
-  if (w == 0) view_copy(e, o);
-  else combine_mem_fb<R, NX, SQRT>(V{const_cast<R*>(upper), um.stride, um.at(w)}, e, o, fb);
-}
-
-// Team versions of the two scan kernels for the square-root form: kTeamVL
-// teams of TL lanes per workgroup; each team is one virtual lane of the scan
-// above (folds K items, joins the Kogge-Stone scan over the teams, rewrites
-// its items' exclusive prefixes) and runs every combination cooperatively.
-template <typename Agg, typename R>
-struct TeamCfg {
-  using V = typename ViewOf<Agg>::type;
-  static constexpr int TL = kTeamLanes;
-  static constexpr int VL = kTeamVL;
-  static constexpr int WGT = VL * TL;
-  static constexpr int SCR = team_scratch_bytes<V>();
-};
-
-template <typename Agg, typename R, typename FB = Fallback>
-__global__ __launch_bounds__((TeamCfg<Agg, R>::WGT)) void k_scan_up_team(
-    const R* __restrict__ in, LevelMap lm, R* __restrict__ out_excl, R* __restrict__ totals,
-    LevelMap tm, FB fb) {
-  if (fb.skip()) return;
-  using Cfg = TeamCfg<Agg, R>;
-  using V = typename Cfg::V;
-  constexpr int NX = Agg_nx<Agg>::value;
-  constexpr int NQ = Agg::NQ;
-  constexpr int TL = Cfg::TL;
-  constexpr int VL = Cfg::VL;
-  __shared__ R lds[2 * NQ * VL];
-  __shared__ __align__(16) char scr[VL * Cfg::SCR];
-  const int t = (int)threadIdx.x / TL;
-  const int r = (int)threadIdx.x % TL;
-  void* my = scr + t * Cfg::SCR;
-  auto slot = [&](int buf, int lane) { return V{lds + buf * NQ * VL, (int64_t)VL, (int64_t)lane}; };
-  const int K = lm.K;
-  const int64_t n = lm.n;
-  R* inm = const_cast<R*>(in);
-  const int64_t base = ((int64_t)blockIdx.x * VL + t) * K;
-  int cur = 0;
-  team_identity(slot(0, t), r);
-  for (int j = 0; j < K; ++j) {
-    const int64_t p = base + j;
-    if (p >= n) break;
-    team_combine<R, NX>(slot(cur, t), V{inm, lm.stride, lm.at(p)}, slot(1 - cur, t), r, my, fb);
-    cur = 1 - cur;
-  }
-  if (cur == 1) {
-    team_sync();
-    team_copy(slot(1, t), slot(0, t), r);
-  }
-  cur = 0;
-  for (int d = 1; d < VL; d <<= 1) {
-    __syncthreads();
-    if (t >= d) team_combine<R, NX>(slot(cur, t - d), slot(cur, t), slot(1 - cur, t), r, my, fb);
-    else team_copy(slot(cur, t), slot(1 - cur, t), r);
-    cur = 1 - cur;
-  }
-  __syncthreads();
-  if (t == VL - 1 && totals != nullptr)
-    team_copy(slot(cur, t), V{totals, tm.stride, tm.at((int64_t)blockIdx.x)}, r);
-  // running exclusive prefix of this team: run = slot(1 - cur, t); once every
-  // team has read its predecessor's inclusive prefix, slot(cur, t) is free
-  V run = slot(1 - cur, t);
-  if (t == 0) team_identity(run, r);
-  else team_copy(slot(cur, t - 1), run, r);
-  __syncthreads();
-  V tmp = slot(cur, t);
-  for (int j = 0; j < K; ++j) {
-    const int64_t p = base + j;
-    if (p >= n) break;
-    const int64_t item = lm.at(p);
-    team_sync();
-    team_copy(run, V{out_excl, lm.stride, item}, r);
-    if (j + 1 == K || p + 1 == n) break;  // the team's inclusive total is not needed
-    team_combine<R, NX>(run, V{inm, lm.stride, item}, tmp, r, my, fb);
-    const V x = run;
-    run = tmp;
-    tmp = x;
-  }
-}
-
-// One item per team: block b covers workgroup b / K of the level and item
-// b % K of each of its teams.
-template <typename Agg, typename R, typename FB = Fallback>
-__global__ __launch_bounds__((TeamCfg<Agg, R>::WGT)) void k_scan_down_team(
-    const R* __restrict__ out_excl, LevelMap lm, const R* __restrict__ upper, LevelMap um,
-    R* __restrict__ dst, FB fb) {
-  if (fb.skip()) return;
-  using Cfg = TeamCfg<Agg, R>;
-  using V = typename Cfg::V;
-  constexpr int NX = Agg_nx<Agg>::value;
-  constexpr int TL = Cfg::TL;
-  constexpr int VL = Cfg::VL;
-  __shared__ __align__(16) char scr[VL * Cfg::SCR];
-  const int t = (int)threadIdx.x / TL;
-  const int r = (int)threadIdx.x % TL;
-  void* my = scr + t * Cfg::SCR;
-  const int K = lm.K;
-  const int64_t w = (int64_t)blockIdx.x / K;
-  const int j = (int)((int64_t)blockIdx.x - w * K);
-  const int64_t p = (w * VL + t) * K + j;
-  if (p >= lm.n) return;  // whole teams leave together; team_combine syncs only within the team
-  const int64_t item = lm.at(p);
-  const V e{const_cast<R*>(out_excl), lm.stride, item};
-  const V o{dst, lm.stride, item};
-  if (w == 0) team_copy(e, o, r);
-  else team_combine<R, NX>(V{const_cast<R*>(upper), um.stride, um.at(w)}, e, o, r, my, fb);
-}
-
-// Quad version of k_scan_up for level 0 of the square-root scans: VL quads
-// per workgroup; each quad is one virtual lane of the scan above (folds K
-// items, joins the Kogge-Stone scan over the quads, rewrites its items'
-// exclusive prefixes) and runs every combination cooperatively.  The level
-// layout is that of k_scan_up with VL lanes, so the two are interchangeable.
-template <typename Agg, typename R, int VL, typename FB = Fallback>
-__global__ __launch_bounds__(VL * kQuadLanes) void k_scan_up_quad(
+// k_scan_up for the square-root form with G lanes per combination
+// (psm_coop.hpp): VL groups per workgroup, each one virtual lane of the scan
+// above (folds K items, joins the Kogge-Stone scan over the groups, rewrites its
+// items' exclusive prefixes).  The level layout is that of k_scan_up with VL
+// lanes, so the two are interchangeable.  One call site combines in all three
+// parts, so the instructions of a combination are fetched once.
+template <typename Agg, typename R, int G, int VL, typename FB = Fallback>
+__global__ __launch_bounds__(VL * G) void k_scan_up_coop(
     const R* __restrict__ in, LevelMap lm, R* __restrict__ out_excl, R* __restrict__ totals,
     LevelMap tm, FB fb) {
   if (fb.skip()) return;
   using V = typename ViewOf<Agg>::type;
-  constexpr int NX = Agg_nx<Agg>::value;
-  constexpr int NQ = Agg::NQ;
-  // buffers 0 and 1: running / scanned aggregates; buffer 2: the quad's next
-  // input item, copied from HBM before it is combined
-  __shared__ R lds[3 * NQ * VL];
-  const int t = (int)threadIdx.x / kQuadLanes;
-  const int r = (int)threadIdx.x % kQuadLanes;
-  auto slot = [&](int buf, int lane) { return V{lds + buf * NQ * VL, (int64_t)VL, (int64_t)lane}; };
-  R* inm = const_cast<R*>(in);
-  const V stage = slot(2, t);
+  constexpr int NQP = odd_words(Agg::NQ);
+  __shared__ R acc[NQP * VL];    // the running / scanned aggregate of each group
+  __shared__ R stage[NQP * VL];  // the group's next input item
+  const int t = (int)threadIdx.x / G;
+  const int r = (int)threadIdx.x % G;
+  R* mine = acc + t * NQP;
+  R* my_stage = stage + t * NQP;
   const int K = lm.K;
   const int64_t n = lm.n;
   const int64_t base = ((int64_t)blockIdx.x * VL + t) * K;
-  int cur = 0;
-  if (base < n) quad_copy(V{inm, lm.stride, lm.at(base)}, slot(0, t), r);
-  else quad_identity(slot(0, t), r);
-  for (int j = 1; j < K; ++j) {
-    const int64_t p = base + j;
-    if (p >= n) break;
-    team_sync();
-    quad_copy(V{inm, lm.stride, lm.at(p)}, stage, r);
-    quad_combine<R, NX>(slot(cur, t), stage, slot(1 - cur, t), r, fb);
-    cur = 1 - cur;
+  constexpr int NQ = Agg::NQ;
+  auto view = [&](const R* p, int64_t pos) { return V{blk<NQ>(const_cast<R*>(p), pos), kBlk, 0}; };
+  {
+    ItemRegs<V, G> move;
+    if (base < n) move.load(view(in, lm.at(blockIdx.x, t, 0)), r);
+    else move.identity(r);
+    move.store(mine, r);
   }
-  if (cur == 1) {
-    team_sync();
-    quad_copy(slot(1, t), slot(0, t), r);
-  }
-  cur = 0;
-  for (int d = 1; d < VL; d <<= 1) {
-    __syncthreads();
-    if (t >= d) quad_combine<R, NX>(slot(cur, t - d), slot(cur, t), slot(1 - cur, t), r, fb);
-    else quad_copy(slot(cur, t), slot(1 - cur, t), r);
-    cur = 1 - cur;
-  }
-  __syncthreads();
-  if (t == VL - 1 && totals != nullptr)
-    quad_copy(slot(cur, t), V{totals, tm.stride, tm.at((int64_t)blockIdx.x)}, r);
-  // running exclusive prefix of this quad: run = slot(1 - cur, t); once every
-  // quad has read its predecessor's inclusive prefix, slot(cur, t) is free
-  V run = slot(1 - cur, t);
-  if (t == 0) quad_identity(run, r);
-  else quad_copy(slot(cur, t - 1), run, r);
-  __syncthreads();
-  V tmp = slot(cur, t);
-  for (int j = 0; j < K; ++j) {
-    const int64_t p = base + j;
-    if (p >= n) break;
-    const int64_t item = lm.at(p);
-    team_sync();
-    quad_copy(run, V{out_excl, lm.stride, item}, r);
-    if (j + 1 == K || p + 1 == n) break;  // the quad's inclusive total is not needed
-    quad_copy(V{inm, lm.stride, item}, stage, r);
-    quad_combine<R, NX>(run, stage, tmp, r, fb);
-    const V x = run;
-    run = tmp;
-    tmp = x;
+  constexpr int kScan = VL == 64 ? 6 : VL == 32 ? 5 : VL == 16 ? 4 : 0;
+  static_assert((1 << kScan) == VL, "groups per workgroup");
+  const int folds = K - 1;
+  const int steps = folds + kScan + folds;
+  for (int step = 0;; ++step) {
+    // an opaque copy of the lane: what the step derives from it (offsets, row
+    // kinds, addresses) is formed anew each time, not hoisted into registers that
+    // live through the combinations
+    int rl = r;
+    asm volatile("" : "+v"(rl));
+    const bool fold = step < folds, scan = !fold && step < folds + kScan;
+    const int j = fold ? step + 1 : step - folds - kScan;   // item of a fold / rewrite step
+    if (step == folds + kScan) {
+      // the workgroup's total, and the exclusive prefix of each group
+      __syncthreads();
+      if (t == VL - 1 && totals != nullptr) {
+        ItemRegs<V, G> move;
+        move.load(mine, rl);
+        move.store(view(totals, tm.at((int64_t)blockIdx.x)), rl);
+      }
+      ItemRegs<V, G> move;
+      if (t == 0) move.identity(rl);
+      else move.load(mine - NQP, rl);
+      __syncthreads();
+      move.store(mine, rl);
+    }
+    if (step >= folds + kScan && base + j < n) {
+      group_sync();
+      ItemRegs<V, G> move;
+      move.load(mine, rl);
+      move.store(view(out_excl, lm.at(blockIdx.x, t, j)), rl);
+    }
+    if (step == steps) break;
+    R* e1 = mine;
+    const R* e2 = my_stage;
+    bool act = base + j < n;
+    if (scan) {
+      const int d = 1 << (step - folds);
+      act = t >= d;
+      e1 = act ? mine - d * NQP : mine;
+      e2 = mine;
+      __syncthreads();
+    } else {
+      if (act) {
+        ItemRegs<V, G> move;
+        move.load(view(in, lm.at(blockIdx.x, t, j)), rl);
+        move.store(my_stage, rl);
+      }
+      group_sync();
+    }
+    // an idle group keeps what it has: its running aggregate is e1 outside the scan
+    CoopStep<V, G> cs;
+    if (act) cs.prepare(e1, e2, !scan, rl, fb);
+    if (scan) __syncthreads();
+    else group_sync();
+    cs.commit(mine, rl);
   }
 }
 
 // ============================================================================
 // 4. filter application
 // ============================================================================
-// Complete exclusive prefix of level-0 item c (chunk c, in scan order when
-// lm.rev).  The level-0 up-sweep leaves each item's prefix within its
-// workgroup; items of workgroup w > 0 still need the prefix of the workgroups
-// before them (level 1: upper[w]).  That last combination -- what a level-0
-// down-sweep would do for every item -- is done here by the lane that uses it,
-// into joined (the free level-0 input buffer).  upper == nullptr: a one-level
-// scan, whose prefixes are already complete.  Returns the buffer holding the
-// prefix and its position *pc.
-template <typename Agg, typename R, bool SQRT, typename FB>
-PSM_DEV const R* level0_prefix(int64_t c, const R* __restrict__ prefix, const LevelMap& lm,
-                               const R* __restrict__ upper, const LevelMap& um,
-                               R* __restrict__ joined, const FB& fb, int64_t* pc) {
-  using V = typename ViewOf<Agg>::type;
-  constexpr int NX = Agg_nx<Agg>::value;
-  const int64_t p = lm.rev ? lm.n - 1 - c : c;
-  *pc = lm.at(p);
-  const int64_t w = p / ((int64_t)lm.K * lm.WG);
-  if (upper == nullptr || w == 0) return prefix;
-  combine_mem_fb<R, NX, SQRT>(V{const_cast<R*>(upper), um.stride, um.at(w)},
-                              V{const_cast<R*>(prefix), lm.stride, *pc}, V{joined, lm.stride, *pc}, fb);
-  return joined;
+// The exclusive prefixes of every scan level, level 0 (the chunks) first: an
+// item's prefix covers the items before it in its own workgroup, the prefix of
+// its workgroup is an item of the next level.
+template <typename R>
+struct ScanLevels {
+  static constexpr int kMax = 16;
+  int n;
+  uint32_t span[kMax];   // chunks per item of the level
+  const R* prefix[kMax];
+  LevelMap map[kMax];
+};
+
+// Takes the first distribution of the scan through the prefixes that precede
+// chunk c, from the top level down.  The whole prefix of a chunk contains the
+// first state of its sequence (HEAD), so it is a distribution (m, L) and
+// taking it through one more aggregate costs half a combination: no
+// A, eta and Z are formed.  Every lane of a wavefront does this for its own chunk
+// with consecutive lanes on consecutive items; it replaces a down-sweep, which
+// would read and write every aggregate of a level once more.
+// Push(view, m, L): (m, L) <- aggregate applied to (m, L).
+template <typename V, typename R, int NX, typename Push>
+PSM_DEV void enter_chunk(int64_t c, const ScanLevels<R>& lv, R (&m)[NX], R (&L)[NX][NX], Push&& push) {
+  const uint32_t p0 = (uint32_t)(lv.map[0].rev ? lv.map[0].n - 1 - c : c);
+  for (int l = lv.n - 1; l >= 0; --l) {
+    const V v{blk<V::QF + 1>(const_cast<R*>(lv.prefix[l]), lv.map[l].at(p0 / lv.span[l])), kBlk, 0};
+    const int f = v.flag();
+    if (f == FLAG_IDENT) continue;
+    if (f == FLAG_HEAD) view_head(v, m, L);
+    else push(v, m, L);
+  }
 }
 
 template <typename R, int NX, int NY, bool SQRT, typename FB = Fallback>
 __global__ __launch_bounds__(kLaneWG) void k_filter_apply(
     int64_t M, int64_t Mp, int chunk, int64_t nchunks, const int64_t* __restrict__ soff, int nseq,
     const R* __restrict__ lin, const R* __restrict__ ys, const R* __restrict__ m0,
-    const R* __restrict__ L0, const R* __restrict__ prefix, LevelMap lm,
-    const R* __restrict__ upper, LevelMap um, R* __restrict__ joined, R* __restrict__ out_m,
+    const R* __restrict__ L0, const R* __restrict__ ref, ScanLevels<R> lv, R* __restrict__ out_m,
     R* __restrict__ out_L, int out_inter, typename AccOf<R>::type* __restrict__ ell_state, FB fb) {
   if (fb.skip()) return;
   using Acc = typename AccOf<R>::type;
@@ -682,29 +650,35 @@ __global__ __launch_bounds__(kLaneWG) void k_filter_apply(
   const int64_t i1 = min(i0 + chunk, M);
   int s = seq_of(soff, nseq, i0);
   R m[NX], L[NX][NX];
-  {
-    // incoming filtered state: (b, U) of the complete exclusive prefix
-    int64_t pc;
-    const R* src = level0_prefix<FAgg<R, NX>, R, SQRT>(c, prefix, lm, upper, um, joined, fb, &pc);
-    int q = NX * NX;
-    ld(src, lm.stride, pc, q, m);
-    ld(src, lm.stride, pc, q, L);
-  }
+  set_zero(m);
+  set_zero(L);
+  enter_chunk<FView<R, NX>>(c, lv, m, L, [&](const FView<R, NX>& v, R (&mm)[NX], R (&LL)[NX][NX]) {
+    filter_push_fb<R, NX, SQRT>(v, mm, LL, fb);
+  });
   for (int64_t i = i0; i < i1; ++i) {
     while (i >= soff[s + 1]) ++s;
     Acc e = Acc(0.0);
     if (i == soff[s]) {
       ld_aos(m0, s, m);
       ld_aos(L0, s, L);
+      // the caller's factor of the prior goes out as it is; the recursion and the
+      // interleaved trajectory take its lower triangular form
+      if (!out_inter) traj_store<!SQRT, R, NX>(out_m, out_L, 0, i, sm.at(c, i - i0), m, L);
+      if constexpr (SQRT) lower_factor(L);
+      if (out_inter) traj_store<!SQRT, R, NX>(out_m, out_L, 1, i, sm.at(c, i - i0), m, L);
+      if constexpr (kCentred<R, SQRT>) to_centred(ref, sm.at(c, i - i0), m);
     } else {
       Step<R, NX, NY> st_;
-      load_trans<!SQRT>(lin, Mp, sm(i - 1), st_);
-      load_obs<!SQRT>(lin, Mp, sm(i), st_);
+      load_trans<!SQRT>(lin, i > i0 ? sm.at(c, i - i0 - 1) : sm.at(c - 1, chunk - 1), st_);
+      load_obs<!SQRT>(lin, sm.at(c, i - i0), st_);
       R y[NY];
       ld_aos(ys, i - s - 1, y);
       e = kf_step_fb<R, NX, NY, SQRT>(st_, y, m, L, fb);
+      R x[NX];
+      copy(m, x);
+      if constexpr (kCentred<R, SQRT>) from_centred(ref, sm.at(c, i - i0), x);
+      traj_store<!SQRT, R, NX>(out_m, out_L, out_inter, i, sm.at(c, i - i0), x, L);
     }
-    traj_store<!SQRT, R, NX>(out_m, out_L, out_inter, Mp, i, sm(i), m, L);
     if (ell_state != nullptr) ell_state[i] = e;
   }
 }
@@ -735,7 +709,7 @@ template <typename R, int NX, int NY, bool SQRT, typename FB = Fallback>
 __global__ __launch_bounds__(kLaneWG) void k_smoother_reduce(
     int64_t M, int64_t Mp, int chunk, int64_t nchunks, const int64_t* __restrict__ soff, int nseq,
     const R* __restrict__ lin, const R* __restrict__ fm, const R* __restrict__ fL, int f_inter,
-    R* __restrict__ elems, R* __restrict__ agg, LevelMap lm, FB fb) {
+    const R* __restrict__ ref, R* __restrict__ elems, R* __restrict__ agg, LevelMap lm, FB fb) {
   if (fb.skip()) return;
   const StateMap sm{chunk};
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -748,7 +722,9 @@ __global__ __launch_bounds__(kLaneWG) void k_smoother_reduce(
   for (int64_t i = i1 - 1; i >= i0; --i) {
     while (i < soff[s]) --s;
     R m[NX], L[NX][NX];
-    traj_load<!SQRT, R, NX>(fm, fL, f_inter, Mp, i, sm(i), m, L);
+    const int64_t pos = sm.at(c, i - i0);
+    traj_load<!SQRT, R, NX>(fm, fL, f_inter, i, pos, m, L);
+    if constexpr (kCentred<R, SQRT>) to_centred(ref, pos, m);
     SAgg<R, NX> e;
     if (i == soff[s + 1] - 1) {
       copy(m, e.g);
@@ -756,26 +732,33 @@ __global__ __launch_bounds__(kLaneWG) void k_smoother_reduce(
       copy(L, e.D);
       e.flag = FLAG_HEAD;
     } else {
+      // a caller's filtered factors may be any square roots
+      if constexpr (SQRT) {
+        if (!f_inter) lower_factor(L);
+      }
       R F[NX][NX], cq[NX][NX], bt[NX];
+      const R* p = blk<Step<R, NX, NY>::NQ>(lin, pos);
       int q = 0;
-      const int64_t pi = sm(i);
-      ld(lin, Mp, pi, q, F);
-      ld_tri<!SQRT>(lin, Mp, pi, q, cq);
-      ld(lin, Mp, pi, q, bt);
+      ld(p, kBlk, 0, q, F);
+      ld_tri<!SQRT>(p, kBlk, 0, q, cq);
+      ld(p, kBlk, 0, q, bt);
       smoother_element_fb<R, NX, SQRT>(F, cq, bt, m, L, e, fb);
     }
-    store_agg(elems, Mp, sm(i), e);
+    store_agg(elems, pos, e);
+    if constexpr (SQRT) {
+      if (!f_inter && e.flag == FLAG_HEAD) lower_factor(e.D);
+    }
     combine_into_fb<R, NX, SQRT>(acc, e, fb);
     copy_agg(e, acc);
   }
-  store_agg(agg, lm.stride, lm.pos(c), acc);
+  store_agg(agg, lm.pos(c), acc);
 }
 
 template <typename R, int NX, bool SQRT, typename FB = Fallback>
 __global__ __launch_bounds__(kLaneWG) void k_smoother_apply(
     int64_t M, int64_t Mp, int chunk, int64_t nchunks, const R* __restrict__ elems,
-    const R* __restrict__ prefix, LevelMap lm, const R* __restrict__ upper, LevelMap um,
-    R* __restrict__ joined, R* __restrict__ out_m, R* __restrict__ out_L, int out_inter, FB fb) {
+    ScanLevels<R> lv, const R* __restrict__ ref, R* __restrict__ out_m, R* __restrict__ out_L, int out_inter,
+    FB fb) {
   if (fb.skip()) return;
   const StateMap sm{chunk};
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -783,24 +766,33 @@ __global__ __launch_bounds__(kLaneWG) void k_smoother_apply(
   const int64_t i0 = c * chunk;
   const int64_t i1 = min(i0 + chunk, M);
   R m[NX], D[NX][NX];
-  {
-    int64_t pc;
-    const R* src = level0_prefix<SAgg<R, NX>, R, SQRT>(c, prefix, lm, upper, um, joined, fb, &pc);
-    int q = 0;
-    ld(src, lm.stride, pc, q, m);
-    q += NX * NX;
-    ld(src, lm.stride, pc, q, D);
-  }
+  set_zero(m);
+  set_zero(D);
+  enter_chunk<SView<R, NX>>(c, lv, m, D, [&](const SView<R, NX>& v, R (&mm)[NX], R (&DD)[NX][NX]) {
+    SAgg<R, NX> e;
+    view_load(v, e);
+    smoother_apply_fb<R, NX, SQRT>(e, mm, DD, fb);
+  });
   for (int64_t i = i1 - 1; i >= i0; --i) {
     SAgg<R, NX> e;
-    load_agg(elems, Mp, sm(i), e);
+    load_agg(elems, sm.at(c, i - i0), e);
     if (e.flag == FLAG_HEAD) {
       copy(e.g, m);
       copy(e.D, D);
     } else {
       smoother_apply_fb<R, NX, SQRT>(e, m, D, fb);
     }
-    traj_store<!SQRT, R, NX>(out_m, out_L, out_inter, Mp, i, sm(i), m, D);
+    R x[NX];
+    copy(m, x);
+    if constexpr (kCentred<R, SQRT>) from_centred(ref, sm.at(c, i - i0), x);
+    if (e.flag == FLAG_HEAD) {
+      // the last filtered factor goes out as it is; the recursion and the
+      // interleaved trajectory take its lower triangular form
+      if (!out_inter) st_aos(out_L, i, D);
+      if constexpr (SQRT) lower_factor(D);
+    }
+    if (out_inter || e.flag != FLAG_HEAD) traj_store<!SQRT, R, NX>(out_m, out_L, out_inter, i, sm.at(c, i - i0), x, D);
+    else st_aos(out_m, i, x);
   }
 }
 
@@ -842,6 +834,10 @@ __global__ __launch_bounds__(kLaneWG) void k_filter_elements(
   ld_aos(m, i, mm_);
   ld_aos(L, i, LL);
   ld_aos(y, i, yy);
+  if constexpr (SQRT) {  // a caller's factors may be any square roots
+    lower_factor(s.cq);
+    lower_factor(LL);
+  }
   FAgg<R, NX> e;
   filter_element<R, NX, NY, SQRT>(s, mm_, LL, yy, e);
   st_aos(A, i, e.A);
@@ -872,6 +868,12 @@ __global__ __launch_bounds__(kLaneWG) void k_filter_combine(int64_t n, FPtrs<R, 
   ld_aos(b.p[3], i, e2.eta); ld_aos(b.p[4], i, e2.Z);
   e1.flag = FLAG_NORMAL;
   e2.flag = FLAG_NORMAL;
+  if constexpr (SQRT) {  // a caller's factors may be any square roots
+    lower_factor(e1.U);
+    lower_factor(e1.Z);
+    lower_factor(e2.U);
+    lower_factor(e2.Z);
+  }
   combine_into<R, NX, SQRT>(e1, e2);
   st_aos(o.p[0], i, e2.A); st_aos(o.p[1], i, e2.b); st_aos(o.p[2], i, e2.U);
   st_aos(o.p[3], i, e2.eta); st_aos(o.p[4], i, e2.Z);
@@ -890,6 +892,10 @@ __global__ __launch_bounds__(kLaneWG) void k_smoother_elements(
   ld_aos(bt, i, bti);
   ld_aos(m, i, mi);
   ld_aos(L, i, Li);
+  if constexpr (SQRT) {  // a caller's factors may be any square roots
+    lower_factor(cqi);
+    lower_factor(Li);
+  }
   SAgg<R, NX> e;
   smoother_element<R, NX, SQRT>(Fi, cqi, bti, mi, Li, e);
   st_aos(g, i, e.g);
@@ -916,6 +922,10 @@ __global__ __launch_bounds__(kLaneWG) void k_smoother_combine(int64_t n, SPtrs<R
   ld_aos(b.p[0], i, e2.g); ld_aos(b.p[1], i, e2.E); ld_aos(b.p[2], i, e2.D);
   e1.flag = FLAG_NORMAL;
   e2.flag = FLAG_NORMAL;
+  if constexpr (SQRT) {  // a caller's factors may be any square roots
+    lower_factor(e1.D);
+    lower_factor(e2.D);
+  }
   combine_into<R, NX, SQRT>(e1, e2);
   st_aos(o.p[0], i, e2.g); st_aos(o.p[1], i, e2.E); st_aos(o.p[2], i, e2.D);
 }

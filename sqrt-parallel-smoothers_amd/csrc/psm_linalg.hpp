@@ -160,51 +160,161 @@ PSM_DEV void copy(const R (&a)[N], R (&b)[N]) {
 }
 
 // ----------------------------------------------------------------------------
+// Householder pivots
+// ----------------------------------------------------------------------------
+// Reflecting the rows of a matrix from the right so that the pivot row x
+// becomes (||x||, 0, ..., 0) maps another row m to
+//     m_0' = p / ||x||,   m_j' = m_j - t x_j  (j > 0),   p = <x, m>,
+//     t = (p / ||x|| + sgn(x_0) m_0) / (||x|| + |x_0|)
+// (the reflector v = x + sgn(x_0) ||x|| e_0, which never cancels, with the
+// first column's sign flipped where that gives -||x||).  p needs the pivot row
+// only, so the inner products of every row run beside the chain that forms the
+// norm, its reciprocal and 1 / (||x|| + |x_0|); a pivot then costs one square
+// root and one reciprocal in sequence.  A pivot row without a norm (exactly
+// zero, or below the range of its square) reflects nothing: f, gs and inv are
+// zero and keep is one.  Applied to the pivot row itself the map gives
+// (||x||, 0, ..., 0), so a kernel may update all rows alike.
+template <typename R>
+struct Pivot {
+  R nrm;   // ||x||
+  R inv;   // 1 / ||x||
+  R f;     // 1 / (||x|| (||x|| + |x_0|))
+  R gs;    // sgn(x_0) / (||x|| + |x_0|)
+  R keep;  // 1 for a pivot row without a norm, else 0
+};
+
+// Smallest ||x||^2 a pivot divides by: the products of its reciprocals stay finite.
+template <typename R> PSM_DEV constexpr double pivot_min() { return 1e-290; }
+template <> PSM_DEV constexpr double pivot_min<float>() { return 1.2e-38; }
+
+// s = sqrt(x), r = 1 / sqrt(x) for a normal, positive x.
+PSM_DEV void sqrt_inv_(double x, double& s, double& r) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double e = fma(-g, h, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  s = fma(fma(-g, g, x), h, g);
+  r = h + h;
+  r = fma(fma(-s, r, 1.0), r, r);
+}
+PSM_DEV void sqrt_inv_(float x, float& s, float& r) {
+  s = sqrtf(x);
+  r = __builtin_amdgcn_rsqf(x);
+}
+template <typename R>
+PSM_DEV void sqrt_inv_(R x, R& s, R& r) {
+  s = sqrt_(x);
+  r = rcp_(s);
+}
+
+// The pivot of a row with first entry x0 and squared norm n2.
+template <typename R>
+PSM_DEV Pivot<R> make_pivot(R x0, R n2) {
+  const bool ok = !(n2 <= R(pivot_min<R>()));  // NaN passes through the norm
+  Pivot<R> p;
+  R s, r;
+  sqrt_inv_(ok ? n2 : R(1), s, r);
+  const R g = rcp_(s + abs_(x0));
+  p.nrm = ok ? s : abs_(x0);
+  p.inv = ok ? r : R(0);
+  p.f = ok ? r * g : R(0);
+  p.gs = ok ? (x0 < R(0) ? -g : g) : R(0);
+  p.keep = ok ? R(0) : R(1);
+  return p;
+}
+
+// Active columns of pivot i of a matrix [X | T] with NL columns on the left and,
+// on the right, NT columns whose lower-triangular shape the pivots keep (row k
+// holds columns NL..NL + k): columns i..NL - 1 and NL..NL + min(i, NT - 1).
+// With NT = 0 it is a plain matrix.
+template <int NL, int NT>
+PSM_DEV constexpr bool pivot_column(int i, int j) {
+  return (j >= i && j < NL) || (j >= NL && j - NL <= i && j - NL < NT);
+}
+
+// Squared norm of pivot row x at pivot i, in two chains.
+template <int NL, int NT, typename R, int NC>
+PSM_DEV R pivot_norm2(const R (&x)[NC], int i) {
+  R a = x[i] * x[i], b = R(0);
+  bool odd = true;
+#pragma unroll
+  for (int j = 0; j < NC; ++j)
+    if (j != i && pivot_column<NL, NT>(i, j)) {
+      if (odd) b = fma(x[j], x[j], b);
+      else a = fma(x[j], x[j], a);
+      odd = !odd;
+    }
+  return a + b;
+}
+
+// Row m reflected by pivot row x at pivot i.
+template <int NL, int NT, typename R, int NC>
+PSM_DEV void pivot_apply(const Pivot<R>& pv, const R (&x)[NC], R (&m)[NC], int i) {
+  R a = x[i] * m[i], b = R(0);
+  bool odd = true;
+#pragma unroll
+  for (int j = 0; j < NC; ++j)
+    if (j != i && pivot_column<NL, NT>(i, j)) {
+      if (odd) b = fma(x[j], m[j], b);
+      else a = fma(x[j], m[j], a);
+      odd = !odd;
+    }
+  const R p = a + b;
+  const R t = fma(pv.gs, m[i], p * pv.f);
+  m[i] = fma(pv.keep, m[i], p * pv.inv);
+#pragma unroll
+  for (int j = 0; j < NC; ++j)
+    if (j != i && pivot_column<NL, NT>(i, j)) m[j] = fma(-t, x[j], m[j]);
+}
+
+// ----------------------------------------------------------------------------
 // tria: in-place Householder triangularisation from the right.
 // On exit M[:, :min(ROWS,COLS)] holds L (lower, non-negative diagonal) and the
 // remaining columns are zero.
 // ----------------------------------------------------------------------------
-template <typename R, int ROWS, int COLS>
-PSM_DEV void tria_inplace(R (&M)[ROWS][COLS]) {
-  constexpr int NR = ROWS < COLS ? ROWS : COLS;
+// The first NP pivots of [X | T] (columns as in pivot_column); the pivot rows
+// are left reduced to their diagonal entry, the columns of later pivots and T
+// keep what the reflections leave there.
+template <int NL, int NT, int NP, typename R, int ROWS, int NC>
+PSM_DEV void tria_pivots(R (&M)[ROWS][NC]) {
 #pragma unroll
-  for (int i = 0; i < NR; ++i) {
-    const R alpha = M[i][i];
-    R sigma = R(0);
+  for (int i = 0; i < NP; ++i) {
+    const Pivot<R> pv = make_pivot(M[i][i], pivot_norm2<NL, NT>(M[i], i));
 #pragma unroll
-    for (int j = i + 1; j < COLS; ++j) sigma = fma(M[i][j], M[i][j], sigma);
-    const R nrm = sqrt_(fma(alpha, alpha, sigma));
-    // v = x - ||x|| e0, computed without cancellation (Parlett's formula).
-    const R v0 = (alpha > R(0)) ? -sigma * rcp_(alpha + nrm) : alpha - nrm;
-    const R vv = fma(v0, v0, sigma);
-    const R f = (vv > R(0)) ? R(2) * rcp_(vv) : R(0);
+    for (int k = i + 1; k < ROWS; ++k) pivot_apply<NL, NT>(pv, M[i], M[k], i);
+    M[i][i] = pv.nrm;
 #pragma unroll
-    for (int k = i + 1; k < ROWS; ++k) {
-      R dot = v0 * M[k][i];
-#pragma unroll
-      for (int j = i + 1; j < COLS; ++j) dot = fma(M[i][j], M[k][j], dot);
-      const R t = f * dot;
-      M[k][i] = fma(-t, v0, M[k][i]);
-#pragma unroll
-      for (int j = i + 1; j < COLS; ++j) M[k][j] = fma(-t, M[i][j], M[k][j]);
-    }
-    M[i][i] = nrm;
-#pragma unroll
-    for (int j = i + 1; j < COLS; ++j) M[i][j] = R(0);
+    for (int j = 0; j < NC; ++j)
+      if (j != i && pivot_column<NL, NT>(i, j)) M[i][j] = R(0);
   }
 }
 
+template <typename R, int ROWS, int COLS>
+PSM_DEV void tria_inplace(R (&M)[ROWS][COLS]) {
+  constexpr int NR = ROWS < COLS ? ROWS : COLS;
+  tria_pivots<COLS, 0, NR>(M);
+}
+
+// tria of [X | T], X ROWS x NL with ROWS <= NL, T lower triangular.
+template <int NL, typename R, int ROWS>
+PSM_DEV void tria_lower_inplace(R (&M)[ROWS][NL + ROWS]) {
+  tria_pivots<NL, ROWS, ROWS>(M);
+}
+
 // A lower-triangular square root of C C^T: C itself when it is lower
-// triangular, else tria(C).  The linearized-model layout keeps only the lower
-// triangle of a noise factor, and a caller's factor (the extended
-// linearization passes chol Q through) may be any square root.
+// triangular, else tria(C).  The recursions and the operators take lower
+// triangular factors, and a caller's (the prior's, a filtered trajectory's,
+// chol Q, which the extended linearization passes through) may be any square root.
+template <typename R>
+PSM_DEV bool nonzero_(R x) { return x != R(0); }
 template <typename R, int N>
 PSM_DEV void lower_factor(R (&C)[N][N]) {
   bool upper = false;
 #pragma unroll
   for (int a = 0; a < N; ++a)
 #pragma unroll
-    for (int b = a + 1; b < N; ++b) upper = upper || (C[a][b] != R(0));
+    for (int b = a + 1; b < N; ++b) upper = upper || nonzero_(C[a][b]);
   if (upper) tria_inplace<R, N, N>(C);
 }
 

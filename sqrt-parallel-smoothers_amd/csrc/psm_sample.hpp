@@ -28,10 +28,10 @@ inline int64_t sample_chunk(int64_t M) {
 }
 
 template <typename R, int NX, bool SQRT>
-PSM_DEV void sample_element(const R* __restrict__ elems, int64_t Mp, int64_t pos,
+PSM_DEV void sample_element(const R* __restrict__ elems, int64_t pos,
                             const R* __restrict__ eps, R (&E)[NX][NX], R (&e)[NX]) {
   SAgg<R, NX> a;
-  load_agg(elems, Mp, pos, a);
+  load_agg(elems, pos, a);
   copy(a.E, E);
   R L[NX][NX];
   if constexpr (SQRT) {
@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kLaneWG) void k_sample_reduce(
   set_zero(ov);
   for (int64_t k = i1 - 1; k >= i0; --k) {
     R E[NX][NX], e[NX];
-    sample_element<R, NX, SQRT>(elems, Mp, sm(k), eps + (k * S + s) * NX, E, e);
+    sample_element<R, NX, SQRT>(elems, sm(k), eps + (k * S + s) * NX, E, e);
     R Pn[NX][NX], on[NX];
     mm(E, Pm, Pn);
     mv(E, ov, on);
@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kLaneWG) void k_sample_bounds(int64_t nch, int S,
 template <typename R, int NX, bool SQRT>
 __global__ __launch_bounds__(kLaneWG) void k_sample_apply(
     int64_t M, int64_t Mp, int chunk, int64_t Cs, int64_t nch, int S, const R* __restrict__ elems,
-    const R* __restrict__ eps, const R* __restrict__ xb, R* __restrict__ out) {
+    const R* __restrict__ eps, const R* __restrict__ xb, const R* __restrict__ ref, R* __restrict__ out) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nch * S) return;
   const int64_t c = t / S;
@@ -116,11 +116,13 @@ __global__ __launch_bounds__(kLaneWG) void k_sample_apply(
   else set_zero(x);
   for (int64_t k = i1 - 1; k >= i0; --k) {
     R E[NX][NX], e[NX], xn[NX];
-    sample_element<R, NX, SQRT>(elems, Mp, sm(k), eps + (k * S + s) * NX, E, e);
+    sample_element<R, NX, SQRT>(elems, sm(k), eps + (k * S + s) * NX, E, e);
     mv(E, x, xn);
 #pragma unroll
     for (int i = 0; i < NX; ++i) x[i] = xn[i] + e[i];
-    st_aos(out, k * S + s, x);
+    copy(x, xn);
+    if constexpr (kCentred<R, SQRT>) from_centred(ref, sm(k), xn);
+    st_aos(out, k * S + s, xn);
   }
 }
 

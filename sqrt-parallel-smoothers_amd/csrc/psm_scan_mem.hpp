@@ -16,6 +16,8 @@ struct FView {
   R* base;
   int64_t stride;
   int64_t idx;
+  static constexpr int NXV = NX;
+  static constexpr int QUNIT = 0;   // first field of the identity's unit matrix (A)
   static constexpr int QA = 0, QB = NX * NX, QU = NX * NX + NX, QE = 2 * NX * NX + NX,
                        QZ = 2 * NX * NX + 2 * NX, QF = 3 * NX * NX + 2 * NX;
   PSM_DEV R& at(int q) const { return base[(int64_t)q * stride + idx]; }
@@ -34,6 +36,8 @@ struct SView {
   R* base;
   int64_t stride;
   int64_t idx;
+  static constexpr int NXV = NX;
+  static constexpr int QUNIT = NX;  // first field of the identity's unit matrix (E)
   static constexpr int QG = 0, QE = NX, QD = NX + NX * NX, QF = NX + 2 * NX * NX;
   PSM_DEV R& at(int q) const { return base[(int64_t)q * stride + idx]; }
   PSM_DEV R& g(int i) const { return at(QG + i); }
@@ -69,166 +73,125 @@ PSM_DEV void view_identity(const SView<R, NX>& d) {
 }
 
 // ---------------------------------------------------------------- square-root filter
+// The rows of FilterArray (psm_core.hpp) one after the other: the reduced pivot
+// rows stay in registers and every other row is read, reflected and used up.
 template <typename R, int NX, typename C = R>
 PSM_DEV void sqrt_combine_mem(const FView<R, NX>& e1, const FView<R, NX>& e2,
                               const FView<R, NX>& out) {
-  C X[2 * NX][2 * NX];
-#pragma unroll
-  for (int i = 0; i < NX; ++i)
-#pragma unroll
-    for (int j = 0; j < NX; ++j) {
-      C acc = C(0);
-#pragma unroll
-      for (int k = 0; k < NX; ++k) acc = fma((C)e1.U(k, i), (C)e2.Z(k, j), acc);
-      X[i][j] = acc;
-      X[i][NX + j] = (i == j) ? C(1) : C(0);
-      X[NX + i][j] = (C)e2.Z(i, j);
-      X[NX + i][NX + j] = C(0);
-    }
-  tria_inplace<C, 2 * NX, 2 * NX>(X);
-  // M1 = U1 Xi11^{-T}
-  C M1[NX][NX];
-#pragma unroll
-  for (int j = 0; j < NX; ++j) {
-    const C inv = rcp_(X[j][j]);
-#pragma unroll
-    for (int r = 0; r < NX; ++r) {
-      C s = (C)e1.U(r, j);
-#pragma unroll
-      for (int k = 0; k < j; ++k) s = fma(-M1[r][k], X[j][k], s);
-      M1[r][j] = s * inv;
-    }
-  }
-  // P = I - M1 Xi21^T
-  C Pm[NX][NX];
-#pragma unroll
-  for (int i = 0; i < NX; ++i)
-#pragma unroll
-    for (int j = 0; j < NX; ++j) {
-      C acc = (i == j) ? C(1) : C(0);
-#pragma unroll
-      for (int k = 0; k < NX; ++k) acc = fma(-M1[i][k], X[NX + j][k], acc);
-      Pm[i][j] = acc;
-    }
-  // v = b1 + U1 (U1^T eta2) ; w = eta2 - Z2 (Z2^T b1)   (last reads of e2.eta, e2.Z)
-  C v[NX], w[NX];
+  FilterArray<C, NX> q;
+  C w[NX], r[2 * NX], Vt[NX][NX];
   {
-    C t1[NX], t2[NX];
+    C Z2[NX][NX];
 #pragma unroll
-    for (int j = 0; j < NX; ++j) {
-      C a1 = C(0), a2 = C(0);
+    for (int k = 0; k < NX; ++k)
 #pragma unroll
-      for (int k = 0; k < NX; ++k) {
-        a1 = fma((C)e1.U(k, j), (C)e2.eta(k), a1);
-        a2 = fma((C)e2.Z(k, j), (C)e1.b(k), a2);
-      }
-      t1[j] = a1;
-      t2[j] = a2;
-    }
+      for (int j = 0; j <= k; ++j) Z2[k][j] = (C)e2.Z(k, j);
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
-      C a1 = (C)e1.b(i), a2 = (C)e2.eta(i);
+      C u[NX];
 #pragma unroll
-      for (int k = 0; k < NX; ++k) {
-        a1 = fma((C)e1.U(i, k), t1[k], a1);
-        a2 = fma(-(C)e2.Z(i, k), t2[k], a2);
-      }
-      v[i] = a1;
-      w[i] = a2;
-    }
-  }
-  // eta = A1^T P^T w + eta1
-  {
-    C PTw[NX];
-#pragma unroll
-    for (int j = 0; j < NX; ++j) {
-      C a = C(0);
-#pragma unroll
-      for (int k = 0; k < NX; ++k) a = fma(Pm[k][j], w[k], a);
-      PTw[j] = a;
-    }
-#pragma unroll
-    for (int i = 0; i < NX; ++i) {
-      C a = (C)e1.eta(i);
-#pragma unroll
-      for (int k = 0; k < NX; ++k) a = fma((C)e1.A(k, i), PTw[k], a);
-      out.eta(i) = (R)(a);
-    }
-  }
-  // Z = tria([A1^T Xi22 | Z1])
-  {
-    C Zc[NX][2 * NX];
-#pragma unroll
-    for (int i = 0; i < NX; ++i)
+      for (int k = i; k < NX; ++k) u[k] = (C)e1.U(k, i);
 #pragma unroll
       for (int j = 0; j < NX; ++j) {
         C acc = C(0);
 #pragma unroll
-        for (int k = j; k < NX; ++k) acc = fma((C)e1.A(k, i), X[NX + k][NX + j], acc);
-        Zc[i][j] = acc;
-        Zc[i][NX + j] = (C)e1.Z(i, j);
+        for (int k = (i > j ? i : j); k < NX; ++k) acc = fma(u[k], Z2[k][j], acc);
+        q.x[i][j] = acc;
       }
-    tria_inplace<C, NX, 2 * NX>(Zc);
+    }
+    q.reduce();
+    C b1[NX], eta2[NX];
+#pragma unroll
+    for (int k = 0; k < NX; ++k) {
+      b1[k] = (C)e1.b(k);
+      eta2[k] = (C)e2.eta(k);
+    }
+    innovation(b1, eta2, Z2, w);
+#pragma unroll
+    for (int j = 0; j < NX; ++j) {
+      C acc = (C)e1.U(j, j) * w[j];
+#pragma unroll
+      for (int k = j + 1; k < NX; ++k) acc = fma((C)e1.U(k, j), w[k], acc);
+      r[j] = C(0);
+      r[NX + j] = acc;
+    }
+    q.reflect(r);
+    // [A1^T Z2 | 0] -> [V^T | Y]: eta and Z = tria([Y | Z1])
+    C Zc[NX][2 * NX], eta[NX];
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      C row[2 * NX], a1[NX];
+      C h = (C)e1.eta(i);
+#pragma unroll
+      for (int k = 0; k < NX; ++k) {
+        a1[k] = (C)e1.A(k, i);
+        h = fma(a1[k], w[k], h);
+      }
+#pragma unroll
+      for (int j = 0; j < NX; ++j) {
+        C acc = a1[j] * Z2[j][j];
+#pragma unroll
+        for (int k = j + 1; k < NX; ++k) acc = fma(a1[k], Z2[k][j], acc);
+        row[j] = acc;
+        row[NX + j] = C(0);
+      }
+      q.reflect(row);
+#pragma unroll
+      for (int j = 0; j < NX; ++j) {
+        Vt[i][j] = row[j];
+        Zc[i][j] = row[NX + j];
+        Zc[i][NX + j] = (C)e1.Z(i, j);
+        h = fma(-row[j], r[j], h);
+      }
+      eta[i] = h;
+    }
+#pragma unroll
+    for (int i = 0; i < NX; ++i) out.eta(i) = (R)eta[i];
+    tria_lower_inplace<NX>(Zc);
 #pragma unroll
     for (int i = 0; i < NX; ++i)
 #pragma unroll
       for (int j = 0; j < NX; ++j) out.Z(i, j) = (R)(Zc[i][j]);
   }
-  // PA1 = P A1 ; Pv = P v
-  C PA1[NX][NX], Pv[NX];
+  // [0 | A2 U1] -> [S | .]: A, b and U = tria([S | U2])
+  C Uc[NX][2 * NX];
 #pragma unroll
   for (int i = 0; i < NX; ++i) {
+    C row[2 * NX], a2[NX];
+    C bb = (C)e2.b(i);
+#pragma unroll
+    for (int k = 0; k < NX; ++k) {
+      a2[k] = (C)e2.A(i, k);
+      bb = fma(a2[k], (C)e1.b(k), bb);
+    }
+#pragma unroll
+    for (int j = 0; j < NX; ++j) {
+      C acc = a2[j] * (C)e1.U(j, j);
+#pragma unroll
+      for (int k = j + 1; k < NX; ++k) acc = fma(a2[k], (C)e1.U(k, j), acc);
+      row[j] = C(0);
+      row[NX + j] = acc;
+    }
+    q.reflect(row);
 #pragma unroll
     for (int j = 0; j < NX; ++j) {
       C acc = C(0);
 #pragma unroll
-      for (int k = 0; k < NX; ++k) acc = fma(Pm[i][k], (C)e1.A(k, j), acc);
-      PA1[i][j] = acc;
+      for (int k = 0; k < NX; ++k) acc = fma(a2[k], (C)e1.A(k, j), acc);
+#pragma unroll
+      for (int k = 0; k < NX; ++k) acc = fma(-row[k], Vt[j][k], acc);
+      out.A(i, j) = (R)acc;
+      Uc[i][j] = row[j];
+      Uc[i][NX + j] = (C)e2.U(i, j);
+      bb = fma(row[j], r[j], bb);
     }
-    C a = C(0);
-#pragma unroll
-    for (int k = 0; k < NX; ++k) a = fma(Pm[i][k], v[k], a);
-    Pv[i] = a;
+    out.b(i) = (R)bb;
   }
-  // S = A2 M1 ; A = A2 PA1 ; b = A2 Pv + b2    (last reads of e2.A, e2.b)
-  C S[NX][NX];
+  tria_lower_inplace<NX>(Uc);
 #pragma unroll
-  for (int i = 0; i < NX; ++i) {
-    C a2[NX];
+  for (int i = 0; i < NX; ++i)
 #pragma unroll
-    for (int k = 0; k < NX; ++k) a2[k] = (C)e2.A(i, k);
-    C bb = (C)e2.b(i);
-#pragma unroll
-    for (int k = 0; k < NX; ++k) bb = fma(a2[k], Pv[k], bb);
-#pragma unroll
-    for (int j = 0; j < NX; ++j) {
-      C s1 = C(0), s2 = C(0);
-#pragma unroll
-      for (int k = 0; k < NX; ++k) {
-        s1 = fma(a2[k], M1[k][j], s1);
-        s2 = fma(a2[k], PA1[k][j], s2);
-      }
-      S[i][j] = s1;
-      out.A(i, j) = (R)(s2);
-    }
-    out.b(i) = (R)(bb);
-  }
-  // U = tria([S | U2])
-  {
-    C Uc[NX][2 * NX];
-#pragma unroll
-    for (int i = 0; i < NX; ++i)
-#pragma unroll
-      for (int j = 0; j < NX; ++j) {
-        Uc[i][j] = S[i][j];
-        Uc[i][NX + j] = (C)e2.U(i, j);
-      }
-    tria_inplace<C, NX, 2 * NX>(Uc);
-#pragma unroll
-    for (int i = 0; i < NX; ++i)
-#pragma unroll
-      for (int j = 0; j < NX; ++j) out.U(i, j) = (R)(Uc[i][j]);
-  }
+    for (int j = 0; j < NX; ++j) out.U(i, j) = (R)(Uc[i][j]);
 }
 
 // ---------------------------------------------------------------- square-root smoother
@@ -267,7 +230,7 @@ PSM_DEV void sqrt_smoother_combine_mem(const SView<R, NX>& e1, const SView<R, NX
       out.E(i, j) = (R)(acc);
     }
   }
-  tria_inplace<C, NX, 2 * NX>(M);
+  tria_lower_inplace<NX>(M);
 #pragma unroll
   for (int i = 0; i < NX; ++i)
 #pragma unroll
@@ -417,6 +380,166 @@ PSM_DEV void combine_mem_fb(const V& e1, const V& e2, const V& out, const FB& fb
         sqrt_smoother_combine_mem<R, NX, double>(e1, e2, out);
       count_fallback(fb);
     }
+  }
+}
+
+// The distribution a HEAD aggregate is: (b, U) of a filter's, (g, D) of a smoother's.
+template <typename R, int NX>
+PSM_DEV void view_head(const FView<R, NX>& v, R (&m)[NX], R (&L)[NX][NX]) {
+#pragma unroll
+  for (int i = 0; i < NX; ++i) {
+    m[i] = v.b(i);
+#pragma unroll
+    for (int j = 0; j < NX; ++j) L[i][j] = v.U(i, j);
+  }
+}
+template <typename R, int NX>
+PSM_DEV void view_head(const SView<R, NX>& v, R (&m)[NX], R (&L)[NX][NX]) {
+#pragma unroll
+  for (int i = 0; i < NX; ++i) {
+    m[i] = v.g(i);
+#pragma unroll
+    for (int j = 0; j < NX; ++j) L[i][j] = v.D(i, j);
+  }
+}
+
+// (m, L) (+) e2: the filtering operator with a distribution on the left (A1, eta1
+// and Z1 are zero), of which only b and U are left to form (see FilterArray).
+template <typename R, int NX, typename C>
+PSM_DEV void sqrt_filter_push(const FView<R, NX>& e2, C (&m)[NX], C (&L)[NX][NX]) {
+  FilterArray<C, NX> q;
+  C r[2 * NX];
+  {
+    C Z2[NX][NX];
+#pragma unroll
+    for (int k = 0; k < NX; ++k)
+#pragma unroll
+      for (int j = 0; j <= k; ++j) Z2[k][j] = (C)e2.Z(k, j);
+#pragma unroll
+    for (int i = 0; i < NX; ++i)
+#pragma unroll
+      for (int j = 0; j < NX; ++j) {
+        C acc = C(0);
+#pragma unroll
+        for (int k = (i > j ? i : j); k < NX; ++k) acc = fma(L[k][i], Z2[k][j], acc);
+        q.x[i][j] = acc;
+      }
+    C eta2[NX], w[NX];
+#pragma unroll
+    for (int k = 0; k < NX; ++k) eta2[k] = (C)e2.eta(k);
+    innovation(m, eta2, Z2, w);
+    innovation_row(L, w, r);
+  }
+  q.reduce();
+  q.reflect(r);
+  C Uc[NX][2 * NX], b[NX];
+#pragma unroll
+  for (int i = 0; i < NX; ++i) {
+    C row[2 * NX], a2[NX];
+    C bb = (C)e2.b(i);
+#pragma unroll
+    for (int k = 0; k < NX; ++k) {
+      a2[k] = (C)e2.A(i, k);
+      bb = fma(a2[k], m[k], bb);
+    }
+#pragma unroll
+    for (int j = 0; j < NX; ++j) {
+      C acc = a2[j] * L[j][j];
+#pragma unroll
+      for (int k = j + 1; k < NX; ++k) acc = fma(a2[k], L[k][j], acc);
+      row[j] = C(0);
+      row[NX + j] = acc;
+    }
+    q.reflect(row);
+#pragma unroll
+    for (int j = 0; j < NX; ++j) {
+      Uc[i][j] = row[j];
+      Uc[i][NX + j] = (C)e2.U(i, j);
+      bb = fma(row[j], r[j], bb);
+    }
+    b[i] = bb;
+  }
+  tria_lower_inplace<NX>(Uc);
+#pragma unroll
+  for (int i = 0; i < NX; ++i) {
+    m[i] = b[i];
+#pragma unroll
+    for (int j = 0; j < NX; ++j) L[i][j] = Uc[i][j];
+  }
+}
+
+// The same for the covariance form (std_combine_core with A1, eta1 and J1 zero).
+template <typename R, int NX>
+PSM_DEV void std_filter_push(const FView<R, NX>& e2, R (&m)[NX], R (&P)[NX][NX]) {
+  // X1 = A2 (I + C1 J2)^{-1} via (I + C1 J2)^T X1^T = A2^T
+  R M1[NX][NX], B1[NX][NX];
+#pragma unroll
+  for (int i = 0; i < NX; ++i)
+#pragma unroll
+    for (int j = 0; j < NX; ++j) {
+      R s1 = (i == j) ? R(1) : R(0);
+#pragma unroll
+      for (int k = 0; k < NX; ++k) s1 = fma(P[j][k], e2.Z(k, i), s1);
+      M1[i][j] = s1;
+      B1[i][j] = e2.A(j, i);
+    }
+  solve_general<R, NX, NX>(M1, B1);   // B1 = X1^T
+  R t[NX], CA[NX][NX];
+#pragma unroll
+  for (int i = 0; i < NX; ++i) {
+    R a = P[i][0] * e2.eta(0);
+#pragma unroll
+    for (int k = 1; k < NX; ++k) a = fma(P[i][k], e2.eta(k), a);
+    t[i] = a + m[i];
+#pragma unroll
+    for (int j = 0; j < NX; ++j) {
+      R c = P[i][0] * e2.A(j, 0);
+#pragma unroll
+      for (int k = 1; k < NX; ++k) c = fma(P[i][k], e2.A(j, k), c);
+      CA[i][j] = c;                    // C1 A2^T
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NX; ++i) {
+    R b = B1[0][i] * t[0];
+#pragma unroll
+    for (int k = 1; k < NX; ++k) b = fma(B1[k][i], t[k], b);
+    m[i] = b + e2.b(i);
+#pragma unroll
+    for (int j = 0; j < NX; ++j) {
+      R c = B1[0][i] * CA[0][j];
+#pragma unroll
+      for (int k = 1; k < NX; ++k) c = fma(B1[k][i], CA[k][j], c);
+      P[i][j] = c + e2.U(i, j);
+    }
+  }
+}
+
+// (m, L) <- aggregate v applied to (m, L), with the FP64 recomputation of an
+// ill-conditioned FP32 factor.
+template <typename R, int NX, bool SQRT, typename FB>
+PSM_DEV void filter_push_fb(const FView<R, NX>& v, R (&m)[NX], R (&L)[NX][NX], const FB& fb) {
+  if constexpr (!SQRT) {
+    std_filter_push<R, NX>(v, m, L);
+  } else if constexpr (kFallback<R, SQRT> && !FB::kRedo) {
+    sqrt_filter_push<R, NX, R>(v, m, L);
+    if (fb.thr > 0.f && ill_conditioned(L, fb.thr)) fb.raise();
+  } else if constexpr (kFallback<R, SQRT>) {
+    R m0[NX], L0[NX][NX];
+    copy(m, m0);
+    copy(L, L0);
+    sqrt_filter_push<R, NX, R>(v, m, L);
+    if (fb.thr > 0.f && ill_conditioned(L, fb.thr)) {
+      double md[NX], Ld[NX][NX];
+      cvt(m0, md);
+      cvt(L0, Ld);
+      sqrt_filter_push<R, NX, double>(v, md, Ld);
+      cvt(md, m);
+      cvt(Ld, L);
+      count_fallback(fb);
+    }
+  } else {
+    sqrt_filter_push<R, NX, R>(v, m, L);
   }
 }
 

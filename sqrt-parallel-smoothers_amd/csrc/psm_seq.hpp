@@ -28,13 +28,13 @@ PSM_DEV void seq_predict(const R (&F)[NX][NX], const R (&cq)[NX][NX], const R (&
     for (int i = 0; i < NX; ++i)
 #pragma unroll
       for (int j = 0; j < NX; ++j) {
-        R acc = R(0);
+        R acc = F[i][j] * L[j][j];
 #pragma unroll
-        for (int k = 0; k < NX; ++k) acc = fma(F[i][k], L[k][j], acc);
+        for (int k = j + 1; k < NX; ++k) acc = fma(F[i][k], L[k][j], acc);
         M[i][j] = acc;
         M[i][NX + j] = cq[i][j];
       }
-    tria_inplace<R, NX, 2 * NX>(M);
+    tria_lower_inplace<NX>(M);
 #pragma unroll
     for (int i = 0; i < NX; ++i)
 #pragma unroll
@@ -81,6 +81,8 @@ __global__ __launch_bounds__(kLaneWG) void k_seq_filter(
   ld_aos(L0, s, L);
   st_aos(out_m, a, m);
   st_aos(out_L, a, L);
+  // the recursion takes lower triangular factors; a caller's may be any square roots
+  if constexpr (SQRT) lower_factor(L);
   Acc acc = Acc(0.0);
   for (int64_t i = a + 1; i < e; ++i) {
     Step<R, NX, NY> st_;
@@ -94,6 +96,7 @@ __global__ __launch_bounds__(kLaneWG) void k_seq_filter(
     }
     tr.row = i - 1;
     linearize_point_w<R, NX, NX, SQRT>(tr, sp, use_sigma, rm, rL, st_.F, st_.cq, st_.bt, fb);
+    if constexpr (SQRT) lower_factor(st_.cq);
     if (nom_m != nullptr) {
       ld_aos(nom_m, i, rm);
       ld_aos(nom_L, i, rL);
@@ -128,6 +131,7 @@ __global__ __launch_bounds__(kLaneWG) void k_seq_smoother(
   ld_aos(fL, e - 1, D);
   st_aos(out_m, e - 1, m);
   st_aos(out_L, e - 1, D);
+  if constexpr (SQRT) lower_factor(D);
   for (int64_t i = e - 2; i >= a; --i) {
     R rm[NX], rL[NX][NX];
     if (nom_m != nullptr) {
@@ -140,9 +144,11 @@ __global__ __launch_bounds__(kLaneWG) void k_seq_smoother(
     R F[NX][NX], cq[NX][NX], bt[NX];
     tr.row = i;
     linearize_point_w<R, NX, NX, SQRT>(tr, sp, use_sigma, rm, rL, F, cq, bt, fb);
+    if constexpr (SQRT) lower_factor(cq);
     R xm[NX], xL[NX][NX];
     ld_aos(fm, i, xm);
     ld_aos(fL, i, xL);
+    if constexpr (SQRT) lower_factor(xL);
     SAgg<R, NX> el;
     smoother_element_fb<R, NX, SQRT>(F, cq, bt, xm, xL, el, fb);
     smoother_apply_fb<R, NX, SQRT>(el, m, D, fb);
