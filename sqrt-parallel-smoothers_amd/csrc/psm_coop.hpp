@@ -48,10 +48,14 @@ PSM_DEV void group_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Keeps the scheduler from moving instructions across a phase of a combination:
-// it would otherwise hoist the operand loads of later phases far ahead and hold
-// them in more registers than two wavefronts per SIMD have.
-#define PSM_PHASE() __builtin_amdgcn_sched_barrier(0)
+// Keeps the scheduler from moving instructions across a phase of a combination by
+// a quad: it would otherwise hoist the operand loads of later phases far ahead and
+// hold them in more registers than two wavefronts per SIMD have.  With one or two
+// rows a lane there is room, and the phases overlap.
+template <int G>
+PSM_DEV void phase() {
+  if constexpr (G == 4) __builtin_amdgcn_sched_barrier(0);
+}
 // Forms x here: results that only some lanes store would otherwise be sunk into
 // that branch, behind the closing triangularisations, their operands live until then.
 template <typename R>
@@ -280,7 +284,7 @@ PSM_DEV bool CoopResult<FView<R, NX>, G>::compute(const R* e1, const R* e2, int 
       for (int k = j + 1; k < n; ++k) wu[j] = fma((C)e1[V::QU + k * n + j], w[k], wu[j]);
     }
   }
-  PSM_PHASE();
+  phase<G>();
 
   // rows of the array: a row of coefficients times the lower triangular Z2 or U1
   C x[NS][2 * n], a[ZS][n];
@@ -329,7 +333,7 @@ PSM_DEV bool CoopResult<FView<R, NX>, G>::compute(const R* e1, const R* e2, int 
         x[s][n + j] = kind == ROW_R ? wu[j] : x[s][n + j];
       }
     }
-    PSM_PHASE();
+    phase<G>();
   });
 
   static_for<0, n>([&](auto ic) {
@@ -346,7 +350,7 @@ PSM_DEV bool CoopResult<FView<R, NX>, G>::compute(const R* e1, const R* e2, int 
       if constexpr (L::live(s, i)) pivot_apply<n, n>(pv, bx, x[s], i);
     });
   });
-  PSM_PHASE();
+  phase<G>();
 
   // A = A2 A1 - S V on the lanes of the U rows (computed on all)
   static_for<0, n>([&](auto jc) {
@@ -368,7 +372,7 @@ PSM_DEV bool CoopResult<FView<R, NX>, G>::compute(const R* e1, const R* e2, int 
       A[s][j] = (R)(p - q);
       form_now(A[s][j]);
     });
-    PSM_PHASE();
+    phase<G>();
   });
 
   // eta = A1^T w + eta1 - V^T r on the low half, b = A2 b1 + b2 + S r on the high one
@@ -400,7 +404,7 @@ PSM_DEV bool CoopResult<FView<R, NX>, G>::compute(const R* e1, const R* e2, int 
       form_now(h[s]);
     });
   }
-  PSM_PHASE();
+  phase<G>();
 
   // Z = tria([Y | Z1]) and U = tria([S | U2]), side by side
   C mn = C(0), mx = C(0);
@@ -516,7 +520,7 @@ PSM_DEV bool CoopResult<SView<R, NX>, G>::compute(const R* e1, const R* e2, int 
       form_now(E[s][j]);
     }
   });
-  PSM_PHASE();
+  phase<G>();
   C mn = C(0), mx = C(0);
   static_for<0, n>([&](auto ic) {
     constexpr int i = decltype(ic)::value;

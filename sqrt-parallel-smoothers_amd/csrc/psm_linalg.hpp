@@ -15,6 +15,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #define PSM_DEV __device__ __forceinline__
 
 namespace psm {
@@ -187,25 +189,34 @@ struct Pivot {
 template <typename R> PSM_DEV constexpr double pivot_min() { return 1e-290; }
 template <> PSM_DEV constexpr double pivot_min<float>() { return 1.2e-38; }
 
-// s = sqrt(x), r = 1 / sqrt(x) for a normal, positive x.
-PSM_DEV void sqrt_inv_(double x, double& s, double& r) {
+// s = sqrt(x), r = 1 / s and g = 1 / (s + a) for a normal, positive x and a >= 0.
+// FP64: the hardware reciprocal square root refined as in sqrt_; the reciprocal's
+// hardware estimate is taken from the unrefined root, beside the refinement, and
+// its two Newton steps use the refined sum.
+PSM_DEV void pivot_scalars(double x, double a, double& s, double& r, double& g) {
   const double y = __builtin_amdgcn_rsq(x);
-  double g = x * y, h = 0.5 * y;
-  const double e = fma(-g, h, 0.5);
-  g = fma(g, e, g);
+  double q = x * y, h = 0.5 * y;
+  g = __builtin_amdgcn_rcp(q + a);
+  const double e = fma(-q, h, 0.5);
+  q = fma(q, e, q);
   h = fma(h, e, h);
-  s = fma(fma(-g, g, x), h, g);
+  s = fma(fma(-q, q, x), h, q);
   r = h + h;
   r = fma(fma(-s, r, 1.0), r, r);
+  const double d = s + a;
+  g = fma(g, fma(-d, g, 1.0), g);
+  g = fma(g, fma(-d, g, 1.0), g);
 }
-PSM_DEV void sqrt_inv_(float x, float& s, float& r) {
+PSM_DEV void pivot_scalars(float x, float a, float& s, float& r, float& g) {
   s = sqrtf(x);
   r = __builtin_amdgcn_rsqf(x);
+  g = rcp_(s + a);
 }
 template <typename R>
-PSM_DEV void sqrt_inv_(R x, R& s, R& r) {
+PSM_DEV void pivot_scalars(R x, R a, R& s, R& r, R& g) {
   s = sqrt_(x);
   r = rcp_(s);
+  g = rcp_(s + a);
 }
 
 // The pivot of a row with first entry x0 and squared norm n2.
@@ -213,13 +224,18 @@ template <typename R>
 PSM_DEV Pivot<R> make_pivot(R x0, R n2) {
   const bool ok = !(n2 <= R(pivot_min<R>()));  // NaN passes through the norm
   Pivot<R> p;
-  R s, r;
-  sqrt_inv_(ok ? n2 : R(1), s, r);
-  const R g = rcp_(s + abs_(x0));
+  R s, r, g;
+  if constexpr (std::is_floating_point<R>::value) {
+    pivot_scalars(n2, abs_(x0), s, r, g);      // whatever they are of a row without a norm, they go unused
+  } else {
+    pivot_scalars(ok ? n2 : R(1), abs_(x0), s, r, g);   // a tangent of theirs would not
+  }
+  r = ok ? r : R(0);
+  g = ok ? g : R(0);
   p.nrm = ok ? s : abs_(x0);
-  p.inv = ok ? r : R(0);
-  p.f = ok ? r * g : R(0);
-  p.gs = ok ? (x0 < R(0) ? -g : g) : R(0);
+  p.inv = r;
+  p.f = r * g;
+  p.gs = x0 < R(0) ? -g : g;
   p.keep = ok ? R(0) : R(1);
   return p;
 }
