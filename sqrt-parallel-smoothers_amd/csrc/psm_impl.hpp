@@ -623,20 +623,26 @@ struct Impl {
 
   // ---------------------------------------------------------------- sampling
   struct SamplePlan {
-    int64_t Cs, nch;
-    size_t off_P, off_o, off_xb, total;
+    int64_t Cs, nch, ngr;
+    size_t off_P, off_o, off_xb, off_P2, off_o2, off_xg, total;
   };
   static SamplePlan sample_plan(const Plan& pl, int S) {
     SamplePlan sp;
     sp.Cs = sample_chunk(pl.M);
     sp.nch = (pl.M + sp.Cs - 1) / sp.Cs;
+    sp.ngr = (sp.nch + sp.Cs - 1) / sp.Cs;
     size_t off = pl.total;
-    sp.off_P = off;
-    off = align_up(off + (size_t)sp.nch * NX * NX * sizeof(R));
-    sp.off_o = off;
-    off = align_up(off + (size_t)sp.nch * S * NX * sizeof(R));
-    sp.off_xb = off;
-    off = align_up(off + (size_t)sp.nch * S * NX * sizeof(R));
+    auto take = [&](int64_t words) {
+      const size_t at = off;
+      off = align_up(off + (size_t)words * sizeof(R));
+      return at;
+    };
+    sp.off_P = take(sp.nch * NX * NX);
+    sp.off_o = take(sp.nch * S * NX);
+    sp.off_xb = take(sp.nch * S * NX);
+    sp.off_P2 = take(sp.ngr * NX * NX);
+    sp.off_o2 = take(sp.ngr * S * NX);
+    sp.off_xg = take(sp.ngr * S * NX);
     sp.total = off;
     return sp;
   }
@@ -666,18 +672,28 @@ struct Impl {
                          (const R*)(ws + pl.off_ref), (R*)(ws + pl.off_selem), (R*)(ws + pl.lv[0].off_in), level_map(pl, 0, 1), f);
     });
     if ((rc = hip_check("k_smoother_reduce"))) return rc;
-    const int64_t lanes = sp.nch * S;
-    hipLaunchKernelGGL((k_sample_reduce<R, NX, SQRT>), dim3(grid_for(lanes, kLaneWG)), dim3(kLaneWG),
-                       0, st, pl.M, pl.Mp, pl.chunk, sp.Cs, sp.nch, S, (const R*)(ws + pl.off_selem),
-                       (const R*)eps, (R*)(ws + sp.off_P), (R*)(ws + sp.off_o));
-    if ((rc = hip_check("k_sample_reduce"))) return rc;
-    hipLaunchKernelGGL((k_sample_bounds<R, NX>), dim3(grid_for(S, kLaneWG)), dim3(kLaneWG), 0, st,
-                       sp.nch, S, (const R*)(ws + sp.off_P), (const R*)(ws + sp.off_o),
-                       (R*)(ws + sp.off_xb));
-    if ((rc = hip_check("k_sample_bounds"))) return rc;
-    hipLaunchKernelGGL((k_sample_apply<R, NX, SQRT>), dim3(grid_for(lanes, kLaneWG)), dim3(kLaneWG),
-                       0, st, pl.M, pl.Mp, pl.chunk, sp.Cs, sp.nch, S, (const R*)(ws + pl.off_selem),
-                       (const R*)eps, (const R*)(ws + sp.off_xb), (const R*)(ws + pl.off_ref), (R*)out);
+    const R* el = (const R*)(ws + pl.off_selem);
+    R *P = (R*)(ws + sp.off_P), *o = (R*)(ws + sp.off_o), *xb = (R*)(ws + sp.off_xb);
+    R *P2 = (R*)(ws + sp.off_P2), *o2 = (R*)(ws + sp.off_o2), *xg = (R*)(ws + sp.off_xg);
+    if (sp.nch > 1) {
+      hipLaunchKernelGGL((k_sample_reduce<R, NX, SQRT>), dim3(grid_for(sp.nch * (S + NX), kLaneWG)),
+                         dim3(kLaneWG), 0, st, pl.M, pl.chunk, sp.Cs, sp.nch, S, el, (const R*)eps, P, o);
+      if ((rc = hip_check("k_sample_reduce"))) return rc;
+      if (sp.ngr > 1) {
+        hipLaunchKernelGGL((k_sample_fold<R, NX>), dim3(grid_for(sp.ngr * (S + NX), kLaneWG)), dim3(kLaneWG), 0, st,
+                           sp.nch, sp.Cs, sp.ngr, S, (const R*)P, (const R*)o, P2, o2);
+        if ((rc = hip_check("k_sample_fold"))) return rc;
+        hipLaunchKernelGGL((k_sample_bounds<R, NX>), dim3(grid_for(S, kLaneWG)), dim3(kLaneWG), 0, st,
+                           sp.ngr, S, (const R*)P2, (const R*)o2, xg);
+        if ((rc = hip_check("k_sample_bounds"))) return rc;
+      }
+      hipLaunchKernelGGL((k_sample_spread<R, NX>), dim3(grid_for(sp.ngr * S, kLaneWG)), dim3(kLaneWG), 0, st,
+                         sp.nch, sp.Cs, sp.ngr, S, (const R*)P, (const R*)o, (const R*)xg, xb);
+      if ((rc = hip_check("k_sample_spread"))) return rc;
+    }
+    hipLaunchKernelGGL((k_sample_apply<R, NX, SQRT>), dim3(grid_for(sp.nch * S, kLaneWG)), dim3(kLaneWG), 0, st,
+                       pl.M, pl.chunk, sp.Cs, sp.nch, S, el, (const R*)eps, (const R*)xb,
+                       (const R*)(ws + pl.off_ref), (R*)out);
     return hip_check("k_sample_apply");
   }
 
