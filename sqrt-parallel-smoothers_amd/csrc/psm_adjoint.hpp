@@ -131,7 +131,15 @@ PSM_DEV void ld_cv(const S* __restrict__ p, int64_t i, D (&v)[N1][N2]) {
 // ---------------------------------------------------------------- per-state buffers
 // FP64 component-major arrays over the states, positions interleaved by
 // StateMap{C} (C = kChunk) so that lane-per-chunk scans read consecutive words.
-constexpr int kChunk = 32;
+//
+// Items per lane of a scan level.  A level is a chain of kChunk steps per launch
+// (1 to 2 us each: the loads' latency) and the levels of M states form a chain of
+// about 2 kChunk log M / log kChunk steps, so a short chunk is the shorter chain
+// while a level does not fill the chip: 65,600 states take 88 steps in 11 launches
+// per scan, 224 in 7 with 32.  The four scans of a step took 1.18 ms with 32 and
+// without the item loaded ahead (each_item), 0.49 with 8.  The aggregates of all
+// levels are a seventh of the states.
+constexpr int kChunk = 8;
 
 template <int N>
 PSM_DEV void ldv(const D* __restrict__ b, int64_t st, int64_t p, int q0, D (&v)[N]) {
@@ -852,6 +860,28 @@ PSM_DEV void step_z(const D (&Mj)[NX][NX], const D (&w)[Sc<NX, CONG>::NW], D (&z
   }
 }
 
+// fn(j, M, w) over the items [j0, j1), with the next item in flight while one is
+// used where both fit in registers.
+template <int NX, bool CONG, typename IO, typename Fn>
+PSM_DEV void each_item(const IO& io, int64_t j0, int64_t j1, Fn fn) {
+  using S = Sc<NX, CONG>;
+  constexpr bool kAhead = !CONG || NX <= 5;
+  D Mj[NX][NX], w[S::NW];
+  if constexpr (kAhead) io.load(j0, Mj, w);
+  for (int64_t j = j0; j < j1; ++j) {
+    if constexpr (kAhead) {
+      D Mn[NX][NX], wn[S::NW];
+      io.load(j + 1 < j1 ? j + 1 : j, Mn, wn);
+      fn(j, Mj, w);
+      copy(Mn, Mj);
+      copy(wn, w);
+    } else {
+      io.load(j, Mj, w);
+      fn(j, Mj, w);
+    }
+  }
+}
+
 // aggregates of chunks of C positions: (prod M, offset of the chunk applied to 0)
 template <int NX, bool CONG, int SRC>
 __global__ __launch_bounds__(64) void k_ascan_reduce(int64_t n, ScanIO<NX, CONG, SRC> io, D* __restrict__ up,
@@ -864,13 +894,12 @@ __global__ __launch_bounds__(64) void k_ascan_reduce(int64_t n, ScanIO<NX, CONG,
   D Ma[NX][NX], z[S::NW];
   set_eye(Ma);
   set_zero(z);
-  for (int64_t j = j0; j < j1; ++j) {
-    D Mj[NX][NX], w[S::NW], T[NX][NX];
-    io.load(j, Mj, w);
+  each_item<NX, CONG>(io, j0, j1, [&](int64_t, const D(&Mj)[NX][NX], const D(&w)[S::NW]) {
+    D T[NX][NX];
     step_z<NX, CONG>(Mj, w, z);
     mm(Mj, Ma, T);
     copy(T, Ma);
-  }
+  });
   const int64_t p = StateMap{kChunk}(c);
   stm(up, ust, p, S::QM, Ma);
   stv(up, ust, p, S::QW, z);
@@ -889,12 +918,10 @@ __global__ __launch_bounds__(64) void k_ascan_apply(int64_t n, ScanIO<NX, CONG, 
   D z[S::NW];
   if (c == 0 || up == nullptr) set_zero(z);
   else ldv(up, ust, StateMap{kChunk}(c - 1), S::QZ, z);
-  for (int64_t j = j0; j < j1; ++j) {
-    D Mj[NX][NX], w[S::NW];
-    io.load(j, Mj, w);
+  each_item<NX, CONG>(io, j0, j1, [&](int64_t j, const D(&Mj)[NX][NX], const D(&w)[S::NW]) {
     step_z<NX, CONG>(Mj, w, z);
     io.store(j, z);
-  }
+  });
 }
 
 // ---------------------------------------------------------------- pass items
