@@ -722,7 +722,13 @@ struct Impl {
       obv.npts = use ? sv.npts : 0;
       const Fallback fb{p->fallback_ratio, p->fallback_count};
       TimedScope ts_("k_seq_filter", st);
-      hipLaunchKernelGGL((k_seq_filter<R, NX, NY, SQRT>), dim3(grid_for(p->n_seq, kLaneWG)),
+      if (nm != nullptr && p->n_seq <= kAheadMaxSeqs)
+        hipLaunchKernelGGL((k_seq_filter_ahead<R, NX, NY, SQRT>), dim3(grid_for(p->n_seq, 64)),
+                           dim3(64 * (1 + SeqFilterAhead<R, NX, NY>::P)), 0, st, p->n_seq, p->state_offsets,
+                           trv, obv, sv, use, (const R*)nm, (const R*)nL, (const R*)ys, (const R*)m0,
+                           (const R*)L0, (R*)om, (R*)oL, ell, fb);
+      else
+        hipLaunchKernelGGL((k_seq_filter<R, NX, NY, SQRT>), dim3(grid_for(p->n_seq, kLaneWG)),
                          dim3(kLaneWG), 0, st, p->n_seq, p->state_offsets, trv, obv, sv, use,
                          (const R*)nm, (const R*)nL, (const R*)ys, (const R*)m0, (const R*)L0,
                          (R*)om, (R*)oL, ell, fb);
@@ -743,7 +749,12 @@ struct Impl {
       trv.npts = use ? sv.npts : 0;
       const Fallback fb{p->fallback_ratio, p->fallback_count};
       TimedScope ts_("k_seq_smoother", st);
-      hipLaunchKernelGGL((k_seq_smoother<R, NX, SQRT>), dim3(grid_for(p->n_seq, kLaneWG)),
+      if (nm != nullptr && p->n_seq <= kAheadMaxSeqs)
+        hipLaunchKernelGGL((k_seq_smoother_ahead<R, NX, SQRT>), dim3(grid_for(p->n_seq, 64)),
+                           dim3(64 * (1 + SeqSmootherAhead<R, NX>::P)), 0, st, p->n_seq, p->state_offsets, trv,
+                           sv, use, (const R*)nm, (const R*)nL, (const R*)fm, (const R*)fL, (R*)om, (R*)oL, fb);
+      else
+        hipLaunchKernelGGL((k_seq_smoother<R, NX, SQRT>), dim3(grid_for(p->n_seq, kLaneWG)),
                          dim3(kLaneWG), 0, st, p->n_seq, p->state_offsets, trv, sv, use,
                          (const R*)nm, (const R*)nL, (const R*)fm, (const R*)fL, (R*)om, (R*)oL,
                          fb);

@@ -157,4 +157,211 @@ __global__ __launch_bounds__(kLaneWG) void k_seq_smoother(
   }
 }
 
+// ---------------------------------------------------------------- ahead of the recursion
+// At a nominal trajectory the linearizations (and, smoothing, the whole smoother
+// elements) do not depend on the recursion.  A workgroup then takes 64 sequences
+// with one wavefront for the recursion and P more that form the next P steps
+// meanwhile, on SIMDs that a batch of up to 64 sequences per CU leaves idle:
+//   round r:  wavefront 1 + p forms step r P + p in registers, while wavefront 0
+//             takes its 64 sequences through the steps of round r - 1 from LDS;
+//             barrier; the new steps go to LDS; barrier.
+// Every lane takes part in every round of the longest of its 64 sequences.
+// 4,096 tracks of 20 to 100 steps, FP64: 345 us a filter and 235 a smoother pass,
+// 725 and 900 with all of a step on the recursion's lane.
+constexpr size_t kLdsBytes = 160 * 1024;
+template <int NW, typename R>
+constexpr int ahead_waves() {
+  return kLdsBytes / (NW * 64 * sizeof(R)) >= 3 ? 3 : (int)(kLdsBytes / (NW * 64 * sizeof(R)));
+}
+// With every workgroup on a CU of its own, the recursion's wavefront has a SIMD
+// to itself; beyond, the forming wavefronts would take the place of other
+// sequences' recursions.
+constexpr int kAheadMaxSeqs = 64 * 256;
+
+// longest of the 64 sequences' step counts, on every lane
+PSM_DEV int64_t wave_max(int64_t n) {
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+    const int64_t o = __shfl_xor((long long)n, d, 64);
+    n = o > n ? o : n;
+  }
+  return n;
+}
+
+// form(j): step j into registers; put(buf, lane): those to LDS; take(buf, lane, j)
+template <int P, int NW, typename R, typename Form, typename Put, typename Take>
+PSM_DEV void seq_ahead(R (&buf)[P][NW * 64], int64_t n, Form&& form, Put&& put, Take&& take) {
+  const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+  const int64_t rounds = (wave_max(n) + P - 1) / P;
+  for (int64_t r = 0; r <= rounds; ++r) {
+    const int64_t j = r * P + (wave - 1);
+    const bool forms = wave > 0 && j < n;
+    if (wave == 0) {
+      for (int p = 0; p < P; ++p) {
+        const int64_t i = (r - 1) * P + p;
+        if (i >= 0 && i < n) take(buf[p], lane, i);
+      }
+    } else if (forms) {
+      form(j);
+    }
+    __syncthreads();
+    if (forms) put(buf[wave - 1], lane);
+    __syncthreads();
+  }
+}
+
+template <typename R, int N1, int N2>
+PSM_DEV void put_words(R* b, int lane, int& q, const R (&a)[N1][N2]) {
+#pragma unroll
+  for (int i = 0; i < N1; ++i)
+#pragma unroll
+    for (int j = 0; j < N2; ++j) b[64 * q++ + lane] = a[i][j];
+}
+template <typename R, int N>
+PSM_DEV void put_words(R* b, int lane, int& q, const R (&a)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) b[64 * q++ + lane] = a[i];
+}
+template <typename R, int N1, int N2>
+PSM_DEV void take_words(const R* b, int lane, int& q, R (&a)[N1][N2]) {
+#pragma unroll
+  for (int i = 0; i < N1; ++i)
+#pragma unroll
+    for (int j = 0; j < N2; ++j) a[i][j] = b[64 * q++ + lane];
+}
+template <typename R, int N>
+PSM_DEV void take_words(const R* b, int lane, int& q, R (&a)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) a[i] = b[64 * q++ + lane];
+}
+
+template <typename R, int NX, int NY>
+struct SeqFilterAhead {
+  static constexpr int NW = 2 * NX * NX + NX + NY * NX + NY * NY + 2 * NY;
+  static constexpr int P = ahead_waves<NW, R>();
+};
+template <typename R, int NX, int NY, bool SQRT>
+__global__ __launch_bounds__(64 * (1 + SeqFilterAhead<R, NX, NY>::P)) void k_seq_filter_ahead(
+    int nseq, const int64_t* __restrict__ soff, ModelView<R> tr, ModelView<R> ob, SigmaView<R> sp,
+    int use_sigma, const R* __restrict__ nom_m, const R* __restrict__ nom_L,
+    const R* __restrict__ ys, const R* __restrict__ m0, const R* __restrict__ L0,
+    R* __restrict__ out_m, R* __restrict__ out_L, typename AccOf<R>::type* __restrict__ ell,
+    Fallback fb) {
+  using Acc = typename AccOf<R>::type;
+  constexpr int NW = SeqFilterAhead<R, NX, NY>::NW, P = SeqFilterAhead<R, NX, NY>::P;
+  __shared__ R buf[P][NW * 64];
+  const int s = blockIdx.x * 64 + ((int)threadIdx.x & 63);
+  const bool have = s < nseq;
+  const int64_t a = have ? soff[s] : 0, e = have ? soff[s + 1] : 1;
+  R m[NX], L[NX][NX];
+  if (have && threadIdx.x < 64) {
+    ld_aos(m0, s, m);
+    ld_aos(L0, s, L);
+    st_aos(out_m, a, m);
+    st_aos(out_L, a, L);
+    if constexpr (SQRT) lower_factor(L);
+  }
+  Acc acc = Acc(0.0);
+  Step<R, NX, NY> f;
+  R y[NY];
+  seq_ahead<P, NW>(buf, e - a - 1,
+    [&](int64_t j) {
+      const int64_t i = a + 1 + j;
+      R rm[NX], rL[NX][NX];
+      ld_aos(ys, i - s - 1, y);
+      ld_aos(nom_m, i - 1, rm);
+      ld_aos(nom_L, i - 1, rL);
+      tr.row = i - 1;
+      linearize_point_w<R, NX, NX, SQRT>(tr, sp, use_sigma, rm, rL, f.F, f.cq, f.bt, fb);
+      if constexpr (SQRT) lower_factor(f.cq);
+      ld_aos(nom_m, i, rm);
+      ld_aos(nom_L, i, rL);
+      ob.row = i;
+      linearize_point_w<R, NX, NY, SQRT>(ob, sp, use_sigma, rm, rL, f.H, f.cr, f.c, fb);
+    },
+    [&](R* b, int lane) {
+      int q = 0;
+      put_words(b, lane, q, f.F);
+      put_words(b, lane, q, f.cq);
+      put_words(b, lane, q, f.bt);
+      put_words(b, lane, q, f.H);
+      put_words(b, lane, q, f.cr);
+      put_words(b, lane, q, f.c);
+      put_words(b, lane, q, y);
+    },
+    [&](const R* b, int lane, int64_t j) {
+      Step<R, NX, NY> g;
+      R yy[NY];
+      int q = 0;
+      take_words(b, lane, q, g.F);
+      take_words(b, lane, q, g.cq);
+      take_words(b, lane, q, g.bt);
+      take_words(b, lane, q, g.H);
+      take_words(b, lane, q, g.cr);
+      take_words(b, lane, q, g.c);
+      take_words(b, lane, q, yy);
+      acc += kf_step_fb<R, NX, NY, SQRT>(g, yy, m, L, fb);
+      st_aos(out_m, a + 1 + j, m);
+      st_aos(out_L, a + 1 + j, L);
+    });
+  if (have && threadIdx.x < 64 && ell != nullptr) ell[s] = acc;
+}
+
+template <typename R, int NX>
+struct SeqSmootherAhead {
+  static constexpr int NW = 2 * NX * NX + NX;
+  static constexpr int P = ahead_waves<NW, R>();
+};
+template <typename R, int NX, bool SQRT>
+__global__ __launch_bounds__(64 * (1 + SeqSmootherAhead<R, NX>::P)) void k_seq_smoother_ahead(
+    int nseq, const int64_t* __restrict__ soff, ModelView<R> tr, SigmaView<R> sp, int use_sigma,
+    const R* __restrict__ nom_m, const R* __restrict__ nom_L, const R* __restrict__ fm,
+    const R* __restrict__ fL, R* __restrict__ out_m, R* __restrict__ out_L, Fallback fb) {
+  constexpr int NW = SeqSmootherAhead<R, NX>::NW, P = SeqSmootherAhead<R, NX>::P;
+  __shared__ R buf[P][NW * 64];
+  const int s = blockIdx.x * 64 + ((int)threadIdx.x & 63);
+  const bool have = s < nseq;
+  const int64_t a = have ? soff[s] : 0, e = have ? soff[s + 1] : 1;
+  R m[NX], D[NX][NX];
+  if (have && threadIdx.x < 64) {
+    ld_aos(fm, e - 1, m);
+    ld_aos(fL, e - 1, D);
+    st_aos(out_m, e - 1, m);
+    st_aos(out_L, e - 1, D);
+    if constexpr (SQRT) lower_factor(D);
+  }
+  SAgg<R, NX> el;
+  seq_ahead<P, NW>(buf, e - a - 1,
+    [&](int64_t j) {
+      const int64_t i = e - 2 - j;
+      R rm[NX], rL[NX][NX], F[NX][NX], cq[NX][NX], bt[NX];
+      ld_aos(nom_m, i, rm);
+      ld_aos(nom_L, i, rL);
+      tr.row = i;
+      linearize_point_w<R, NX, NX, SQRT>(tr, sp, use_sigma, rm, rL, F, cq, bt, fb);
+      if constexpr (SQRT) lower_factor(cq);
+      ld_aos(fm, i, rm);
+      ld_aos(fL, i, rL);
+      if constexpr (SQRT) lower_factor(rL);
+      smoother_element_fb<R, NX, SQRT>(F, cq, bt, rm, rL, el, fb);
+    },
+    [&](R* b, int lane) {
+      int q = 0;
+      put_words(b, lane, q, el.g);
+      put_words(b, lane, q, el.E);
+      put_words(b, lane, q, el.D);
+    },
+    [&](const R* b, int lane, int64_t j) {
+      SAgg<R, NX> g;
+      g.flag = 0;
+      int q = 0;
+      take_words(b, lane, q, g.g);
+      take_words(b, lane, q, g.E);
+      take_words(b, lane, q, g.D);
+      smoother_apply_fb<R, NX, SQRT>(g, m, D, fb);
+      st_aos(out_m, e - 2 - j, m);
+      st_aos(out_L, e - 2 - j, D);
+    });
+}
+
 }  // namespace psm

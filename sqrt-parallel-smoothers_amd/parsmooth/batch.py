@@ -31,8 +31,8 @@ def _noise_dim(model) -> int:
 
 
 # Lower bound of the sequential filter + smoother time per step of one lane
-# (measured: ~18 us in FP64 on MI355X for the bearings model).
-SEQ_STEP_MS_MIN = 0.004
+# (measured: 5.8 us in FP64 on MI355X for the bearings model).
+SEQ_STEP_MS_MIN = 0.0015
 
 
 class IteratedSmoother:
