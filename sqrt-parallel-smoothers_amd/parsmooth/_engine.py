@@ -4,6 +4,7 @@ one call into libparsmooth_hip.so."""
 from __future__ import annotations
 
 import ctypes
+import os
 from typing import Optional, Sequence
 
 import numpy as np
@@ -42,6 +43,27 @@ def compute_dtype(x0) -> torch.dtype:
     return torch.float64
 
 
+def states_per_chunk(n_states: int) -> int:
+    """States per chunk, 0 for the library's choice (4 to 16: 32,768 chunks).
+
+    A lane's chain through a state of its chunk is longer than one through a level
+    of the scan, and up to 4096 chunks (8192 with a fan-in of 2) the 16-lane scan has
+    three levels however many there are: few states take chunks as short as that
+    allows (six iterations, FP64, against 4: T = 200 638 us at 1, 843; 3,000 845 at
+    1, 1035; 6,000 942 at 2, 1118; 12,000 1079 at 3, 1159; 20,000 1235 at 3, 1299;
+    beyond 24,576 it takes a fourth level and gains 1 % either way).  Where the chip
+    is full many times over, the scan's share is what counts, and shrinks with the
+    chunk (FP32, two iterations: 1,024 ragged tracks of up to 4,096 4.12 ms at 24,
+    4.40 at 16; up to 8,192 7.50 at 40, 8.00; 4,096 of those 28.1 at 40, 29.2)."""
+    if n_states <= 3 * 4096:
+        return -(-n_states // 4096)
+    if n_states <= 3 * 8192:
+        return -(-n_states // 8192)
+    if n_states >= 1 << 21:
+        return 40 if n_states >= 1 << 22 else 24
+    return 0
+
+
 class Problem:
     """Dims, dtype, form and the sequence layout of one batch.
 
@@ -64,13 +86,18 @@ class Problem:
         self.dtype = dtype
         self.sqrt = sqrt
         self.dev = dev
-        self.state_offsets = torch.as_tensor(offs).to(dev)
+        # one sequence: [0, n_states] filled in on the device, since a copy from host
+        # memory would wait for what the stream still has to do
+        self.state_offsets = torch.arange(0, 2 * self.n_states, self.n_states, device=dev) \
+            if self.n_seq == 1 else torch.as_tensor(offs).to(dev)
         code = N.dtype_code(dtype) if tangent_code is None else int(tangent_code)
         if not N.lib().psm_supported(code, N.FORM_SQRT if sqrt else N.FORM_STD, self.nx, self.ny):
             raise NotImplementedError(f"no compiled kernels for nx={nx}, ny={ny}, dtype code {code}")
         # FP64 re-triangularisation fallback of the FP32 square-root path
         self.fallback_counter = torch.zeros(1, dtype=torch.int64, device=dev)
         ratio = FP32_FALLBACK_RATIO if (code in (N.PSM_F32, N.PSM_F32_TANGENT) and sqrt) else 0.0
+        if tangent_code is None and not chunk and "PSM_CHUNK" not in os.environ:
+            chunk = states_per_chunk(self.n_states)
         self.struct = N.PsmProblem(code, N.FORM_SQRT if sqrt else N.FORM_STD,
                                    self.nx, self.ny, self.n_seq, int(chunk), self.n_states,
                                    self.state_offsets.data_ptr(), float(ratio), 0,
