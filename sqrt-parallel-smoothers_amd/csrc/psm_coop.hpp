@@ -1,4 +1,4 @@
-// Cooperative square-root scan operators: G lanes run one combination.
+// Cooperative scan operators: G lanes run one combination.
 //
 // One lane running a whole combination issues a chain of thousands of dependent
 // instructions, and a scan level seldom has enough items to hide it.  Here a
@@ -7,7 +7,8 @@
 // being reduced (FilterArray in psm_core.hpp); a pivot row is broadcast inside
 // the group with DPP moves (no LDS round trip) and every lane reflects its own
 // rows, so a pivot costs its broadcast, one square root and one reciprocal
-// whatever the number of rows.
+// whatever the number of rows.  (The covariance form is dealt out by columns: see
+// its operators below.)
 //
 // The 3 n + 1 rows of the filtering array are dealt out so that the n rows that
 // become Z lie on the low half of the group and the n rows that become U on the
@@ -220,10 +221,10 @@ struct FilterRows {
 
 // The lane's part of a combination's result, held in registers until the group
 // may overwrite an operand.
-template <typename V, int G> struct CoopResult;
+template <typename V, int G, bool SQRT = true> struct CoopResult;
 
 template <typename R, int NX, int G>
-struct CoopResult<FView<R, NX>, G> {
+struct CoopResult<FView<R, NX>, G, true> {
   using V = FView<R, NX>;
   using L = FilterRows<NX, G>;
   static constexpr int n = NX, NS = L::NS, ZS = L::ZS, HL = L::HL;
@@ -258,7 +259,7 @@ struct CoopResult<FView<R, NX>, G> {
 
 template <typename R, int NX, int G>
 template <typename C, bool ILL>
-PSM_DEV bool CoopResult<FView<R, NX>, G>::compute(const R* e1, const R* e2, int r, float thr) {
+PSM_DEV bool CoopResult<FView<R, NX>, G, true>::compute(const R* e1, const R* e2, int r, float thr) {
   const bool high = r >= HL;
 
   // w = eta2 - Z2 (Z2^T b1) and w^T U1, on every lane
@@ -444,7 +445,7 @@ PSM_DEV bool CoopResult<FView<R, NX>, G>::compute(const R* e1, const R* e2, int 
 // forms the rows of D and the high half those of E; in a quad every lane forms
 // both of its rows.
 template <typename R, int NX, int G>
-struct CoopResult<SView<R, NX>, G> {
+struct CoopResult<SView<R, NX>, G, true> {
   using V = SView<R, NX>;
   static constexpr int n = NX;
   static constexpr bool SPLIT = G >= 2 * NX;
@@ -480,7 +481,7 @@ struct CoopResult<SView<R, NX>, G> {
 
 template <typename R, int NX, int G>
 template <typename C, bool ILL>
-PSM_DEV bool CoopResult<SView<R, NX>, G>::compute(const R* e1, const R* e2, int r, float thr) {
+PSM_DEV bool CoopResult<SView<R, NX>, G, true>::compute(const R* e1, const R* e2, int r, float thr) {
   const bool high = SPLIT && r >= RL;
   const int rr = high ? r - RL : r;
   C y[NS][2 * n];
@@ -548,6 +549,191 @@ PSM_DEV bool CoopResult<SView<R, NX>, G>::compute(const R* e1, const R* e2, int 
   return false;
 }
 
+// ---------------------------------------------------------------- covariance form
+// e1 (+) e2 of (A, b, C, eta, J) (parsmooth/parallel/_operators.py:22-44), C and J
+// symmetric.  With N = I + J2 C1 and w = eta2 - J2 b1 one elimination gives
+//   X1^T = N^-1 A2^T,  Y = N^-1 J2 A1,  y = N^-1 w
+// and the same two products with C1 and A2 all of
+//   C = (A2 C1 X1^T)^T + C2,  A = A2 (A1 - C1 Y),  b = A2 (b1 + C1 y) + b2,
+// and the one with A1^T  J = A1^T Y + J1,  eta = A1^T y + eta1.
+// (A and b so, as what they are without the second aggregate's information and a
+// correction, round less than by way of X1 A1 and X1 (b1 + C1 eta2).)
+// Every lane holds columns of [N | A2^T | J2 A1 | w] (3 n + 1 of them, 16 for n = 5):
+// a pivot is the broadcast of one column, on which every lane finds the same row
+// to exchange, and an update of n entries.  Eliminating above the diagonal as well
+// (Gauss-Jordan) takes the back substitution, and its n further broadcasts, out of
+// the chain.  A scan launch of 4097 states takes 13 us at n = 5 and one of 5004
+// states 24 at n = 6; the lane-per-combination kernel, which spills, 121 and 251.
+template <typename R, int NX, int G>
+struct CoopResult<FView<R, NX>, G, false> {
+  using V = FView<R, NX>;
+  static constexpr int n = NX, NC = 3 * n + 1, NS = (NC + G - 1) / G;
+  static_assert(n <= G, "the pivot columns lie in the first slot");
+  static constexpr bool has_info(int s) { return (s + 1) * G > 2 * n; }   // columns of Y and y
+  R z[NS][n];   // column of J, or eta
+  R o[NS][n];   // row of C, column of A, or b
+
+  PSM_DEV void write(R* out, int flag, int r) const {
+    static_for<0, NS>([&](auto sc) {
+      constexpr int s = decltype(sc)::value;
+      const int q = s * G + r;
+      const bool isx = q >= n && q < 2 * n, isw = q == 3 * n;
+      if (q >= n && q < NC) {
+        R* op = isx ? out + V::QU + (q - n) * n : isw ? out + V::QB : out + V::QA + (q - 2 * n);
+        const int step = isx || isw ? 1 : n;
+#pragma unroll
+        for (int k = 0; k < n; ++k) op[k * step] = o[s][k];
+      }
+      if constexpr (has_info(s)) {
+        if (q >= 2 * n && q < NC) {
+          R* op = isw ? out + V::QE : out + V::QZ + (q - 2 * n);
+          const int step = isw ? 1 : n;
+#pragma unroll
+          for (int k = 0; k < n; ++k) op[k * step] = z[s][k];
+        }
+      }
+    });
+    if (r == 0) out[V::QF] = R(flag);
+  }
+
+  template <typename C, bool ILL>
+  PSM_DEV bool compute(const R* e1, const R* e2, int r, float) {
+    static_assert(std::is_same<C, R>::value && !ILL, "no recomputation in this form");
+    R x[NS][n], v[NS][n];
+    static_for<0, NS>([&](auto sc) {
+      constexpr int s = decltype(sc)::value;
+      const int q = s * G + r;
+      const bool isn = q < n, isx = !isn && q < 2 * n, isj = !isn && !isx && q < 3 * n;
+      // column of C1, row of A2, column of A1, or b1
+      const R* ap = isn ? e1 + V::QU + q : isx ? e2 + V::QA + (q - n) * n : isj ? e1 + V::QA + (q - 2 * n) : e1 + V::QB;
+      const int step = isn || isj ? n : 1;
+#pragma unroll
+      for (int k = 0; k < n; ++k) v[s][k] = ap[k * step];
+#pragma unroll
+      for (int i = 0; i < n; ++i) {
+        R acc = e2[V::QZ + i * n] * v[s][0];
+#pragma unroll
+        for (int k = 1; k < n; ++k) acc = fma(e2[V::QZ + i * n + k], v[s][k], acc);
+        const R add = isn && i == q ? R(1) : R(0);
+        x[s][i] = isx ? v[s][i] : isn || isj ? acc + add : e2[V::QE + i] - acc;
+      }
+    });
+    static_for<0, n>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      R p[n];
+#pragma unroll
+      for (int k = 0; k < n; ++k) p[k] = from_lane<G, i>(x[0][k]);
+#pragma unroll
+      for (int k = i + 1; k < n; ++k) {
+        const bool sw = abs_(p[k]) > abs_(p[i]);
+        const R t = p[i];
+        p[i] = sw ? p[k] : t;
+        p[k] = sw ? t : p[k];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          const R u = x[s][i];
+          x[s][i] = sw ? x[s][k] : u;
+          x[s][k] = sw ? u : x[s][k];
+        }
+      }
+      const R inv = rcp_(p[i]);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        x[s][i] *= inv;
+#pragma unroll
+        for (int k = 0; k < n; ++k)
+          if (k != i) x[s][k] = fma(-p[k], x[s][i], x[s][k]);
+      }
+    });
+    static_for<0, NS>([&](auto sc) {
+      constexpr int s = decltype(sc)::value;
+      const int q = s * G + r;
+      const bool isx = q < 2 * n, isj = !isx && q < 3 * n, isw = q == 3 * n;
+      if constexpr (has_info(s)) {
+        const R* zp = isj ? e1 + V::QZ + (q - 2 * n) : e1 + V::QE;
+        const int step = isj ? n : 1;
+#pragma unroll
+        for (int j = 0; j < n; ++j) {
+          R acc = e1[V::QA + j] * x[s][0];
+#pragma unroll
+          for (int k = 1; k < n; ++k) acc = fma(e1[V::QA + k * n + j], x[s][k], acc);
+          z[s][j] = acc + zp[j * step];
+        }
+      }
+      R t[n];
+#pragma unroll
+      for (int j = 0; j < n; ++j) {
+        R acc = e1[V::QU + j * n] * x[s][0];
+#pragma unroll
+        for (int k = 1; k < n; ++k) acc = fma(e1[V::QU + j * n + k], x[s][k], acc);
+        t[j] = isx ? acc : isj ? v[s][j] - acc : v[s][j] + acc;
+      }
+      const R* op = isx ? e2 + V::QU + (q >= n ? q - n : 0) * n : e2 + V::QB;
+#pragma unroll
+      for (int j = 0; j < n; ++j) {
+        R acc = e2[V::QA + j * n] * t[0];
+#pragma unroll
+        for (int k = 1; k < n; ++k) acc = fma(e2[V::QA + j * n + k], t[k], acc);
+        o[s][j] = isx || isw ? acc + op[j] : acc;
+      }
+    });
+    return false;
+  }
+};
+
+// g = E2 g1 + g2, E = E2 E1, D = E2 D1 E2^T + D2 (parsmooth/parallel/_operators.py:95-101):
+// the low half forms the rows of D, the high half those of E.
+template <typename R, int NX, int G>
+struct CoopResult<SView<R, NX>, G, false> {
+  using V = SView<R, NX>;
+  static constexpr int n = NX, HL = G / 2;
+  static_assert(n <= HL, "one row per lane of a half");
+  R f[n], g;
+
+  PSM_DEV void write(R* out, int flag, int r) const {
+    const bool high = r >= HL;
+    const int i = high ? r - HL : r;
+    if (i < n) {
+      R* op = out + (high ? V::QE : V::QD) + i * n;
+      out[V::QG + i] = g;   // the same value on both halves
+#pragma unroll
+      for (int j = 0; j < n; ++j) op[j] = f[j];
+    }
+    if (r == 0) out[V::QF] = R(flag);
+  }
+
+  template <typename C, bool ILL>
+  PSM_DEV bool compute(const R* e1, const R* e2, int r, float) {
+    static_assert(std::is_same<C, R>::value && !ILL, "no recomputation in this form");
+    const bool high = r >= HL;
+    const int row = high ? r - HL : r;
+    const int i = row < n ? row : 0;
+    const R* mp = e1 + (high ? V::QE : V::QD);
+    R a[n], t[n];
+    g = R(0);
+#pragma unroll
+    for (int k = 0; k < n; ++k) {
+      a[k] = e2[V::QE + i * n + k];
+      g = fma(a[k], e1[V::QG + k], g);
+    }
+    g += e2[V::QG + i];
+#pragma unroll
+    for (int j = 0; j < n; ++j) {
+      t[j] = a[0] * mp[j];
+#pragma unroll
+      for (int k = 1; k < n; ++k) t[j] = fma(a[k], mp[k * n + j], t[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < n; ++j) {
+      R acc = e2[V::QD + i * n + j];
+#pragma unroll
+      for (int k = 0; k < n; ++k) acc = fma(e2[V::QE + j * n + k], t[k], acc);
+      f[j] = high ? t[j] : acc;
+    }
+    return false;
+  }
+};
+
 // One combination by a group, in two halves so that the result may overwrite an
 // operand of this or of another group: prepare() reads e1 and e2, commit() writes.
 // Between them the caller synchronises the groups that read what this one
@@ -555,10 +741,10 @@ PSM_DEV bool CoopResult<SView<R, NX>, G>::compute(const R* e1, const R* e2, int 
 // recomputation in FP64 when the combined factor is ill-conditioned (the rule
 // of combine_mem_fb).  The flags and the decision are the same on every lane of
 // a group, so the group stays together.
-template <typename V, int G>
+template <typename V, int G, bool SQRT>
 struct CoopStep {
   using R = typename V::real_type;
-  CoopResult<V, G> res;
+  CoopResult<V, G, SQRT> res;
   int flag = -1;   // of the result; negative: nothing to write
 
   // the result goes where e2 is (scan: e2 holds an item's running aggregate and
@@ -576,7 +762,7 @@ struct CoopStep {
       }
       return;
     }
-    constexpr bool FBK = kFallback<R, true>;
+    constexpr bool FBK = kFallback<R, SQRT>;
     const bool ill = res.template compute<R, FBK>(e1, e2, r, fb.thr);
     if constexpr (FBK && !FB::kRedo) {
       if (fb.thr > 0.f && ill && r == 0) fb.raise();

@@ -235,13 +235,14 @@ struct Impl {
   using Acc = typename AccOf<R>::type;
   // Level 0 of a scan (the chunk aggregates: many items) runs one lane per
   // combination with WG lanes per workgroup, or four (PSM_SCAN_QUAD) or sixteen
-  // (PSM_SCAN_ROW).  The square-root form in float / double runs the levels above
-  // (few items, a latency chain) with 16 lanes per combination, kRowVL
+  // (PSM_SCAN_ROW); the covariance form has no kernels for four lanes or half
+  // workgroups.  The levels above (few items, a latency chain) run in float /
+  // double with 16 lanes per combination, kRowVL
   // combinations per workgroup, when scan_k has the PSM_SCAN_TEAM bit, or by
   // default (scan_k without a fan-in; the PSM_SCAN_TEAM environment variable
   // set to 0 turns the default off).
-  static constexpr bool TEAM = SQRT && (std::is_same<R, float>::value ||
-                                        std::is_same<R, double>::value);
+  static constexpr bool TEAM = std::is_same<R, float>::value || std::is_same<R, double>::value;
+  static constexpr bool QUAD = TEAM && SQRT;
   static constexpr int WG = scan_wg<FA, R>() < scan_wg<SA, R>() ? scan_wg<FA, R>() : scan_wg<SA, R>();
 
   static bool team_requested(const psm_problem_t* p) {
@@ -261,23 +262,27 @@ struct Impl {
   // beyond, four lanes (T = 131,072: 1.59 ms against 1.67 and 1.89; the ragged
   // batches of 0.5 to 17 million states are 6 to 18 % faster than with one lane),
   // 32 groups per workgroup so that three workgroups share a CU's LDS.
+  // The covariance form's combination has one form with 16 lanes and one with one
+  // (which spills): 16 lanes at every size (one cubature pass of T = 4096 at 4 states
+  // a chunk: 207 us against 431 with one lane; up to T = 524,288 no one-lane schedule
+  // was among the best six).
   struct Level0 {
     int lanes, wg, k;
   };
   static Level0 default_level0(int64_t nchunks) {
     if (nchunks <= 4096) return Level0{16, kRowVL, 1};
-    if (nchunks <= 20000) return Level0{16, kRowVL, 2};
+    if (nchunks <= 20000 || !QUAD) return Level0{16, kRowVL, 2};
     return Level0{4, WG / 2, 2};
   }
 
   static Plan plan(const psm_problem_t* p) {
     const bool team = TEAM && team_requested(p);
-    const bool half = TEAM && (p->scan_k & PSM_SCAN_HALF) != 0;
+    const bool half = QUAD && (p->scan_k & PSM_SCAN_HALF) != 0;
     Level0 l0{1, half ? WG / 2 : WG, team ? 2 : 4};
     if (TEAM && (p->scan_k & PSM_SCAN_ROW)) {
       l0.lanes = 16;
       l0.wg = kRowVL;
-    } else if (TEAM && (p->scan_k & PSM_SCAN_QUAD)) {
+    } else if (QUAD && (p->scan_k & PSM_SCAN_QUAD)) {
       l0.lanes = 4;
     } else if (team && (p->scan_k & ~PSM_SCAN_TOP_MASK) == 0) {
       const int c = resolve_chunk(p);
@@ -468,7 +473,7 @@ struct Impl {
         using F = decltype(f);
         auto coop = [&](auto gl, auto vl) {
           constexpr int G = decltype(gl)::value, VL = decltype(vl)::value;
-          hipLaunchKernelGGL((k_scan_up_coop<Agg, R, G, VL, F>), dim3((unsigned)s.nwg), dim3(VL * G), 0, st,
+          hipLaunchKernelGGL((k_scan_up_coop<Agg, R, SQRT, G, VL, F>), dim3((unsigned)s.nwg), dim3(VL * G), 0, st,
                              (const R*)in, level_map(pl, l, 0), out, tot, tm, f);
         };
         auto lane = [&](auto vl) {
@@ -477,7 +482,7 @@ struct Impl {
                              (const R*)in, level_map(pl, l, 0), out, tot, tm, f);
         };
         using I = std::integral_constant<int, WG>;
-        if constexpr (TEAM) {
+        if constexpr (QUAD) {
           using H = std::integral_constant<int, WG / 2>;
           if (lanes == 16) {
             coop(std::integral_constant<int, 16>{}, std::integral_constant<int, kRowVL>{});
@@ -489,6 +494,9 @@ struct Impl {
           } else {
             lane(I{});
           }
+        } else if constexpr (TEAM) {
+          if (lanes == 16) coop(std::integral_constant<int, 16>{}, std::integral_constant<int, kRowVL>{});
+          else lane(I{});
         } else {
           lane(I{});
         }

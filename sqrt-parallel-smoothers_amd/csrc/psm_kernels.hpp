@@ -511,13 +511,13 @@ __global__ __launch_bounds__(WG) void k_scan_up(const R* __restrict__ in, LevelM
   }
 }
 
-// k_scan_up for the square-root form with G lanes per combination
+// k_scan_up with G lanes per combination
 // (psm_coop.hpp): VL groups per workgroup, each one virtual lane of the scan
 // above (folds K items, joins the Kogge-Stone scan over the groups, rewrites its
 // items' exclusive prefixes).  The level layout is that of k_scan_up with VL
 // lanes, so the two are interchangeable.  One call site combines in all three
 // parts, so the instructions of a combination are fetched once.
-template <typename Agg, typename R, int G, int VL, typename FB = Fallback>
+template <typename Agg, typename R, bool SQRT, int G, int VL, typename FB = Fallback>
 __global__ __launch_bounds__(VL * G) void k_scan_up_coop(
     const R* __restrict__ in, LevelMap lm, R* __restrict__ out_excl, R* __restrict__ totals,
     LevelMap tm, FB fb) {
@@ -592,7 +592,7 @@ __global__ __launch_bounds__(VL * G) void k_scan_up_coop(
       group_sync();
     }
     // an idle group keeps what it has: its running aggregate is e1 outside the scan
-    CoopStep<V, G> cs;
+    CoopStep<V, G, SQRT> cs;
     if (act) cs.prepare(e1, e2, !scan, rl, fb);
     if (scan) __syncthreads();
     else group_sync();

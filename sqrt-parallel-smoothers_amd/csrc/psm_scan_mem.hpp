@@ -468,48 +468,53 @@ PSM_DEV void sqrt_filter_push(const FView<R, NX>& e2, C (&m)[NX], C (&L)[NX][NX]
   }
 }
 
-// The same for the covariance form (std_combine_core with A1, eta1 and J1 zero).
+// The same for the covariance form: with N = I + J2 P, w = eta2 - J2 m and
+// [X1^T | y] = N^-1 [A2^T | w],  m' = A2 (m + P y) + b2 and P' = X1 (P A2^T) + C2.
 template <typename R, int NX>
 PSM_DEV void std_filter_push(const FView<R, NX>& e2, R (&m)[NX], R (&P)[NX][NX]) {
-  // X1 = A2 (I + C1 J2)^{-1} via (I + C1 J2)^T X1^T = A2^T
-  R M1[NX][NX], B1[NX][NX];
+  R N[NX][NX], B[NX][NX + 1];
 #pragma unroll
-  for (int i = 0; i < NX; ++i)
+  for (int i = 0; i < NX; ++i) {
+    R jm = e2.Z(i, 0) * m[0];
+#pragma unroll
+    for (int k = 1; k < NX; ++k) jm = fma(e2.Z(i, k), m[k], jm);
+    B[i][NX] = e2.eta(i) - jm;
 #pragma unroll
     for (int j = 0; j < NX; ++j) {
       R s1 = (i == j) ? R(1) : R(0);
 #pragma unroll
-      for (int k = 0; k < NX; ++k) s1 = fma(P[j][k], e2.Z(k, i), s1);
-      M1[i][j] = s1;
-      B1[i][j] = e2.A(j, i);
+      for (int k = 0; k < NX; ++k) s1 = fma(P[j][k], e2.Z(k, i), s1);   // (I + P J2)^T
+      N[i][j] = s1;
+      B[i][j] = e2.A(j, i);
     }
-  solve_general<R, NX, NX>(M1, B1);   // B1 = X1^T
-  R t[NX], CA[NX][NX];
+  }
+  solve_general<R, NX, NX + 1>(N, B);
+  R v[NX], CA[NX][NX];
 #pragma unroll
   for (int i = 0; i < NX; ++i) {
-    R a = P[i][0] * e2.eta(0);
+    R a = P[i][0] * B[0][NX];
 #pragma unroll
-    for (int k = 1; k < NX; ++k) a = fma(P[i][k], e2.eta(k), a);
-    t[i] = a + m[i];
+    for (int k = 1; k < NX; ++k) a = fma(P[i][k], B[k][NX], a);
+    v[i] = m[i] + a;
 #pragma unroll
     for (int j = 0; j < NX; ++j) {
       R c = P[i][0] * e2.A(j, 0);
 #pragma unroll
       for (int k = 1; k < NX; ++k) c = fma(P[i][k], e2.A(j, k), c);
-      CA[i][j] = c;                    // C1 A2^T
+      CA[i][j] = c;                    // P A2^T
     }
   }
 #pragma unroll
   for (int i = 0; i < NX; ++i) {
-    R b = B1[0][i] * t[0];
+    R b = e2.A(i, 0) * v[0];
 #pragma unroll
-    for (int k = 1; k < NX; ++k) b = fma(B1[k][i], t[k], b);
+    for (int k = 1; k < NX; ++k) b = fma(e2.A(i, k), v[k], b);
     m[i] = b + e2.b(i);
 #pragma unroll
     for (int j = 0; j < NX; ++j) {
-      R c = B1[0][i] * CA[0][j];
+      R c = B[0][i] * CA[0][j];
 #pragma unroll
-      for (int k = 1; k < NX; ++k) c = fma(B1[k][i], CA[k][j], c);
+      for (int k = 1; k < NX; ++k) c = fma(B[k][i], CA[k][j], c);
       P[i][j] = c + e2.U(i, j);
     }
   }
