@@ -126,7 +126,7 @@ typedef struct psm_problem {
   /* bits 0-7: scan items folded per lane (0: the PSM_SCAN_K environment
    * variable, else 2 with 16-lane upper levels and 4 without);
    * PSM_SCAN_TEAM: levels above the first run 16 lanes per combination
-   * (square-root form, float / double); with bits 0-7 clear they do so by
+   * (float / double); with bits 0-7 clear they do so by
    * default, unless the PSM_SCAN_TEAM environment variable is 0;
    * PSM_SCAN_HALF: level 0 of the scan runs 32-lane workgroups (square-root
    * form, float / double): twice the workgroups, half the LDS each, one
@@ -136,7 +136,7 @@ typedef struct psm_problem {
    * float / double): the level layout is the same, each combination's chain
    * of dependent operations about a third;
    * PSM_SCAN_ROW: level 0 of the scan runs 16 lanes per combination, 16
-   * combinations per workgroup (square-root form, float / double; it takes
+   * combinations per workgroup (float / double; it takes
    * precedence over PSM_SCAN_QUAD and PSM_SCAN_HALF): the shortest chain, for
    * the few items of a short sequence;
    * bits 16-23 (PSM_SCAN_TOP_MASK): a level whose items fit one workgroup
@@ -256,7 +256,7 @@ int psm_filter_smoother(const psm_problem_t* prob, const psm_model_t* trans,
                         size_t workspace_bytes, int32_t use_graph, void* stream);
 
 /* Size of the library-owned workspace of psm_filter_smoother_noalloc (per GPU). */
-#define PSM_STATIC_WORKSPACE_BYTES (64u << 20)
+#define PSM_STATIC_WORKSPACE_BYTES (72u << 20)
 
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under hipGraph capture, tight serving loops, harnesses that
@@ -265,8 +265,8 @@ int psm_filter_smoother(const psm_problem_t* prob, const psm_model_t* trans,
  * creation), eager on the caller's stream.  The scan workspace is a static
  * device buffer of PSM_STATIC_WORKSPACE_BYTES that each GPU holds until the
  * process ends; problems whose psm_workspace_bytes exceeds it are rejected
- * with PSM_E_WORKSPACE (64 MiB holds a single FP64 nx=5 sequence of about
- * 41,000 steps).  Every call on one GPU shares that buffer: calls that
+ * with PSM_E_WORKSPACE (72 MiB holds a single FP64 nx=5 sequence of about
+ * 51,000 steps).  Every call on one GPU shares that buffer: calls that
  * overlap on one GPU (concurrent streams or threads) race and must be
  * serialised by the caller.  Nothing in it needs to start at zero. */
 int psm_filter_smoother_noalloc(const psm_problem_t* prob, const psm_model_t* trans,
@@ -417,10 +417,10 @@ int psm_math_check(int64_t n, const double* x, double* out_rcp, double* out_sqrt
 /* Schedule autotuner (no reference counterpart: the reference's schedule is
  * XLA's).  Times psm_filter_smoother (eager, on `stream`) for candidate
  * schedules whose workspace fits workspace_bytes: first chunk in {2, 4, 8, 16,
- * 32} states per lane x scan fan-in scan_k in {2, 4, 8}, with and without
- * PSM_SCAN_TEAM and PSM_SCAN_HALF, and with PSM_SCAN_TEAM | PSM_SCAN_QUAD
- * with and without PSM_SCAN_HALF, and with PSM_SCAN_TEAM | PSM_SCAN_ROW at
- * fan-in 1 and 2 (square-root form in float / double); then
+ * 32}, and 1 up to 8192 states, per lane x scan fan-in scan_k in {2, 4, 8},
+ * with and without PSM_SCAN_TEAM and PSM_SCAN_HALF, and with PSM_SCAN_TEAM |
+ * PSM_SCAN_QUAD with and without PSM_SCAN_HALF (square-root form in float /
+ * double), and with PSM_SCAN_TEAM | PSM_SCAN_ROW at fan-in 1 and 2; then
  * the chunks at 5/8 .. 7/4 of the best chunk (those that are not powers of
  * two, at most 64) with the three best scan_k values.  Returns the fastest in
  * *best_chunk / *best_scan_k (and its time per pass in *best_ms, may be

@@ -938,18 +938,21 @@ int psm_autotune(const psm_problem_t* p, const psm_model_t* trans, const psm_mod
   };
   // stage 1: power-of-two chunks x scan modes (fan-in {2, 4, 8} x {per-lane,
   // 16-lane upper levels, half-wave level 0, both, quad level 0, quad + half-wave},
-  // 16-lane level 0 at fan-in 1 and 2); stage 2: chunks between the stage-1
+  // 16-lane level 0 at fan-in 1 and 2; the covariance form has the first and the
+  // last of these); stage 2: chunks between the stage-1
   // sizes (5/8 .. 7/4 of the best one) with the three best scan modes.  Chunk
   // sizes that are not powers of two avoid a nearly empty last workgroup when
   // the state count is just above a power of two (T + 1 states).
-  static const int32_t chunks[] = {2, 4, 8, 16, 32};
-  const bool team_ok = p->form == PSM_FORM_SQRT && (p->dtype == PSM_F32 || p->dtype == PSM_F64);
+  std::vector<int32_t> chunks = {2, 4, 8, 16, 32};
+  if (p->n_states <= 8192) chunks.insert(chunks.begin(), 1);
+  const bool row_ok = p->dtype == PSM_F32 || p->dtype == PSM_F64;
+  const bool team_ok = p->form == PSM_FORM_SQRT && row_ok;
   std::vector<int32_t> scan_modes;
   for (int32_t mode : {0, PSM_SCAN_TEAM, PSM_SCAN_HALF, PSM_SCAN_TEAM | PSM_SCAN_HALF,
                        PSM_SCAN_TEAM | PSM_SCAN_QUAD, PSM_SCAN_TEAM | PSM_SCAN_QUAD | PSM_SCAN_HALF})
     if (mode == 0 || team_ok)
       for (int32_t k : {2, 4, 8}) scan_modes.push_back(k | mode);
-  if (team_ok)
+  if (row_ok)
     for (int32_t k : {1, 2}) scan_modes.push_back(k | PSM_SCAN_TEAM | PSM_SCAN_ROW);
   std::vector<TuneResult> res;
   for (int32_t c : chunks) {

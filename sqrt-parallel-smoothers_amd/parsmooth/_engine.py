@@ -111,7 +111,7 @@ class Problem:
     # with or without the 16-lane upper scan levels (N.SCAN_TEAM), the half-wave
     # level 0 (N.SCAN_HALF) and the four-lane level 0 (N.SCAN_QUAD), and the
     # 16-lane level 0 (N.SCAN_ROW), both with 16-lane upper levels
-    TUNE_CHUNKS = (2, 4, 8, 16, 32)
+    TUNE_CHUNKS = (2, 4, 8, 16, 32)   # and 1 up to 8192 states
     TUNE_SCAN_K = tuple(k | f for f in (0, N.SCAN_TEAM, N.SCAN_HALF, N.SCAN_TEAM | N.SCAN_HALF,
                                         N.SCAN_TEAM | N.SCAN_QUAD,
                                         N.SCAN_TEAM | N.SCAN_QUAD | N.SCAN_HALF)
@@ -133,7 +133,7 @@ class Problem:
         nominal and keep the fastest; returns (chunk, scan_k, ms per pass)."""
         saved = (self.struct.chunk, self.struct.scan_k)
         need = 0
-        for c in range(2, 65):  # the refinement stage may pick any chunk up to 64
+        for c in range(1, 65):  # the refinement stage may pick any chunk up to 64
             for k in self.TUNE_SCAN_K:
                 self.struct.chunk, self.struct.scan_k = c, k
                 need = max(need, int(N.lib().psm_workspace_bytes(ctypes.byref(self.struct))))
