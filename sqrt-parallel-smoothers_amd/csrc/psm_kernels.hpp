@@ -242,11 +242,11 @@ PSM_DEV void linearize_point_wide(const ModelView<R>& md, const SigmaView<R>& sp
   widen(bW, b);
 }
 
-template <typename R, int NIN, int NOUT, bool SQRT, typename FB>
+template <typename R, int NIN, int NOUT, bool SQRT, typename FB, typename PC = NoPoints>
 PSM_DEV void linearize_point_w(const ModelView<R>& md, const SigmaView<R>& sp, int use_sigma,
                                const R (&m)[NIN], const R (&Lx)[NIN][NIN], R (&F)[NOUT][NIN],
                                R (&C)[NOUT][NOUT], R (&b)[NOUT], const FB& fb,
-                               const PointCache<R>& pc = PointCache<R>{nullptr, 0, 0}) {
+                               const PC& pc = PC{}) {
   if constexpr (kFallback<R, SQRT> && !FB::kRedo) {
     // FP32 square-root pass without FP64 code: a point the centred regression
     // cannot take (conditional moments, a negative weight) or whose factor is
@@ -337,6 +337,20 @@ __global__ __launch_bounds__(kLaneWG) void k_linearize_states(
     int use_sigma, const R* __restrict__ nom_m, const R* __restrict__ nom_L, int nom_inter,
     R* __restrict__ lin, R* __restrict__ ref, FB fb) {
   if (fb.skip()) return;
+  // FP32: the rule is converted once per workgroup, and the regressions' increments
+  // wait in LDS for their residual passes
+  constexpr bool kSingle = std::is_same<R, float>::value;
+  constexpr int kPts = kSingle ? 2 * NX + 1 : 1, kOut = kSingle ? (NX > NY ? NX : NY) : 1;
+  __shared__ R increments[kPts * kOut * (kSingle ? kLaneWG : 1)], rule[kPts * (NX + 2)];
+  const bool staged = kSingle && use_sigma && sp.npts <= kPts;
+  if (staged) {
+    for (int q = threadIdx.x; q < sp.npts * NX; q += kLaneWG) rule[q] = sp.pxi(q);
+    for (int p = threadIdx.x; p < sp.npts; p += kLaneWG) {
+      rule[kPts * NX + p] = sp.pwm(p);
+      rule[kPts * (NX + 1) + p] = sp.pwc(p);
+    }
+    __syncthreads();
+  }
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= Mp) return;
   const int64_t g = (int64_t)C << 6;
@@ -349,51 +363,54 @@ __global__ __launch_bounds__(kLaneWG) void k_linearize_states(
   R m[NX], L[NX][NX];
   traj_load<!SQRT, R, NX>(nom_m, nom_L, nom_inter, i, t, m, L);
   R* lp = blk<Step<R, NX, NY>::NQ>(lin, t);
-  // FP32: the regression's increments wait in LDS for its residual pass
-  PointCache<R> pc{nullptr, 0, 0};
-  if constexpr (std::is_same<R, float>::value) {
-    __shared__ float fcache[(2 * NX + 1) * NX * kLaneWG];
-    pc = PointCache<R>{fcache + threadIdx.x, kLaneWG, 2 * NX + 1};
-  }
-  {
-    R F[NX][NX], Cq[NX][NX], b[NX];
-    linearize_point_w<R, NX, NX, SQRT>(tr, sp, use_sigma, m, L, F, Cq, b, fb, pc);
-    if constexpr (kCentred<R, SQRT>) {
-      R next[NX];
-      copy(m, next);
-      if (i + 1 < M) {
-        if (nom_inter) {
-          // the next slot of this chunk, or the first of the next
-          const int64_t pos = (r >> 6) + 1 < C ? t + 64 : StateMap{C}(i + 1);
-          int q = 0;
-          ld(blk<kTrajWords<!SQRT, NX>>(nom_m, pos), kBlk, 0, q, next);
-        } else {
-          ld_aos(nom_m, i + 1, next);
+  auto run = [&](const auto& pc) {
+    {
+      R F[NX][NX], Cq[NX][NX], b[NX];
+      linearize_point_w<R, NX, NX, SQRT>(tr, sp, use_sigma, m, L, F, Cq, b, fb, pc);
+      if constexpr (kCentred<R, SQRT>) {
+        R next[NX];
+        copy(m, next);
+        if (i + 1 < M) {
+          if (nom_inter) {
+            // the next slot of this chunk, or the first of the next
+            const int64_t pos = (r >> 6) + 1 < C ? t + 64 : StateMap{C}(i + 1);
+            int q = 0;
+            ld(blk<kTrajWords<!SQRT, NX>>(nom_m, pos), kBlk, 0, q, next);
+          } else {
+            ld_aos(nom_m, i + 1, next);
+          }
         }
+        int q = 0;
+        st(blk<NX>(ref, t), kBlk, 0, q, m);
+        centre(F, m, next, b);
       }
       int q = 0;
-      st(blk<NX>(ref, t), kBlk, 0, q, m);
-      centre(F, m, next, b);
+      st(lp, kBlk, 0, q, F);
+      if constexpr (SQRT) lower_factor(Cq);
+      st_tri(lp, kBlk, 0, q, Cq);
+      st(lp, kBlk, 0, q, b);
     }
-    int q = 0;
-    st(lp, kBlk, 0, q, F);
-    if constexpr (SQRT) lower_factor(Cq);
-    st_tri(lp, kBlk, 0, q, Cq);
-    st(lp, kBlk, 0, q, b);
-  }
-  if (do_obs) {
-    R H[NY][NX], Cr[NY][NY], c[NY];
-    linearize_point_w<R, NX, NY, SQRT>(ob, sp, use_sigma, m, L, H, Cr, c, fb);
-    if constexpr (kCentred<R, SQRT>) {
-      const R zero[NY] = {};
-      centre(H, m, zero, c);
+    if (do_obs) {
+      R H[NY][NX], Cr[NY][NY], c[NY];
+      linearize_point_w<R, NX, NY, SQRT>(ob, sp, use_sigma, m, L, H, Cr, c, fb, pc);
+      if constexpr (kCentred<R, SQRT>) {
+        const R zero[NY] = {};
+        centre(H, m, zero, c);
+      }
+      int q = Step<R, NX, NY>::NTRANS;
+      st(lp, kBlk, 0, q, H);
+      if constexpr (SQRT) lower_factor(Cr);
+      st_tri(lp, kBlk, 0, q, Cr);
+      st(lp, kBlk, 0, q, c);
     }
-    int q = Step<R, NX, NY>::NTRANS;
-    st(lp, kBlk, 0, q, H);
-    if constexpr (SQRT) lower_factor(Cr);
-    st_tri(lp, kBlk, 0, q, Cr);
-    st(lp, kBlk, 0, q, c);
+  };
+  if constexpr (kSingle) {
+    if (staged) {
+      run(PointCache<R>{increments + threadIdx.x, kLaneWG, rule, rule + kPts * NX, rule + kPts * (NX + 1)});
+      return;
+    }
   }
+  run(NoPoints{});
 }
 
 // ============================================================================

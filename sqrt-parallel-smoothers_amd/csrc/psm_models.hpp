@@ -540,9 +540,24 @@ PSM_DEV void model_at_mean(const ModelView<R, S>& md, const R (&m)[NIN], R (&f0)
   model_value<R, NIN, NOUT>(m0, m, f0);
 }
 
+// Terms of an increment that are the same for every point: the coordinated turn's at
+// the mean's turn rate.
+template <typename R> struct MeanTerms {
+  R a, b, c, s;
+};
 template <typename R, int NIN, int NOUT, typename S>
-PSM_DEV void model_increment(const ModelView<R, S>& md, const R (&m)[NIN], const R (&d)[NIN],
-                             const R (&f0)[NOUT], R (&df)[NOUT]) {
+PSM_DEV MeanTerms<R> mean_terms(const ModelView<R, S>& md, const R (&m)[NIN]) {
+  MeanTerms<R> t{R(0), R(0), R(0), R(0)};
+  if constexpr (NIN == 5 && NOUT == 5) {
+    R u, v;
+    if (md.kind == PSM_MODEL_COORDINATED_TURN) ct_terms_single(m[4], md.par(0), t.a, t.b, u, v, t.c, t.s);
+  }
+  return t;
+}
+
+template <typename R, int NIN, int NOUT, typename S>
+PSM_DEV void model_increment(const ModelView<R, S>& md, const MeanTerms<R>& t0, const R (&m)[NIN],
+                             const R (&d)[NIN], const R (&f0)[NOUT], R (&df)[NOUT]) {
   if (md.kind == PSM_MODEL_LINEAR) {
 #pragma unroll
     for (int i = 0; i < NOUT; ++i) {
@@ -556,10 +571,9 @@ PSM_DEV void model_increment(const ModelView<R, S>& md, const R (&m)[NIN], const
   if constexpr (NIN == 5 && NOUT == 5) {
     if (md.kind == PSM_MODEL_COORDINATED_TURN) {
       const R dt = md.par(0);
-      R a0, b0, c0, s0, a1, b1, c1, s1, u, v;
-      ct_terms_single(m[4], dt, a0, b0, u, v, c0, s0);
+      R a1, b1, c1, s1, u, v;
       ct_terms_single(m[4] + d[4], dt, a1, b1, u, v, c1, s1);
-      const R da = a1 - a0, db = b1 - b0, dc = c1 - c0, ds = s1 - s0;
+      const R da = a1 - t0.a, db = b1 - t0.b, dc = c1 - t0.c, ds = s1 - t0.s;
       df[0] = d[0] + a1 * d[2] - b1 * d[3] + (da * m[2] - db * m[3]);
       df[1] = d[1] + b1 * d[2] + a1 * d[3] + (db * m[2] + da * m[3]);
       df[2] = c1 * d[2] + s1 * d[3] + (dc * m[2] + ds * m[3]);
@@ -593,37 +607,57 @@ PSM_DEV void model_increment(const ModelView<R, S>& md, const R (&m)[NIN], const
 // Phi - F P F^T nor the rounding of a large mean reaches the noise factor.
 // Two passes over the points: the mean and the cross-covariance, then the
 // residual columns, which read the increments back from the caller's per-lane
-// scratch (pc) when it holds them, else evaluate them again.
+// scratch (PointCache), or without one (NoPoints) evaluate them again.
 // Returns false, with nothing written, when some wc is negative.
 // ----------------------------------------------------------------------------
-// Per-lane scratch for the increments of one regression (value i of point p
-// at base[(p * NOUT + i) * stride]), used when there are at most cap points.
+// Scratch of one regression: the increments per lane (value i of point p at
+// base[(p * NOUT + i) * stride]), and the rule, which every lane reads, converted to
+// the compute type once.
 template <typename R> struct PointCache {
+  static constexpr bool kOn = true;
   R* base;
   int stride;
-  int cap;
+  const R* xi;
+  const R* wm;
+  const R* wc;
+};
+struct NoPoints {
+  static constexpr bool kOn = false;
 };
 
-template <typename R, int NIN, int NOUT, bool SQRT, typename S>
+template <typename R, int NIN, int NOUT, bool SQRT, typename S, typename PC = NoPoints>
 PSM_DEV bool linearize_sigma_centred(const ModelView<R, S>& md, const SigmaView<R>& sp, const R (&m)[NIN],
                                      const R (&L)[NIN][NIN], R (&F)[NOUT][NIN], R (&C)[NOUT][NOUT],
-                                     R (&b)[NOUT], const PointCache<R>& pc = PointCache<R>{nullptr, 0, 0}) {
+                                     R (&b)[NOUT], const PC& pc = PC{}) {
   for (int p = 0; p < sp.npts; ++p)
     if (sp.wc[p] < 0.0) return false;
   R f0[NOUT];
   model_at_mean<R, NIN, NOUT>(md, m, f0);
+  const MeanTerms<R> t0 = mean_terms<R, NIN, NOUT>(md, m);
+  auto xi = [&](int q) {
+    if constexpr (PC::kOn) return pc.xi[q];
+    else return sp.pxi(q);
+  };
+  auto wmean = [&](int p) {
+    if constexpr (PC::kOn) return pc.wm[p];
+    else return sp.pwm(p);
+  };
+  auto wcov = [&](int p) {
+    if constexpr (PC::kOn) return pc.wc[p];
+    else return sp.pwc(p);
+  };
   // point p: displacement d = L xi_p and increment f = f(m + d) - f(m)
   auto point = [&](int p, R (&d)[NIN], R (&f)[NOUT]) {
 #pragma unroll
     for (int i = 0; i < NIN; ++i) {
       R s = R(0);
 #pragma unroll
-      for (int j = 0; j < NIN; ++j) s = fma(L[i][j], sp.pxi(p * NIN + j), s);
+      for (int j = 0; j < NIN; ++j) s = fma(L[i][j], xi(p * NIN + j), s);
       d[i] = s;
     }
     ModelView<R, S> mp = md;
     mp.pt = p;
-    model_increment<R, NIN, NOUT>(mp, m, d, f0, f);
+    model_increment<R, NIN, NOUT>(mp, t0, m, d, f0, f);
   };
   // one pass for the weighted mean of the increments and their
   // cross-covariance with the displacements:
@@ -633,15 +667,14 @@ PSM_DEV bool linearize_sigma_centred(const ModelView<R, S>& md, const SigmaView<
   set_zero(mf);
   set_zero(Psi);
   set_zero(sd);
-  const bool keep = pc.base != nullptr && sp.npts <= pc.cap;
   for (int p = 0; p < sp.npts; ++p) {
     R d[NIN], f[NOUT];
     point(p, d, f);
-    if (keep) {
+    if constexpr (PC::kOn) {
 #pragma unroll
       for (int i = 0; i < NOUT; ++i) pc.base[(p * NOUT + i) * pc.stride] = f[i];
     }
-    const R wm = sp.pwm(p), wc = sp.pwc(p);
+    const R wm = wmean(p), wc = wcov(p);
 #pragma unroll
     for (int i = 0; i < NOUT; ++i) mf[i] = fma(wm, f[i], mf[i]);
 #pragma unroll
@@ -676,12 +709,12 @@ PSM_DEV bool linearize_sigma_centred(const ModelView<R, S>& md, const SigmaView<
   // residual of point p
   auto residual = [&](int p, R (&r)[NOUT]) {
     R d[NIN], f[NOUT];
-    if (keep) {
+    if constexpr (PC::kOn) {
 #pragma unroll
       for (int i = 0; i < NIN; ++i) {
         R s = R(0);
 #pragma unroll
-        for (int j = 0; j < NIN; ++j) s = fma(L[i][j], sp.pxi(p * NIN + j), s);
+        for (int j = 0; j < NIN; ++j) s = fma(L[i][j], xi(p * NIN + j), s);
         d[i] = s;
       }
 #pragma unroll
@@ -716,7 +749,7 @@ PSM_DEV bool linearize_sigma_centred(const ModelView<R, S>& md, const SigmaView<
         set_zero(r);
         const bool live = p0 + k < sp.npts;
         if (live) residual(p0 + k, r);
-        const R sw = live ? sqrt_(sp.pwc(p0 + k)) : R(0);
+        const R sw = live ? sqrt_(wcov(p0 + k)) : R(0);
 #pragma unroll
         for (int i = 0; i < NOUT; ++i) Ab[i][NOUT + k] = sw * r[i];
       }
@@ -738,7 +771,7 @@ PSM_DEV bool linearize_sigma_centred(const ModelView<R, S>& md, const SigmaView<
     for (int p = 0; p < sp.npts; ++p) {
       R r[NOUT];
       residual(p, r);
-      const R w = sp.pwc(p);
+      const R w = wcov(p);
 #pragma unroll
       for (int i = 0; i < NOUT; ++i)
 #pragma unroll
