@@ -96,8 +96,11 @@ class Problem:
         # FP64 re-triangularisation fallback of the FP32 square-root path
         self.fallback_counter = torch.zeros(1, dtype=torch.int64, device=dev)
         ratio = FP32_FALLBACK_RATIO if (code in (N.PSM_F32, N.PSM_F32_TANGENT) and sqrt) else 0.0
-        if tangent_code is None and not chunk and "PSM_CHUNK" not in os.environ:
-            chunk = states_per_chunk(self.n_states)
+        if not chunk and "PSM_CHUNK" not in os.environ:
+            # tangent types scan with one lane per combination: the library's choice,
+            # longer where the chip is full (FP64, a million states: 349 ms at 40, 392)
+            chunk = states_per_chunk(self.n_states) if tangent_code is None else \
+                40 if self.n_states >= 1 << 20 else 0
         self.struct = N.PsmProblem(code, N.FORM_SQRT if sqrt else N.FORM_STD,
                                    self.nx, self.ny, self.n_seq, int(chunk), self.n_states,
                                    self.state_offsets.data_ptr(), float(ratio), 0,
