@@ -1,0 +1,75 @@
+"""Errors that single precision must not have: shifts that grow with the length of a
+sequence or with the size of the coordinates.  The references are the FP64 passes
+(compared with the oracle elsewhere) or the FP64 oracle, on the same FP32-rounded
+inputs.
+"""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if not torch.cuda.is_available():  # pragma: no cover
+    pytest.skip("needs a HIP device", allow_module_level=True)
+
+from parsmooth import FunctionalModel, MVNSqrt  # noqa: E402
+from parsmooth import models as M  # noqa: E402
+from parsmooth.batch import IteratedSmoother  # noqa: E402
+from parsmooth.data import bearings_data_batch  # noqa: E402
+from parsmooth.linearization import cubature, unscented  # noqa: E402
+
+DEV = torch.device("cuda", 0)
+DT = float(np.float32(0.01))
+S1, S2 = (-1.5, 0.5), (1.0, 1.0)
+npy = lambda x: x.detach().double().cpu().numpy()
+r32 = lambda a: np.asarray(a, np.float32).astype(np.float64)
+
+
+def turn_models(dtype, s1=S1, s2=S2):
+    Q, R, obs_f, trans_f = M.make_parameters(0.01, 0.1, 0.5, DT, s1, s2)
+    t = lambda a: torch.as_tensor(r32(a), device=DEV).to(dtype)
+    return (FunctionalModel(trans_f, MVNSqrt(t(np.zeros(5)), t(np.linalg.cholesky(Q)))),
+            FunctionalModel(obs_f, MVNSqrt(t(np.zeros(2)), t(np.linalg.cholesky(R)))))
+
+
+@pytest.mark.parametrize("method", [cubature, unscented], ids=["cubature", "unscented"])
+def test_loglikelihood_of_long_sequences(method):
+    """The log-likelihood's error per step, one way for every sequence, is at most one
+    FP32 rounding (2^-24): a step's term is a sum of values of about 1 whose roundings
+    go both ways, and what does not average out is a factor of the model that is off
+    the same way at every step."""
+    T, B = 1000, 200
+    rng = np.random.RandomState(0)
+    x0 = np.array([3.0, 2.0, 1.0, 0.0]) + 0.3 * rng.randn(B, 4)
+    states, obs = bearings_data_batch([T] * B, x0, DT, 0.5, S1, S2, q=3.16, seed=1)
+    ys, m0 = np.concatenate(obs), np.stack([s[0] for s in states]) + 0.1 * rng.randn(B, 5)
+    L0 = np.repeat(0.3 * np.eye(5)[None], B, 0)
+    nom, ell = None, {}
+    for dtype in (torch.float64, torch.float32):
+        t = lambda a: torch.as_tensor(r32(a), device=DEV).to(dtype)
+        run = IteratedSmoother([T] * B, *turn_models(dtype), method, dtype=dtype)
+        run.set_data(t(ys), t(m0), t(L0))
+        if nom is None:   # a nominal near the posterior, the same for both types
+            mean, fac = run.run(2, (t(np.concatenate(states)), t(np.repeat(0.1 * np.eye(5)[None], B * (T + 1), 0))))
+            nom = r32(npy(mean)), r32(npy(fac))
+        ell[dtype] = npy(run.run(1, tuple(map(t, nom)), return_loglikelihood=True)[2])
+    shift = np.median(ell[torch.float32] - ell[torch.float64]) / T
+    assert abs(shift) <= 2.0 ** -24, shift
+
+
+# the points' bearings on both sides of the negative x axis, where a bearing jumps by
+# 2 pi, and far from the sensors
+@pytest.mark.parametrize("mean", [(-6.0, 0.55), (-6.0, 0.4), (-6.0, 0.5), (-40.0, 1.02), (3.0, 2.0), (150.0, 90.0)])
+def test_bearing_regression(mean):
+    """F, the noise factor and b of one cubature regression.  F is the points' increments
+    over their distances: FP32 leaves it 1e-5 of its size (the increments are sums of ten
+    terms with errors of a few 2^-24 each, over factors whose condition is below 10)."""
+    m = r32(np.array([*mean, 1.0, -0.5, 0.3]))
+    L = r32(np.tril(0.1 + 0.05 * np.arange(25).reshape(5, 5) / 25) + 0.4 * np.eye(5))
+    out = {}
+    for dtype in (torch.float64, torch.float32):
+        t = lambda a: torch.as_tensor(a, device=DEV).to(dtype)
+        out[dtype] = [npy(a) for a in cubature(turn_models(dtype)[1], MVNSqrt(t(m), t(L)))]
+    F = out[torch.float64][0]
+    for a, b, size in zip(out[torch.float32], out[torch.float64], (0.0, 0.0, np.abs(F).max() * np.abs(m).max())):
+        assert np.abs(a - b).max() <= 1e-5 * max(np.abs(b).max(), size), (a, b)
