@@ -226,10 +226,22 @@ PSM_DEV void widen(const B (&a)[M][N], A (&b)[M][N]) {
   for (int i = 0; i < M; ++i) widen(a[i], b[i]);
 }
 
-template <typename R, int NIN, int NOUT, bool SQRT>
+// b <- b + F m - next, formed in FP64
+template <typename R, int NO, int NI, typename N>
+PSM_DEV void centre(const R (&F)[NO][NI], const R (&m)[NI], const N (&next)[NO], R (&b)[NO]) {
+#pragma unroll
+  for (int a = 0; a < NO; ++a) {
+    double s = (double)b[a] - (double)next[a];
+#pragma unroll
+    for (int k = 0; k < NI; ++k) s = fma((double)F[a][k], (double)m[k], s);
+    b[a] = (R)s;
+  }
+}
+
+template <typename R, int NIN, int NOUT, bool SQRT, typename From>
 PSM_DEV void linearize_point_wide(const ModelView<R>& md, const SigmaView<R>& sp, int use_sigma,
                                   const R (&m)[NIN], const R (&Lx)[NIN][NIN], R (&F)[NOUT][NIN],
-                                  R (&C)[NOUT][NOUT], R (&b)[NOUT]) {
+                                  R (&C)[NOUT][NOUT], R (&b)[NOUT], const From& from) {
   using W = typename WiderOf<R>::type;
   const ModelView<W, R> mw{md.kind, md.params, md.q_mean, md.q_chol, md.row, md.pt, md.npts};
   const SigmaView<W> sw{sp.npts, sp.xi, sp.wm, sp.wc};
@@ -237,16 +249,17 @@ PSM_DEV void linearize_point_wide(const ModelView<R>& md, const SigmaView<R>& sp
   widen(m, mW);
   widen(Lx, LW);
   linearize_point<W, NIN, NOUT, SQRT>(mw, sw, use_sigma, mW, LW, FW, CW, bW);
+  if constexpr (From::kNominal) centre(FW, mW, from.next, bW);
   widen(FW, F);
   widen(CW, C);
   widen(bW, b);
 }
 
-template <typename R, int NIN, int NOUT, bool SQRT, typename FB, typename PC = NoPoints>
+template <typename R, int NIN, int NOUT, bool SQRT, typename FB, typename PC = NoPoints, typename From = FromZero>
 PSM_DEV void linearize_point_w(const ModelView<R>& md, const SigmaView<R>& sp, int use_sigma,
                                const R (&m)[NIN], const R (&Lx)[NIN][NIN], R (&F)[NOUT][NIN],
                                R (&C)[NOUT][NOUT], R (&b)[NOUT], const FB& fb,
-                               const PC& pc = PC{}) {
+                               const PC& pc = PC{}, const From& from = From{}) {
   if constexpr (kFallback<R, SQRT> && !FB::kRedo) {
     // FP32 square-root pass without FP64 code: a point the centred regression
     // cannot take (conditional moments, a negative weight) or whose factor is
@@ -254,20 +267,22 @@ PSM_DEV void linearize_point_w(const ModelView<R>& md, const SigmaView<R>& sp, i
     // linearizes every point again with the FP64 path below
     if (!use_sigma) {
       linearize_extended<R, NIN, NOUT>(md, m, F, C, b);
+      if constexpr (From::kNominal) centre(F, m, from.next, b);
       return;
     }
     const bool done = md.kind != PSM_MODEL_CONDITIONAL &&
-                      linearize_sigma_centred<R, NIN, NOUT, true>(md, sp, m, Lx, F, C, b, pc);
+                      linearize_sigma_centred<R, NIN, NOUT, true>(md, sp, m, Lx, F, C, b, pc, from);
     if (!done || (fb.thr > 0.0f && ill_conditioned(C, fb.thr))) fb.raise();
   } else if constexpr (IsSingle<R>::value) {
     if (!use_sigma) {
       linearize_extended<R, NIN, NOUT>(md, m, F, C, b);
+      if constexpr (From::kNominal) centre(F, m, from.next, b);
       return;
     }
     bool done = false;
     if (md.kind != PSM_MODEL_CONDITIONAL) {
       if constexpr (SQRT) {
-        done = linearize_sigma_centred<R, NIN, NOUT, true>(md, sp, m, Lx, F, C, b, pc);
+        done = linearize_sigma_centred<R, NIN, NOUT, true>(md, sp, m, Lx, F, C, b, pc, from);
         if constexpr (kFallback<R, SQRT>) {
           if (done && fb.thr > 0.0f && ill_conditioned(C, fb.thr)) {
             count_fallback(fb);
@@ -277,10 +292,10 @@ PSM_DEV void linearize_point_w(const ModelView<R>& md, const SigmaView<R>& sp, i
       } else {
         R Lc[NIN][NIN];
         cholesky(Lx, Lc);   // get_mvnsqrt (parsmooth/linearization/_common.py:9-14)
-        done = linearize_sigma_centred<R, NIN, NOUT, false>(md, sp, m, Lc, F, C, b, pc);
+        done = linearize_sigma_centred<R, NIN, NOUT, false>(md, sp, m, Lc, F, C, b, pc, from);
       }
     }
-    if (!done) linearize_point_wide<R, NIN, NOUT, SQRT>(md, sp, use_sigma, m, Lx, F, C, b);
+    if (!done) linearize_point_wide<R, NIN, NOUT, SQRT>(md, sp, use_sigma, m, Lx, F, C, b, from);
   } else {
     linearize_point<R, NIN, NOUT, SQRT>(md, sp, use_sigma, m, Lx, F, C, b);
   }
@@ -289,8 +304,11 @@ PSM_DEV void linearize_point_w(const ModelView<R>& md, const SigmaView<R>& sp, i
 // Centred states of the FP32 square-root passes.  Between the linearization and
 // the output every mean is a difference from the nominal mean of its state:
 // x_k = n_k + d_k turns x_{k+1} = F x_k + b into d_{k+1} = F d_k + b', b' = b + F n_k
-// - n_{k+1}, and y = H x + c into y = H d + c', c' = c + H n_k (formed in FP64, where
-// n_k, n_{k+1} and F are exact).  The rounding of an aggregate's A (about 1 on
+// - n_{k+1}, and y = H x + c into y = H d + c', c' = c + H n_k.  Under the extended rule
+// these sums are formed in FP64, where n_k, n_{k+1} and F are exact; a regression's
+// b' is E f - n_{k+1} (model_minus and the mean increment): by way of b, which FP32
+// rounds at the size of x, every step had that rounding for an offset (8.6e-6 at a
+// position of 300, against a process noise of 5.8e-5).  The rounding of an aggregate's A (about 1 on
 // its diagonal, so 6e-8 a step, adding up along a sequence) multiplies d, of the
 // size of the posterior's spread, and not x, a position of 10 to 1000: the
 // smoothed means of a T = 16,385 pass were 1.5e-5 of their norm off a 64-bit
@@ -300,17 +318,6 @@ PSM_DEV void linearize_point_w(const ModelView<R>& md, const SigmaView<R>& sp, i
 template <typename R, bool SQRT>
 constexpr bool kCentred = SQRT && std::is_same<R, float>::value;
 
-// b <- b + F m - next
-template <typename R, int NO, int NI>
-PSM_DEV void centre(const R (&F)[NO][NI], const R (&m)[NI], const R (&next)[NO], R (&b)[NO]) {
-#pragma unroll
-  for (int a = 0; a < NO; ++a) {
-    double s = (double)b[a] - (double)next[a];
-#pragma unroll
-    for (int k = 0; k < NI; ++k) s = fma((double)F[a][k], (double)m[k], s);
-    b[a] = (R)s;
-  }
-}
 // m -/+ the nominal mean at interleaved position pos
 template <typename R, int NX>
 PSM_DEV void to_centred(const R* __restrict__ ref, int64_t pos, R (&m)[NX]) {
@@ -366,7 +373,6 @@ __global__ __launch_bounds__(kLaneWG) void k_linearize_states(
   auto run = [&](const auto& pc) {
     {
       R F[NX][NX], Cq[NX][NX], b[NX];
-      linearize_point_w<R, NX, NX, SQRT>(tr, sp, use_sigma, m, L, F, Cq, b, fb, pc);
       if constexpr (kCentred<R, SQRT>) {
         R next[NX];
         copy(m, next);
@@ -382,7 +388,9 @@ __global__ __launch_bounds__(kLaneWG) void k_linearize_states(
         }
         int q = 0;
         st(blk<NX>(ref, t), kBlk, 0, q, m);
-        centre(F, m, next, b);
+        linearize_point_w<R, NX, NX, SQRT>(tr, sp, use_sigma, m, L, F, Cq, b, fb, pc, FromNominal<R, NX>{next});
+      } else {
+        linearize_point_w<R, NX, NX, SQRT>(tr, sp, use_sigma, m, L, F, Cq, b, fb, pc);
       }
       int q = 0;
       st(lp, kBlk, 0, q, F);
@@ -392,10 +400,11 @@ __global__ __launch_bounds__(kLaneWG) void k_linearize_states(
     }
     if (do_obs) {
       R H[NY][NX], Cr[NY][NY], c[NY];
-      linearize_point_w<R, NX, NY, SQRT>(ob, sp, use_sigma, m, L, H, Cr, c, fb, pc);
       if constexpr (kCentred<R, SQRT>) {
         const R zero[NY] = {};
-        centre(H, m, zero, c);
+        linearize_point_w<R, NX, NY, SQRT>(ob, sp, use_sigma, m, L, H, Cr, c, fb, pc, FromNominal<R, NY>{zero});
+      } else {
+        linearize_point_w<R, NX, NY, SQRT>(ob, sp, use_sigma, m, L, H, Cr, c, fb, pc);
       }
       int q = Step<R, NX, NY>::NTRANS;
       st(lp, kBlk, 0, q, H);

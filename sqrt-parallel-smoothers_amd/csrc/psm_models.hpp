@@ -583,6 +583,35 @@ PSM_DEV MeanTerms<R> mean_terms(const ModelView<R, S>& md, const R (&m)[NIN]) {
   return t;
 }
 
+// f(m) - next, of which f(m) is f0 in R, formed in FP64 from the terms of the models
+// that are linear in what may be large: next is usually near f(m), and both may be large.
+template <typename R, int NIN, int NOUT, typename S>
+PSM_DEV void model_minus(const ModelView<R, S>& md, const MeanTerms<R>& t0, const R (&m)[NIN],
+                         const R (&f0)[NOUT], const R (&next)[NOUT], double (&r)[NOUT]) {
+#pragma unroll
+  for (int i = 0; i < NOUT; ++i) r[i] = (double)f0[i] - (double)next[i];
+  if (md.kind == PSM_MODEL_LINEAR) {
+#pragma unroll
+    for (int i = 0; i < NOUT; ++i) {
+      double s = -(double)next[i];
+#pragma unroll
+      for (int j = 0; j < NIN; ++j) s = fma((double)md.par(i * NIN + j), (double)m[j], s);
+      r[i] = s;
+    }
+    return;
+  }
+  if constexpr (NIN == 5 && NOUT == 5) {
+    if (md.kind == PSM_MODEL_COORDINATED_TURN) {
+      const double a = t0.a, b = t0.b, c = t0.c, s = t0.s, vx = m[2], vy = m[3];
+      r[0] = fma(a, vx, fma(-b, vy, (double)m[0] - (double)next[0]));
+      r[1] = fma(b, vx, fma(a, vy, (double)m[1] - (double)next[1]));
+      r[2] = fma(c, vx, fma(s, vy, -(double)next[2]));
+      r[3] = fma(-s, vx, fma(c, vy, -(double)next[3]));
+      r[4] = (double)m[4] - (double)next[4];
+    }
+  }
+}
+
 template <typename R, int NIN, int NOUT, typename S>
 PSM_DEV void model_increment(const ModelView<R, S>& md, const MeanTerms<R>& t0, const R (&m)[NIN],
                              const R (&d)[NIN], const R (&f0)[NOUT], R (&df)[NOUT]) {
@@ -675,11 +704,22 @@ template <typename R> struct PointCache {
 struct NoPoints {
   static constexpr bool kOn = false;
 };
+// Where the offset of a linearization y = F x + b starts: at zero (b as it stands), or,
+// with x and y differences from a nominal, at the nominal value of y: b = E f - next,
+// for which F is not used.
+struct FromZero {
+  static constexpr bool kNominal = false;
+};
+template <typename R, int N>
+struct FromNominal {
+  static constexpr bool kNominal = true;
+  const R (&next)[N];
+};
 
-template <typename R, int NIN, int NOUT, bool SQRT, typename S, typename PC = NoPoints>
+template <typename R, int NIN, int NOUT, bool SQRT, typename S, typename PC, typename From>
 PSM_DEV bool linearize_sigma_centred(const ModelView<R, S>& md, const SigmaView<R>& sp, const R (&m)[NIN],
                                      const R (&L)[NIN][NIN], R (&F)[NOUT][NIN], R (&C)[NOUT][NOUT],
-                                     R (&b)[NOUT], const PC& pc = PC{}) {
+                                     R (&b)[NOUT], const PC& pc, const From& from) {
   for (int p = 0; p < sp.npts; ++p)
     if (sp.wc[p] < 0.0) return false;
   R f0[NOUT];
@@ -749,6 +789,12 @@ PSM_DEV bool linearize_sigma_centred(const ModelView<R, S>& md, const SigmaView<
     for (int i = 0; i < NOUT; ++i)
 #pragma unroll
       for (int j = 0; j < NIN; ++j) F[i][j] = Y[j][i];
+  }
+  if constexpr (From::kNominal) {
+    double at[NOUT];
+    model_minus<R, NIN, NOUT>(md, t0, m, f0, from.next, at);
+#pragma unroll
+    for (int i = 0; i < NOUT; ++i) b[i] = (R)(at[i] + ((double)mf[i] + (double)md.qm(i)));
   }
   // residual of point p, of which G sums wc xi r^T
   R G[NIN][NOUT];
@@ -847,12 +893,14 @@ PSM_DEV bool linearize_sigma_centred(const ModelView<R, S>& md, const SigmaView<
 #pragma unroll
       for (int j = 0; j < NIN; ++j) F[i][j] += Y[j][i];
   }
+  if constexpr (!From::kNominal) {
 #pragma unroll
-  for (int i = 0; i < NOUT; ++i) {
-    R s = f0[i];
+    for (int i = 0; i < NOUT; ++i) {
+      R s = f0[i];
 #pragma unroll
-    for (int j = 0; j < NIN; ++j) s = fma(-F[i][j], m[j], s);
-    b[i] = (s + mf[i]) + md.qm(i);
+      for (int j = 0; j < NIN; ++j) s = fma(-F[i][j], m[j], s);
+      b[i] = (s + mf[i]) + md.qm(i);
+    }
   }
   return true;
 }

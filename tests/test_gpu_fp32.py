@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 if not torch.cuda.is_available():  # pragma: no cover
     pytest.skip("needs a HIP device", allow_module_level=True)
 
+import parsmooth  # noqa: E402
 from parsmooth import FunctionalModel, MVNSqrt  # noqa: E402
 from parsmooth import models as M  # noqa: E402
 from parsmooth.batch import IteratedSmoother  # noqa: E402
@@ -73,3 +74,32 @@ def test_bearing_regression(mean):
     F = out[torch.float64][0]
     for a, b, size in zip(out[torch.float32], out[torch.float64], (0.0, 0.0, np.abs(F).max() * np.abs(m).max())):
         assert np.abs(a - b).max() <= 1e-5 * max(np.abs(b).max(), size), (a, b)
+
+
+@pytest.mark.parametrize("method", [cubature, unscented], ids=["cubature", "unscented"])
+def test_regressions_far_from_the_origin(method):
+    """A filter pass on a track and its sensors moved by 4096 units: the coordinated
+    turn and the bearings see no difference, and the nominal is on the grid of FP32
+    numbers of that size, so that the move is exact.  The moved means have the rounding
+    to that grid (half a spacing of 2^-11) on top of the passes' own 2e-5, the
+    log-likelihood a few roundings of values of about 1 a step."""
+    T, move, grid = 400, 4096.0, 2.0 ** -11
+    states, obs = bearings_data_batch([T], [[3.0, 2.0, 1.0, 0.0]], DT, 0.5, S1, S2, q=3.16, seed=4)
+    rng = np.random.RandomState(2)
+    nm = states[0].astype(np.float64) + 0.03 * rng.randn(T + 1, 5)
+    nm[:, :2] = np.round(nm[:, :2] / grid) * grid
+    nL = np.repeat((0.3 * np.eye(5) + 0.02 * np.tril(np.ones((5, 5))))[None], T + 1, 0)
+    t = lambda a: torch.as_tensor(r32(a), device=DEV).to(torch.float32)
+    out = {}
+    for at in (0.0, move):
+        by = np.array([at, at, 0.0, 0.0, 0.0])
+        models = turn_models(torch.float32, *(tuple(at + v for v in s) for s in (S1, S2)))
+        nom = t(nm + by), t(nL)
+        assert np.array_equal(npy(nom[0]), r32(nm) + by)
+        filt, ell = parsmooth.filtering(t(obs[0]), MVNSqrt(t(nm[0] + by), t(0.3 * np.eye(5))), *models, method, MVNSqrt(*nom),
+                                        return_loglikelihood=True)
+        out[at] = npy(filt.mean) - by, npy(filt.chol), float(ell)
+    (m0, f0, e0), (m1, f1, e1) = out[0.0], out[move]
+    np.testing.assert_allclose(m1, m0, rtol=0, atol=0.5 * grid + 2e-5)
+    np.testing.assert_allclose(f1, f0, rtol=0, atol=1e-5)
+    assert abs(e1 - e0) <= T * 4 * 2.0 ** -24, (e1, e0)
