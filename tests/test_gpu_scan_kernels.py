@@ -7,6 +7,10 @@ Tolerances: as in the other parity tests, FP64 1e-9 relative to max(1,
 4,100 x 2^-53 x a condition number below 1e3), FP32 1e-4 for means and 1e-3 for
 covariances against the oracle on the same FP32-rounded inputs.
 """
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -73,6 +77,7 @@ def check_pass(nx, ny, lengths, sqrt, dtype, schedules, seed=0, sequential=False
         ells.append(ell)
     tm, tc, te = (1e-9, 1e-9, 1e-9) if dtype == torch.float64 else (1e-4, 1e-3, 1e-3)
     n = sum(T + 1 for T in lengths)
+    counts = []
     for sch in schedules:
         r = IteratedSmoother(list(lengths), td, od, method, sqrt=sqrt, dtype=dtype, sequential=sequential)
         if sch is not None:
@@ -86,6 +91,8 @@ def check_pass(nx, ny, lengths, sqrt, dtype, schedules, seed=0, sequential=False
             close(npy(gm[s]), ref[0], tm, what + " mean")
             close(gram(npy(gL[s])) if sqrt else npy(gL[s]), gram(ref[1]) if sqrt else ref[1], tc, what + " cov")
             close(npy(ell)[s], np.asarray(ells[s]), te, what + " log-likelihood")
+        counts.append(r.fallback_count())
+    return counts
 
 
 # chunk 1, so that the level edges (1, 16, 256, 4096 items of one, two, three and
@@ -171,6 +178,34 @@ def test_sampling_chunks(states, sqrt, samples):
     # the recursion uses the noise factors themselves; a filtered factor of the
     # oracle is lower triangular with a positive diagonal, as the kernels' are
     close(npy(got), ref, 1e-9, f"{states} states, {samples} samples")
+
+
+GUARDED = """
+import sys
+sys.path[:0] = {path!r}
+import torch
+from tests.test_gpu_scan_kernels import N, ROW, QUAD, check_pass, extended, cubature
+from parsmooth import set_fp32_fallback
+set_fp32_fallback(1.0)
+for method in (extended, cubature):
+    count = check_pass(5, 2, [1500, 1, 700], True, torch.float32,
+                       [None, (1, 1 | ROW), (2, 2 | QUAD), (2, 2 | QUAD | N.SCAN_HALF), (2, 2), (4, 2)], seed=8, method=method)
+    print(method.__name__, "recomputed", count, flush=True)
+    assert all(n > 0 for n in count)
+print("guarded launches agree")
+"""
+
+
+def test_guarded_recomputation():
+    """Every kernel of an FP32 pass as the pair of launches that large problems take
+    (PSM_FB_SINGLE_WAVES=0, read once per process), with the threshold at which every
+    check raises its flag: the second launches run, on 1, 4 and 16 lanes a
+    combination, find their inputs as the first had them, and count."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    code = GUARDED.format(path=[root, os.path.join(root, "sqrt-parallel-smoothers_amd")])
+    out = subprocess.run([sys.executable, "-c", code], env={**os.environ, "PSM_FB_SINGLE_WAVES": "0"}, cwd=root,
+                         capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0 and "guarded launches agree" in out.stdout, out.stdout + out.stderr
 
 
 def _build(theta, nx=2):
