@@ -508,8 +508,8 @@ struct Impl {
   }
 
   static int linearize_states(const Plan& pl, const psm_model_t* tr, const psm_model_t* ob,
-                              const psm_sigma_t* sg, const void* nm, const void* nL, char* ws,
-                              hipStream_t st, const Fallback& fb, Guards& g) {
+                              const psm_sigma_t* sg, const void* nm, const void* nL, RefSource<R> rs,
+                              char* ws, hipStream_t st, const Fallback& fb, Guards& g) {
     int use = 0;
     SigmaView<R> sv = sigma_view<R>(sg, &use);
     ModelView<R> trv = model_view<R>(tr);
@@ -519,11 +519,14 @@ struct Impl {
     // nm == nullptr: the nominal is the workspace trajectory (state-interleaved)
     const int inter = nm == nullptr ? 1 : 0;
     if (inter) nm = ws + pl.off_traj;
+    const bool linear = !use && tr->kind == PSM_MODEL_LINEAR;
+    rs.mode = linear && rs.fm ? REF_FILTERED
+              : linear && ob && ob->kind == PSM_MODEL_LINEAR ? REF_CHECKED : REF_NOMINAL;
     TimedScope ts_("k_linearize_states", st);
     launch_fb(fb, g, grid_for(pl.Mp, kLaneWG), grid_for(pl.Mp, kLaneWG), [&](auto f) {
       hipLaunchKernelGGL((k_linearize_states<R, NX, NY, SQRT, decltype(f)>), dim3(grid_for(pl.Mp, kLaneWG)),
                          dim3(kLaneWG), 0, st, pl.M, pl.Mp, pl.chunk, trv, obv, ob ? 1 : 0, sv, use,
-                         (const R*)nm, (const R*)nL, inter, (R*)(ws + pl.off_lin), (R*)(ws + pl.off_ref), f);
+                         (const R*)nm, (const R*)nL, inter, rs, (R*)(ws + pl.off_lin), (R*)(ws + pl.off_ref), f);
     });
     return hip_check("k_linearize_states");
   }
@@ -543,7 +546,8 @@ struct Impl {
     const Fallback fb{p->fallback_ratio, p->fallback_count};
     Guards g = guards(pl, ws, st);
     if (!lin_done) {
-      rc = linearize_states(pl, tr, ob, sg, nm, nL, ws, st, fb, g);
+      rc = linearize_states(pl, tr, ob, sg, nm, nL,
+                            RefSource<R>{0, p->state_offsets, p->n_seq, (const R*)ys, (const R*)m0, nullptr}, ws, st, fb, g);
       if (rc) return rc;
     }
     const R* lin = (const R*)(ws + pl.off_lin);
@@ -604,7 +608,8 @@ struct Impl {
     const Fallback fb{p->fallback_ratio, p->fallback_count};
     Guards g = guards(pl, ws, st);
     if (!lin_done) {
-      rc = linearize_states(pl, tr, nullptr, sg, nm, nL, ws, st, fb, g);
+      rc = linearize_states(pl, tr, nullptr, sg, nm, nL,
+                            RefSource<R>{0, p->state_offsets, p->n_seq, nullptr, nullptr, (const R*)fm}, ws, st, fb, g);
       if (rc) return rc;
     }
     // fm == nullptr: the filtered trajectory is the workspace trajectory; om ==
@@ -677,7 +682,8 @@ struct Impl {
     char* ws = (char*)wsv;
     const Fallback fb{p->fallback_ratio, p->fallback_count};
     Guards g = guards(pl, ws, st);
-    int rc = linearize_states(pl, tr, nullptr, sg, nm, nL, ws, st, fb, g);
+    int rc = linearize_states(pl, tr, nullptr, sg, nm, nL,
+                              RefSource<R>{0, p->state_offsets, p->n_seq, nullptr, nullptr, (const R*)fm}, ws, st, fb, g);
     if (rc) return rc;
     // smoother elements at every state (the chunk aggregates it also forms are not used)
     launch_fb(fb, g, grid_for(pl.nchunks, kLaneWG), grid_for(pl.nchunks, kLaneWG), [&](auto f) {

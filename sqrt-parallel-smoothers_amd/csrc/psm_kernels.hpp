@@ -267,7 +267,7 @@ PSM_DEV void linearize_point_w(const ModelView<R>& md, const SigmaView<R>& sp, i
     // linearizes every point again with the FP64 path below
     if (!use_sigma) {
       linearize_extended<R, NIN, NOUT>(md, m, F, C, b);
-      if constexpr (From::kNominal) centre(F, m, from.next, b);
+      if constexpr (From::kNominal) centre(F, from.at, from.next, b);
       return;
     }
     const bool done = md.kind != PSM_MODEL_CONDITIONAL &&
@@ -276,7 +276,7 @@ PSM_DEV void linearize_point_w(const ModelView<R>& md, const SigmaView<R>& sp, i
   } else if constexpr (IsSingle<R>::value) {
     if (!use_sigma) {
       linearize_extended<R, NIN, NOUT>(md, m, F, C, b);
-      if constexpr (From::kNominal) centre(F, m, from.next, b);
+      if constexpr (From::kNominal) centre(F, from.at, from.next, b);
       return;
     }
     bool done = false;
@@ -313,12 +313,71 @@ PSM_DEV void linearize_point_w(const ModelView<R>& md, const SigmaView<R>& sp, i
 // size of the posterior's spread, and not x, a position of 10 to 1000: the
 // smoothed means of a T = 16,385 pass were 1.5e-5 of their norm off a 64-bit
 // recursion, and are 1.8e-6 with this.  ref holds n_k (blocked at the states'
-// interleaved positions, NX words).  Trajectories hold n + d in either layout, so that a
+// interleaved positions, NX words; RefSource).  Trajectories hold n + d in either layout, so that a
 // launch sequence and the host loop over the same passes agree bit for bit.
 template <typename R, bool SQRT>
 constexpr bool kCentred = SQRT && std::is_same<R, float>::value;
 
-// m -/+ the nominal mean at interleaved position pos
+// Which values the means are held relative to.  A regression and the nonlinear models
+// take the nominal, which their result depends on in any case.  A linear model
+// under the extended rule does not, and must not lose the digits of a nominal that is
+// far from the states, or all of them to one that is not finite: with a linear
+// transition a smoother or a sampler takes the filtered mean, and with a linear
+// observation too a filter takes the prior mean where there is one, the nominal
+// in the components that are observed, as far as their contributions to an observation
+// are no larger than twice the observation, and zero elsewhere (constant velocity in
+// the plane, T = 5,000, means against FP64: a nominal near the states 2.5e-8 of the
+// norm off; zeros, one 1e4 or 1e6 away or not a number 1.5e-7, where relative to it
+// they were 2.4e-6 and 1.9e-4 off or lost; absolute means were 2.8e-7 off).
+enum { REF_NOMINAL = 0, REF_CHECKED = 1, REF_FILTERED = 2 };
+template <typename R>
+struct RefSource {
+  int mode;
+  const int64_t* soff;
+  int nseq;
+  const R* ys;
+  const R* m0;
+  const R* fm;
+};
+// The reference of state i, whose nominal mean is n.
+template <typename R, int NX, int NY>
+PSM_DEV void ref_mean(const RefSource<R>& rs, const ModelView<R>& ob, int64_t i, const R (&n)[NX], R (&ref)[NX]) {
+  copy(n, ref);
+  if (rs.mode == REF_FILTERED) {
+    ld_aos(rs.fm, i, ref);
+  } else if (rs.mode == REF_CHECKED) {
+    const int s = seq_of(rs.soff, rs.nseq, i);
+    if (i == rs.soff[s]) {
+      ld_aos(rs.m0, s, ref);
+    } else {
+      R y[NY];
+      ld_aos(rs.ys, i - s - 1, y);
+      bool seen[NX], far[NX];
+#pragma unroll
+      for (int j = 0; j < NX; ++j) seen[j] = far[j] = false;
+#pragma unroll
+      for (int r = 0; r < NY; ++r) {
+        R a = R(0);
+#pragma unroll
+        for (int j = 0; j < NX; ++j) a += ob.par(r * NX + j) != R(0) ? abs_(ob.par(r * NX + j) * n[j]) : R(0);
+        const bool ok = a <= R(2) * abs_(y[r] - ob.qm(r));   // not for NaN
+#pragma unroll
+        for (int j = 0; j < NX; ++j) {
+          if (ob.par(r * NX + j) != R(0)) {
+            seen[j] = true;
+            far[j] = far[j] || !ok;
+          }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < NX; ++j) ref[j] = seen[j] && !far[j] ? n[j] : R(0);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NX; ++j) ref[j] = isfinite(ref[j]) ? ref[j] : R(0);
+}
+
+// m -/+ the reference mean at interleaved position pos
 template <typename R, int NX>
 PSM_DEV void to_centred(const R* __restrict__ ref, int64_t pos, R (&m)[NX]) {
   R n[NX];
@@ -342,7 +401,7 @@ template <typename R, int NX, int NY, bool SQRT, typename FB = Fallback>
 __global__ __launch_bounds__(kLaneWG) void k_linearize_states(
     int64_t M, int64_t Mp, int C, ModelView<R> tr, ModelView<R> ob, int do_obs, SigmaView<R> sp,
     int use_sigma, const R* __restrict__ nom_m, const R* __restrict__ nom_L, int nom_inter,
-    R* __restrict__ lin, R* __restrict__ ref, FB fb) {
+    RefSource<R> rs, R* __restrict__ lin, R* __restrict__ ref, FB fb) {
   if (fb.skip()) return;
   // FP32: the rule is converted once per workgroup, and the regressions' increments
   // wait in LDS for their residual passes
@@ -369,26 +428,30 @@ __global__ __launch_bounds__(kLaneWG) void k_linearize_states(
   ob.row = i;
   R m[NX], L[NX][NX];
   traj_load<!SQRT, R, NX>(nom_m, nom_L, nom_inter, i, t, m, L);
+  R at[NX];
+  if constexpr (kCentred<R, SQRT>) ref_mean<R, NX, NY>(rs, ob, i, m, at);
   R* lp = blk<Step<R, NX, NY>::NQ>(lin, t);
   auto run = [&](const auto& pc) {
     {
       R F[NX][NX], Cq[NX][NX], b[NX];
       if constexpr (kCentred<R, SQRT>) {
         R next[NX];
-        copy(m, next);
+        copy(at, next);
         if (i + 1 < M) {
+          R n[NX];
           if (nom_inter) {
             // the next slot of this chunk, or the first of the next
             const int64_t pos = (r >> 6) + 1 < C ? t + 64 : StateMap{C}(i + 1);
             int q = 0;
-            ld(blk<kTrajWords<!SQRT, NX>>(nom_m, pos), kBlk, 0, q, next);
+            ld(blk<kTrajWords<!SQRT, NX>>(nom_m, pos), kBlk, 0, q, n);
           } else {
-            ld_aos(nom_m, i + 1, next);
+            ld_aos(nom_m, i + 1, n);
           }
+          ref_mean<R, NX, NY>(rs, ob, i + 1, n, next);
         }
         int q = 0;
-        st(blk<NX>(ref, t), kBlk, 0, q, m);
-        linearize_point_w<R, NX, NX, SQRT>(tr, sp, use_sigma, m, L, F, Cq, b, fb, pc, FromNominal<R, NX>{next});
+        st(blk<NX>(ref, t), kBlk, 0, q, at);
+        linearize_point_w<R, NX, NX, SQRT>(tr, sp, use_sigma, m, L, F, Cq, b, fb, pc, FromNominal<R, NX, NX>{at, next});
       } else {
         linearize_point_w<R, NX, NX, SQRT>(tr, sp, use_sigma, m, L, F, Cq, b, fb, pc);
       }
@@ -402,7 +465,7 @@ __global__ __launch_bounds__(kLaneWG) void k_linearize_states(
       R H[NY][NX], Cr[NY][NY], c[NY];
       if constexpr (kCentred<R, SQRT>) {
         const R zero[NY] = {};
-        linearize_point_w<R, NX, NY, SQRT>(ob, sp, use_sigma, m, L, H, Cr, c, fb, pc, FromNominal<R, NY>{zero});
+        linearize_point_w<R, NX, NY, SQRT>(ob, sp, use_sigma, m, L, H, Cr, c, fb, pc, FromNominal<R, NX, NY>{at, zero});
       } else {
         linearize_point_w<R, NX, NY, SQRT>(ob, sp, use_sigma, m, L, H, Cr, c, fb, pc);
       }

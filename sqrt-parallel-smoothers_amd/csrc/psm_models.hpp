@@ -705,15 +705,16 @@ struct NoPoints {
   static constexpr bool kOn = false;
 };
 // Where the offset of a linearization y = F x + b starts: at zero (b as it stands), or,
-// with x and y differences from a nominal, at the nominal value of y: b = E f - next,
-// for which F is not used.
+// with x and y differences from `at` and `next`, there: b + F at - next.  Where x is
+// linearized at `at`, that is E f - next, without F.
 struct FromZero {
   static constexpr bool kNominal = false;
 };
-template <typename R, int N>
+template <typename R, int NIN, int NOUT>
 struct FromNominal {
   static constexpr bool kNominal = true;
-  const R (&next)[N];
+  const R (&at)[NIN];
+  const R (&next)[NOUT];
 };
 
 template <typename R, int NIN, int NOUT, bool SQRT, typename S, typename PC, typename From>

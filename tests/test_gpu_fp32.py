@@ -7,6 +7,8 @@ import numpy as np
 import pytest
 import torch
 
+from oracle import psm_oracle as O
+
 pytestmark = pytest.mark.gpu
 
 if not torch.cuda.is_available():  # pragma: no cover
@@ -16,8 +18,8 @@ import parsmooth  # noqa: E402
 from parsmooth import FunctionalModel, MVNSqrt  # noqa: E402
 from parsmooth import models as M  # noqa: E402
 from parsmooth.batch import IteratedSmoother  # noqa: E402
-from parsmooth.data import bearings_data_batch  # noqa: E402
-from parsmooth.linearization import cubature, unscented  # noqa: E402
+from parsmooth.data import bearings_data_batch, cv_model, lgssm_data  # noqa: E402
+from parsmooth.linearization import cubature, extended, unscented  # noqa: E402
 
 DEV = torch.device("cuda", 0)
 DT = float(np.float32(0.01))
@@ -103,3 +105,65 @@ def test_regressions_far_from_the_origin(method):
     np.testing.assert_allclose(m1, m0, rtol=0, atol=0.5 * grid + 2e-5)
     np.testing.assert_allclose(f1, f0, rtol=0, atol=1e-5)
     assert abs(e1 - e0) <= T * 4 * 2.0 ** -24, (e1, e0)
+
+
+NOMINALS = {"near": lambda x: x, "far": lambda x: x + 1e4, "farther": lambda x: -1e6 + 0 * x,
+            "nan": lambda x: np.where(np.arange(len(x))[:, None] % 7 == 3, np.nan, x),
+            "infinite": lambda x: np.where(np.arange(len(x))[:, None] % 2 == 0, np.inf, -np.inf) + 0 * x}
+
+
+@pytest.mark.parametrize("nominal", NOMINALS)
+def test_linear_models_do_not_use_the_nominal(nominal):
+    """A linear model under the extended rule does not depend on the nominal: neither a
+    far one nor one that is not finite may cost its result anything.  Bounds: FP32
+    means and factors are held to 2^-24 of their size, and a pass adds a few tens of
+    such errors: 2e-6."""
+    T = 700
+    F, Q, H, R = (r32(a) for a in cv_model())
+    cQ, cR = r32(np.linalg.cholesky(Q)), r32(np.linalg.cholesky(R))
+    m0, L0 = r32([30.0, -20.0, 1.0, 2.0]), r32(np.eye(4))
+    x, ys = (r32(a) for a in lgssm_data(m0, F, H, cR @ cR.T, cQ @ cQ.T, np.zeros(4), np.zeros(2), T, random_state=3))
+    to, oo = O.FunctionalModel(O.Linear(F), O.MVNSqrt(np.zeros(4), cQ)), O.FunctionalModel(O.Linear(H), O.MVNSqrt(np.zeros(2), cR))
+    f, ell = O.filtering(ys, O.MVNSqrt(m0, L0), to, oo, O.extended, None, True, return_loglikelihood=True)
+    ref = O.smoothing(to, f, O.extended, None, True)
+    t = lambda a: torch.as_tensor(np.asarray(a, np.float32), device=DEV)
+    td = FunctionalModel(M.LinearFunction(t(F)), MVNSqrt(t(np.zeros(4)), t(cQ)))
+    od = FunctionalModel(M.LinearFunction(t(H)), MVNSqrt(t(np.zeros(2)), t(cR)))
+    x0, nom = MVNSqrt(t(m0), t(L0)), MVNSqrt(t(NOMINALS[nominal](x)), t(np.tile(np.eye(4), (T + 1, 1, 1))))
+
+    def near(got, want, what):
+        got, want = npy(got), np.asarray(want)
+        assert np.abs(got - want).max() <= 2e-6 * np.abs(want).max(), (nominal, what, np.abs(got - want).max())
+
+    fd, ell_d = parsmooth.filtering(t(ys), x0, td, od, extended, nom, return_loglikelihood=True)
+    near(fd.mean, f[0], "filtered mean")
+    near(ell_d, ell, "log-likelihood")
+    exact = MVNSqrt(t(f[0]), t(f[1]))
+    near(parsmooth.smoothing(td, exact, extended, nom).mean, O.smoothing(to, O.MVNSqrt(r32(f[0]), r32(f[1])), O.extended, None, True)[0],
+         "smoothed mean")
+    post = parsmooth.filter_smoother(t(ys), x0, td, od, extended, nom)
+    near(post.mean, ref[0], "mean of the joint pass")
+    for k in (2, 3):
+        post = parsmooth.iterated_smoothing(t(ys), x0, td, od, extended, nom, criterion=parsmooth.FixedIterations(k))
+        near(post.mean, ref[0], f"{k} iterations")
+    eps = np.random.RandomState(1).randn(T + 1, 3, 4)
+    near(parsmooth.sampling(t(eps), 3, td, exact, extended, nom),
+         O.sampling(r32(eps), to, O.MVNSqrt(r32(f[0]), r32(f[1])), O.extended, O.MVNSqrt(f[0], f[1])), "samples")
+
+
+def test_unused_nominal_components():
+    """The coordinated turn with positions observed linearly uses the nominal's
+    velocity and turn rate only: its positions may be anything."""
+    T = 300
+    states, _ = bearings_data_batch([T], [[3.0, 2.0, 1.0, 0.0]], DT, 0.5, S1, S2, q=3.16, seed=5)
+    x = states[0].astype(np.float64)
+    t = lambda a: torch.as_tensor(np.asarray(a, np.float32), device=DEV)
+    ys = t(x[1:, :2] + 0.1 * np.random.RandomState(0).randn(T, 2))
+    od = FunctionalModel(M.LinearFunction(t(np.eye(2, 5))), MVNSqrt(t(np.zeros(2)), t(0.1 * np.eye(2))))
+    x0, L = MVNSqrt(t(x[0]), t(0.3 * np.eye(5))), t(np.tile(0.1 * np.eye(5), (T + 1, 1, 1)))
+    out = []
+    for fill in (0.0, np.nan):
+        nm = x.copy()
+        nm[:, :2] = fill
+        out.append(parsmooth.filter_smoother(ys, x0, turn_models(torch.float32)[0], od, extended, MVNSqrt(t(nm), L)))
+    assert torch.equal(out[0].mean, out[1].mean) and torch.equal(out[0].chol, out[1].chol)
