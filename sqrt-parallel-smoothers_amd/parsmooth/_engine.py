@@ -68,10 +68,15 @@ class Problem:
     """Dims, dtype, form and the sequence layout of one batch.
 
     ``lengths[s]`` is the number of observations of sequence s; it owns
-    ``lengths[s] + 1`` states (its prior state first)."""
+    ``lengths[s] + 1`` states (its prior state first).
+
+    A kept problem may be used on any stream: its offsets are in place when the
+    constructor returns.  ``one_call``: the problem serves only calls on the current
+    stream, and its offsets may be filled in on it (a copy from host memory would
+    wait for what the stream still has to do)."""
 
     def __init__(self, nx: int, ny: int, lengths: Sequence[int], dtype: torch.dtype, sqrt: bool,
-                 dev, chunk: int = 0, tangent_code: Optional[int] = None):
+                 dev, chunk: int = 0, tangent_code: Optional[int] = None, one_call: bool = False):
         lengths = np.asarray(lengths, dtype=np.int64).reshape(-1)
         if lengths.size == 0 or np.any(lengths < 1):
             raise ValueError("every sequence needs at least one observation")
@@ -86,15 +91,13 @@ class Problem:
         self.dtype = dtype
         self.sqrt = sqrt
         self.dev = dev
-        # one sequence: [0, n_states] filled in on the device, since a copy from host
-        # memory would wait for what the stream still has to do
+        # FP64 re-triangularisation fallback of the FP32 square-root path
+        self.fallback_counter = torch.zeros(1, dtype=torch.int64, device=dev)
         self.state_offsets = torch.arange(0, 2 * self.n_states, self.n_states, device=dev) \
-            if self.n_seq == 1 else torch.as_tensor(offs).to(dev)
+            if one_call and self.n_seq == 1 else torch.as_tensor(offs).to(dev)
         code = N.dtype_code(dtype) if tangent_code is None else int(tangent_code)
         if not N.lib().psm_supported(code, N.FORM_SQRT if sqrt else N.FORM_STD, self.nx, self.ny):
             raise NotImplementedError(f"no compiled kernels for nx={nx}, ny={ny}, dtype code {code}")
-        # FP64 re-triangularisation fallback of the FP32 square-root path
-        self.fallback_counter = torch.zeros(1, dtype=torch.int64, device=dev)
         ratio = FP32_FALLBACK_RATIO if (code in (N.PSM_F32, N.PSM_F32_TANGENT) and sqrt) else 0.0
         if not chunk and "PSM_CHUNK" not in os.environ:
             # tangent types scan with one lane per combination: the library's choice,

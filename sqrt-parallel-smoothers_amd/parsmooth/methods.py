@@ -145,7 +145,7 @@ class _Iteration:
         self.m0 = m0.reshape(1, self.nx)
         self.L0 = to_dev(x0[1], self.dtype, self.dev).reshape(1, self.nx, self.nx)
         self.x0 = x0
-        self.prob = Problem(self.nx, self.ny, [self.T], self.dtype, self.sqrt, self.dev)
+        self.prob = Problem(self.nx, self.ny, [self.T], self.dtype, self.sqrt, self.dev, one_call=True)
         self.mods = Models(self.prob, transition_model, observation_model, self.method)
 
     def nominal(self, traj):

@@ -63,7 +63,7 @@ def sampling(key, n_samples: int, transition_model, filter_trajectory: Union[MVN
     nom_L = to_dev(nominal_trajectory[1], dtype, dev).reshape(n_states, nx, nx)
     n_samples = int(n_samples)
     eps = _normals(key, (n_states, n_samples, nx), dtype, dev)
-    prob = Problem(nx, 1, [n_states - 1], dtype, sqrt, dev)
+    prob = Problem(nx, 1, [n_states - 1], dtype, sqrt, dev, one_call=True)
     mods = Models(prob, transition_model, None, resolve(linearization_method))
     mods.prepare(nom_m, nom_L, obs=False)
     nbytes = int(N.lib().psm_sample_workspace_bytes(ctypes.byref(prob.struct), n_samples))

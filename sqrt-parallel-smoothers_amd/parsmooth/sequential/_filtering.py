@@ -31,7 +31,7 @@ def filtering(observations, x0: Union[MVNSqrt, MVNStandard], transition_model, o
     T = ys.shape[0]
     ys = ys.reshape(T, -1)
     ny = ys.shape[1]
-    prob = Problem(nx, ny, [T], dtype, sqrt, dev)
+    prob = Problem(nx, ny, [T], dtype, sqrt, dev, one_call=True)
     mods = Models(prob, transition_model, observation_model, method)
     L0 = to_dev(x0[1], dtype, dev).reshape(1, nx, nx)
     nom_m = nom_L = None

@@ -29,7 +29,7 @@ def smoothing(transition_model, filter_trajectory: Union[MVNSqrt, MVNStandard],
     n_states, nx = fm.shape
     fL = to_dev(filter_trajectory[1], dtype, dev).reshape(n_states, nx, nx)
     method = resolve(linearization_method)
-    prob = Problem(nx, 1, [n_states - 1], dtype, sqrt, dev)
+    prob = Problem(nx, 1, [n_states - 1], dtype, sqrt, dev, one_call=True)
     mods = Models(prob, transition_model, None, method)
     nom_m = nom_L = None
     if nominal_trajectory is not None:

@@ -93,6 +93,31 @@ def test_runner_graph_on_user_stream():
     assert torch.equal(m_g, m_e) and torch.equal(L_g, L_e) and torch.equal(ell_g, ell_e)
 
 
+def test_runner_built_on_another_stream():
+    """A kept runner's sequence offsets are in place when its constructor returns,
+    whatever its stream still has to do, so that another stream may run it at once."""
+    ys, x0, trans, obs = _case(700, 8)
+    init = t(np.tile([0.1, 0.2, 1.0, 0.0, 0.0], (701, 1))), t(np.tile(np.eye(5), (701, 1, 1)))
+    ref = IteratedSmoother([700], trans, obs, extended)
+    ref.set_data(ys, x0[0][None], x0[1][None])
+    want = [x.clone() for x in ref.run(2, init, use_graph=False, return_loglikelihood=True)]
+    work = torch.rand(4096, 4096, device=DEV)
+    torch.cuda.synchronize()
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(a):
+        for _ in range(60):
+            work = work @ work
+            work = work / work.norm()
+        r = IteratedSmoother([700], trans, obs, extended)
+    with torch.cuda.stream(b):
+        offsets = r.prob.state_offsets.clone()
+        r.set_data(ys, x0[0][None], x0[1][None])
+        got = r.run(2, init, use_graph=False, return_loglikelihood=True)
+        assert offsets.tolist() == [0, 701]
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
 def test_graph_cache_drops_least_recently_used():
     """More distinct graphs than the cache keeps (64): every call still returns
     its eager result, including calls whose graph was dropped and captured
