@@ -61,6 +61,13 @@ struct SampleItem {
       R s = a.g[i];
 #pragma unroll
       for (int j = 0; j <= i; ++j) s = fma(L[i][j], eps[j], s);
+      if constexpr (SQRT) {
+        // the last state's is the caller's filtered factor, any square root
+        if (a.flag == FLAG_HEAD) {
+#pragma unroll
+          for (int j = i + 1; j < NX; ++j) s = fma(L[i][j], eps[j], s);
+        }
+      }
       y[i] = off ? s : R(0);
 #pragma unroll
       for (int j = 0; j < NX; ++j) y[i] = fma(a.E[i][j], x[j], y[i]);

@@ -180,6 +180,25 @@ def test_sampling_chunks(states, sqrt, samples):
     close(npy(got), ref, 1e-9, f"{states} states, {samples} samples")
 
 
+@pytest.mark.parametrize("states", [2, 17, 257])
+def test_sampling_of_any_factors(states):
+    """Filtered factors that are square roots without a triangle of zeros: the last
+    state's draw is its mean and that factor times the normals, as it stands."""
+    nx, T, samples = 3, states - 1, 5
+    F, cQ, b, H, cR, c, m0, L0, obs = problem(nx, 2, [T], 5, torch.float64)
+    t = lambda a: torch.as_tensor(np.ascontiguousarray(a), device=DEV)
+    to = O.FunctionalModel(O.Linear(F), O.MVNSqrt(b, cQ))
+    oo = O.FunctionalModel(O.Linear(H), O.MVNSqrt(c, cR))
+    filt = O.filtering(obs[0], O.MVNSqrt(m0[0], L0[0]), to, oo, O.extended, None, True)
+    turned = filt[1] @ np.linalg.qr(np.random.RandomState(2).randn(states, nx, nx))[0]
+    filt = O.MVNSqrt(filt[0], turned)
+    eps = np.random.RandomState(1).randn(states, samples, nx)
+    ref = O.sampling(eps, to, filt, O.extended, filt)
+    traj = MVNSqrt(t(filt[0]), t(turned))
+    got = parsmooth.sampling(t(eps), samples, FunctionalModel(M.LinearFunction(t(F)), MVNSqrt(t(b), t(cQ))), traj, extended, traj)
+    close(npy(got), ref, 1e-9, f"{states} states")
+
+
 GUARDED = """
 import sys
 sys.path[:0] = {path!r}
