@@ -357,7 +357,7 @@ PSM_DEV void sqrt_absorb(FAgg<R, NX>& a, const Step<R, NX, NY>& s, const R (&y)[
     x[0] = a.Z[i][i];
 #pragma unroll
     for (int j = 0; j < NY; ++j) x[1 + j] = G[j][i];
-    const Pivot<R> pv = make_pivot(x[0], pivot_norm2<1 + NY, 0>(x, 0));
+    const PivotOf<R> pv = make_pivot(x[0], pivot_norm2<1 + NY, 0>(x, 0));
     a.Z[i][i] = pv.nrm;
 #pragma unroll
     for (int k = i + 1; k < NX; ++k) {
@@ -396,7 +396,7 @@ PSM_DEV void sqrt_absorb(FAgg<R, NX>& a, const Step<R, NX, NY>& s, const R (&y)[
 template <typename R, int NX>
 struct FilterArray {
   R x[NX][2 * NX];
-  Pivot<R> pv[NX];
+  PivotOf<R> pv[NX];
   // x[:, :NX] = W on entry
   PSM_DEV void reduce() {
 #pragma unroll

@@ -63,9 +63,12 @@ template <typename B> PSM_DEV DualT<B> fma(DualT<B> a, DualT<B> b, DualT<B> c) {
 // derivative of sqrt taken as 0 at 0 (zero rows carry zero tangents)
 template <typename B> PSM_DEV DualT<B> sqrt_(DualT<B> a) {
   const B s = sqrt_(a.v);
-  return {s, s > B(0) ? a.d / (B(2) * s) : B(0)};
+  return {s, s > B(0) ? B(0.5) * a.d * rcp_(s) : B(0)};
 }
-template <typename B> PSM_DEV DualT<B> rcp_(DualT<B> a) { return DualT<B>(1.0) / a; }
+template <typename B> PSM_DEV DualT<B> rcp_(DualT<B> a) {
+  const B r = rcp_(a.v);
+  return {r, -(a.d * r) * r};
+}
 template <typename B> PSM_DEV DualT<B> abs_(DualT<B> a) { return a.v < B(0) ? -a : a; }
 // a zero whose tangent is not zero counts
 template <typename B> PSM_DEV bool nonzero_(DualT<B> a) { return a.v != B(0) || a.d != B(0); }

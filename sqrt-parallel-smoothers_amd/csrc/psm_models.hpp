@@ -402,52 +402,27 @@ PSM_DEV void linearize_sigma(const ModelView<R, S>& md, const SigmaView<R>& sp, 
       // point (the reference triangularises all columns at once); a batch
       // past the last point is padded with zero columns
       batched = true;
-      if constexpr (is_dual<R>::value) {
-        // tangent types: one column at a time by rotations of (diagonal, column),
-        // since a batch beside its tangents spills (154 to 294 registers)
-        for (int p = 0; p < sp.npts; ++p) {
-          R x[NOUT], w;
-          point(p, x, w);
-          const R sw = sqrt_(w);
+      for (int p0 = 0; p0 < sp.npts; p0 += kSigmaBatch) {
+        R Ab[NOUT][NOUT + kSigmaBatch];
 #pragma unroll
-          for (int i = 0; i < NOUT; ++i) x[i] = sw * x[i];
+        for (int i = 0; i < NOUT; ++i)
 #pragma unroll
-          for (int i = 0; i < NOUT; ++i) {
-            const R n2 = fma(Acc[i][i], Acc[i][i], x[i] * x[i]);
-            const bool ok = !(n2 <= R(pivot_min<R>()));
-            const R inv = rcp_(sqrt_(ok ? n2 : R(1)));
-            const R c = ok ? Acc[i][i] * inv : R(1), sn = ok ? x[i] * inv : R(0);
+          for (int j = 0; j < NOUT; ++j) Ab[i][j] = Acc[i][j];
 #pragma unroll
-            for (int k = i; k < NOUT; ++k) {
-              const R t = Acc[k][i];
-              Acc[k][i] = fma(c, t, sn * x[k]);
-              x[k] = fma(c, x[k], -(sn * t));
-            }
-          }
+        for (int k = 0; k < kSigmaBatch; ++k) {
+          R d[NOUT], w = R(0);
+          set_zero(d);
+          const bool live = p0 + k < sp.npts;
+          if (live) point(p0 + k, d, w);
+          const R sw = live ? sqrt_(w) : R(0);
+#pragma unroll
+          for (int i = 0; i < NOUT; ++i) Ab[i][NOUT + k] = sw * d[i];
         }
-      } else {
-        for (int p0 = 0; p0 < sp.npts; p0 += kSigmaBatch) {
-          R Ab[NOUT][NOUT + kSigmaBatch];
+        tria_inplace<R, NOUT, NOUT + kSigmaBatch>(Ab);
 #pragma unroll
-          for (int i = 0; i < NOUT; ++i)
+        for (int i = 0; i < NOUT; ++i)
 #pragma unroll
-            for (int j = 0; j < NOUT; ++j) Ab[i][j] = Acc[i][j];
-#pragma unroll
-          for (int k = 0; k < kSigmaBatch; ++k) {
-            R d[NOUT], w = R(0);
-            set_zero(d);
-            const bool live = p0 + k < sp.npts;
-            if (live) point(p0 + k, d, w);
-            const R sw = live ? sqrt_(w) : R(0);
-#pragma unroll
-            for (int i = 0; i < NOUT; ++i) Ab[i][NOUT + k] = sw * d[i];
-          }
-          tria_inplace<R, NOUT, NOUT + kSigmaBatch>(Ab);
-#pragma unroll
-          for (int i = 0; i < NOUT; ++i)
-#pragma unroll
-            for (int j = 0; j < NOUT; ++j) Acc[i][j] = Ab[i][j];
-        }
+          for (int j = 0; j < NOUT; ++j) Acc[i][j] = Ab[i][j];
       }
     }
   }
