@@ -43,23 +43,32 @@ def compute_dtype(x0) -> torch.dtype:
     return torch.float64
 
 
-def states_per_chunk(n_states: int) -> int:
+def states_per_chunk(n_states: int, nx: int = 5, dtype: torch.dtype = torch.float64) -> int:
     """States per chunk, 0 for the library's choice (4 to 16: 32,768 chunks).
 
     A lane's chain through a state of its chunk is longer than one through a level
-    of the scan, and up to 4096 chunks (8192 with a fan-in of 2) the 16-lane scan has
-    three levels however many there are: few states take chunks as short as that
-    allows (six iterations, FP64, against 4: T = 200 638 us at 1, 843; 3,000 845 at
-    1, 1035; 6,000 942 at 2, 1118; 12,000 1079 at 3, 1159; 20,000 1235 at 3, 1299;
-    beyond 24,576 it takes a fourth level and gains 1 % either way).  Where the chip
-    is full many times over, the scan's share is what counts, and shrinks with the
-    chunk (FP32, two iterations: 1,024 ragged tracks of up to 4,096 4.12 ms at 24,
-    4.40 at 16; up to 8,192 7.50 at 40, 8.00; 4,096 of those 28.1 at 40, 29.2)."""
+    of the scan, and up to 4096 chunks the 16-lane scan has three levels of 16 groups,
+    however many chunks there are: up to 3 * 4096 states the chunk is as short as
+    that allows (six iterations, FP64, nx = 5, against 4: T = 200 568 us at 1, 758;
+    3,000 757 at 1, 927; 4,500 813 at 2, 951; 11,000 953 at 3, 1025).  With more
+    chunks the fan-in of 2 keeps three levels up to 32,768 of them, and what a chunk
+    costs and saves crosses slowly: the lines at 8192 chunks and 24,576 states are
+    measured (15,000 1022 at 2, 1074 at 3; 24,000 1119 at 3, 1202 at 4; 26,000 1199
+    at 3, 1202 at 4, 1147 at 2; 60,000 1360 at 4, 1470 at 2).  FP32, the covariance
+    form and nx = 2 and 6 cross at the same sizes: from 200 to 24,000 states the rule is
+    1 to 33 % faster than a chunk of 4 in all of them.
+
+    Where the chip is full many times over, the scan's share is what counts, and
+    shrinks with the chunk (one iteration, against 16: FP64, nx = 5, 2.2 million states
+    2.47 ms at 24, 2.61; 4.2 million 4.32 at 40, 4.72; 8.5 million 8.62 at 40, 9.00; FP32
+    1.46, 1.58; 2.59, 2.80; 5.03, 5.21; the covariance form, nx 4 to 8, and nx 2 in FP64
+    gain up to 11 % and lose at most 3).  FP32 items of one or two dimensions are too small for
+    it (nx = 2, 4.2 million states: 784 us at 16, 889 at 40)."""
     if n_states <= 3 * 4096:
         return -(-n_states // 4096)
     if n_states <= 3 * 8192:
         return -(-n_states // 8192)
-    if n_states >= 1 << 21:
+    if n_states >= 1 << 21 and nx * dtype.itemsize >= 16:
         return 40 if n_states >= 1 << 22 else 24
     return 0
 
@@ -99,13 +108,9 @@ class Problem:
         if not N.lib().psm_supported(code, N.FORM_SQRT if sqrt else N.FORM_STD, self.nx, self.ny):
             raise NotImplementedError(f"no compiled kernels for nx={nx}, ny={ny}, dtype code {code}")
         ratio = FP32_FALLBACK_RATIO if (code in (N.PSM_F32, N.PSM_F32_TANGENT) and sqrt) else 0.0
-        if not chunk and "PSM_CHUNK" not in os.environ:
-            # tangent types scan with one lane per combination: the library's choice,
-            # longer where the chip is full (FP64, a million states: 349 ms at 40, 392)
-            chunk = states_per_chunk(self.n_states) if tangent_code is None else \
-                40 if self.n_states >= 1 << 20 else 0
+        self.tangent = tangent_code is not None
         self.struct = N.PsmProblem(code, N.FORM_SQRT if sqrt else N.FORM_STD,
-                                   self.nx, self.ny, self.n_seq, int(chunk), self.n_states,
+                                   self.nx, self.ny, self.n_seq, int(chunk) or self.default_chunk(), self.n_states,
                                    self.state_offsets.data_ptr(), float(ratio), 0,
                                    self.fallback_counter.data_ptr())
         self.ws_bytes = int(N.lib().psm_workspace_bytes(ctypes.byref(self.struct)))
@@ -123,9 +128,20 @@ class Problem:
                                         N.SCAN_TEAM | N.SCAN_QUAD | N.SCAN_HALF)
                         for k in (2, 4, 8)) + tuple(k | N.SCAN_TEAM | N.SCAN_ROW for k in (1, 2))
 
+    def default_chunk(self) -> int:
+        """The chunk of a problem for which none is asked (0: the library's choice)."""
+        if "PSM_CHUNK" in os.environ:
+            return 0
+        if self.tangent:
+            # tangent types scan with one lane per combination: the library's choice,
+            # longer where the chip is full (FP64, a million states: 349 ms at 40, 392)
+            return 40 if self.n_states >= 1 << 20 else 0
+        return states_per_chunk(self.n_states, self.nx, self.dtype)
+
     def set_schedule(self, chunk: int, scan_k: int):
-        """Fix the launch schedule (0 = library default) and resize the workspace."""
-        self.struct.chunk = int(chunk)
+        """Fix the launch schedule and resize the workspace.  (0, 0) is a new problem's
+        schedule; with a scan_k of its own, chunk 0 is the library's choice."""
+        self.struct.chunk = int(chunk) if chunk or scan_k else self.default_chunk()
         self.struct.scan_k = int(scan_k)
         nbytes = int(N.lib().psm_workspace_bytes(ctypes.byref(self.struct)))
         if nbytes == 0:

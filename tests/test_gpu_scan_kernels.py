@@ -145,15 +145,21 @@ def test_sequential_ahead(nseq, nx, ny, sqrt):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64], ids=["fp32", "fp64"])
 @pytest.mark.parametrize("n_states", [1, 4096, 4097, 8192, 8193, 12288, 12289, 24576, 24577, 1 << 21, 1 << 22])
 def test_states_per_chunk(n_states, dtype):
-    """The chunk rule at its lines: chunks as it says, and a pass of the shorter
-    ones agrees with the oracle (test_level_edges does the short ones)."""
+    """The chunk rule at its lines: chunks as it says, for a problem as it is made and
+    after set_schedule(0, 0), and a pass of the shorter ones agrees with the oracle
+    (test_level_edges does the short ones)."""
     from parsmooth._engine import Problem, states_per_chunk
     want = {1: 1, 4096: 1, 4097: 2, 8192: 2, 8193: 3, 12288: 3, 12289: 2, 24576: 3, 24577: 0, 1 << 21: 24, 1 << 22: 40}
     assert states_per_chunk(n_states) == want[n_states]
     if n_states > 1:
         p = Problem(2, 1, [n_states - 1], dtype, True, DEV)
-        assert p.struct.chunk == want[n_states]
+        small = dtype == torch.float32 and n_states >= 1 << 21   # two FP32 words a state: the library's choice
+        assert p.struct.chunk == (0 if small else want[n_states])
         assert p.state_offsets.tolist() == [0, n_states]
+        p.set_schedule(5, 2)
+        assert (p.struct.chunk, p.struct.scan_k) == (5, 2)
+        p.set_schedule(0, 0)
+        assert (p.struct.chunk, p.struct.scan_k) == (0 if small else want[n_states], 0)
     if n_states in (8193, 12289):
         check_pass(2, 1, [n_states - 1], True, dtype, [None])
 
