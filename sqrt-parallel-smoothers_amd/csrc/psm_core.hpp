@@ -60,12 +60,12 @@ struct SAgg {
 };
 
 // ---------------------------------------------------------------- SoA load / store
-// Component q of item i lives at base[q * stride + i].  The workspace's buffers
-// hold their items in blocks of kBlk positions, the NQ components of a block one
-// after the other (blk): one component of 64 consecutive positions is 64
-// consecutive words, the components of an item lie within one block (a few KB
-// apart at fixed offsets, which fit the instructions' immediate offsets, instead
-// of one far-away stream each), and kBlk is the component stride.
+// The workspace's buffers hold their items in blocks of kBlk positions, the NQ
+// components of a block one after the other: component q of position p lies at
+// blk(base, p)[q * kBlk].  One component of 64 consecutive positions is 64 consecutive
+// words, and the components of an item lie within one block (a few KB apart at
+// fixed offsets, which fit the instructions' immediate offsets, instead of one
+// far-away stream each).
 constexpr int kBlk = 64;
 template <int NQ, typename R>
 PSM_DEV R* blk(R* base, int64_t pos) {
@@ -134,17 +134,6 @@ PSM_DEV void load_obs(const R* base, int64_t pos, Step<R, NX, NY>& s) {
   ld(p, kBlk, 0, q, s.c);
 }
 
-template <typename R, int NX>
-PSM_DEV void load_agg(const R* base, int64_t pos, FAgg<R, NX>& a) {
-  const R* p = blk<FAgg<R, NX>::NQ>(base, pos);
-  int q = 0;
-  ld(p, kBlk, 0, q, a.A);
-  ld(p, kBlk, 0, q, a.b);
-  ld(p, kBlk, 0, q, a.U);
-  ld(p, kBlk, 0, q, a.eta);
-  ld(p, kBlk, 0, q, a.Z);
-  a.flag = (int)p[q * kBlk];
-}
 template <typename R, int NX>
 PSM_DEV void store_agg(R* base, int64_t pos, const FAgg<R, NX>& a) {
   R* p = blk<FAgg<R, NX>::NQ>(base, pos);

@@ -55,7 +55,6 @@ struct Plan {
   int64_t M = 0;
   int64_t Mp = 0;  // padded state count of the per-state buffers
   int chunk = 0;
-  int wg = 0;      // scan workgroup size
   bool team = false;  // 16 lanes per combination above level 0
   int lanes0 = 1;     // lanes per combination at level 0
   int64_t nchunks = 0;
@@ -107,7 +106,6 @@ inline Plan make_plan(const psm_problem_t* p, size_t rsize, int nlin, int nqf, i
   pl.chunk = resolve_chunk(p);
   pl.nchunks = (pl.M + pl.chunk - 1) / pl.chunk;
   pl.Mp = state_stride(pl.M, pl.chunk);
-  pl.wg = wg;
   const int nq = nqf > nqs ? nqf : nqs;
   size_t off = 0;
   pl.off_lin = off;
@@ -392,11 +390,9 @@ struct Impl {
     return hip_check("k_smoother_combine");
   }
 
-  // Exclusive scan of the level-0 aggregates; *final_off receives the workspace
-  // offset of the complete exclusive prefixes.
   static LevelMap level_map(const Plan& pl, int l, int rev) {
     const ScanLevel& s = pl.lv[l];
-    return LevelMap{s.n, s.stride, s.K, s.wg, rev};
+    return LevelMap{s.n, s.K, s.wg, rev};
   }
 
   // FP32 square-root passes launch each kernel twice: without FP64 code and
@@ -464,7 +460,7 @@ struct Impl {
       lv->map[l] = level_map(pl, l, l == 0 ? rev0 : 0);
       const bool top = l + 1 == pl.nlevels;
       R* tot = top ? nullptr : (R*)(ws + pl.lv[l + 1].off_in);
-      const LevelMap tm = top ? LevelMap{0, 0, 1, WG, 0} : level_map(pl, l + 1, 0);
+      const LevelMap tm = top ? LevelMap{0, 1, WG, 0} : level_map(pl, l + 1, 0);
       TimedScope ts_(l == 0 ? (filt ? "k_fscan_up_l0" : "k_sscan_up_l0")
                             : (filt ? "k_fscan_up" : "k_sscan_up"), st);
       // lanes per combination of the kernel this level runs
@@ -560,7 +556,7 @@ struct Impl {
     TimedScope ts_("k_filter_reduce", st);
     launch_fb(fb, g, grid_for(pl.nchunks, kLaneWG), grid_for(pl.nchunks, kLaneWG), [&](auto f) {
       hipLaunchKernelGGL((k_filter_reduce<R, NX, NY, SQRT, decltype(f)>), dim3(grid_for(pl.nchunks, kLaneWG)),
-                         dim3(kLaneWG), 0, st, pl.M, pl.Mp, pl.chunk, pl.nchunks, p->state_offsets,
+                         dim3(kLaneWG), 0, st, pl.M, pl.chunk, pl.nchunks, p->state_offsets,
                          p->n_seq, lin, (const R*)ys, (const R*)m0, (const R*)L0, (const R*)(ws + pl.off_ref),
                          (R*)(ws + pl.lv[0].off_in), level_map(pl, 0, 0), f);
     });
@@ -573,7 +569,7 @@ struct Impl {
     TimedScope ts_("k_filter_apply", st);
     launch_fb(fb, g, grid_for(pl.nchunks, kLaneWG), grid_for(pl.nchunks, kLaneWG), [&](auto f) {
       hipLaunchKernelGGL((k_filter_apply<R, NX, NY, SQRT, decltype(f)>), dim3(grid_for(pl.nchunks, kLaneWG)),
-                         dim3(kLaneWG), 0, st, pl.M, pl.Mp, pl.chunk, pl.nchunks, p->state_offsets,
+                         dim3(kLaneWG), 0, st, pl.M, pl.chunk, pl.nchunks, p->state_offsets,
                          p->n_seq, lin, (const R*)ys, (const R*)m0, (const R*)L0, (const R*)(ws + pl.off_ref),
                          lv, (R*)om, (R*)oL, om_inter, ell_state, f);
     });
@@ -621,7 +617,7 @@ struct Impl {
     TimedScope ts_("k_smoother_reduce", st);
     launch_fb(fb, g, grid_for(pl.nchunks, kLaneWG), grid_for(pl.nchunks, kLaneWG), [&](auto f) {
       hipLaunchKernelGGL((k_smoother_reduce<R, NX, NY, SQRT, decltype(f)>),
-                         dim3(grid_for(pl.nchunks, kLaneWG)), dim3(kLaneWG), 0, st, pl.M, pl.Mp, pl.chunk,
+                         dim3(grid_for(pl.nchunks, kLaneWG)), dim3(kLaneWG), 0, st, pl.M, pl.chunk,
                          pl.nchunks, p->state_offsets, p->n_seq, (const R*)(ws + pl.off_lin), (const R*)fm,
                          (const R*)fL, fm_inter, (const R*)(ws + pl.off_ref), (R*)(ws + pl.off_selem), (R*)(ws + pl.lv[0].off_in),
                          level_map(pl, 0, 1), f);
@@ -634,7 +630,7 @@ struct Impl {
       TimedScope ts_("k_smoother_apply", st);
       launch_fb(fb, g, grid_for(pl.nchunks, kLaneWG), grid_for(pl.nchunks, kLaneWG), [&](auto f) {
         hipLaunchKernelGGL((k_smoother_apply<R, NX, SQRT, decltype(f)>), dim3(grid_for(pl.nchunks, kLaneWG)),
-                           dim3(kLaneWG), 0, st, pl.M, pl.Mp, pl.chunk, pl.nchunks,
+                           dim3(kLaneWG), 0, st, pl.M, pl.chunk, pl.nchunks,
                            (const R*)(ws + pl.off_selem), lv, (const R*)(ws + pl.off_ref), (R*)om, (R*)oL, om_inter, f);
       });
     }
@@ -688,7 +684,7 @@ struct Impl {
     // smoother elements at every state (the chunk aggregates it also forms are not used)
     launch_fb(fb, g, grid_for(pl.nchunks, kLaneWG), grid_for(pl.nchunks, kLaneWG), [&](auto f) {
       hipLaunchKernelGGL((k_smoother_reduce<R, NX, NY, SQRT, decltype(f)>), dim3(grid_for(pl.nchunks, kLaneWG)),
-                         dim3(kLaneWG), 0, st, pl.M, pl.Mp, pl.chunk, pl.nchunks, p->state_offsets,
+                         dim3(kLaneWG), 0, st, pl.M, pl.chunk, pl.nchunks, p->state_offsets,
                          p->n_seq, (const R*)(ws + pl.off_lin), (const R*)fm, (const R*)fL, 0,
                          (const R*)(ws + pl.off_ref), (R*)(ws + pl.off_selem), (R*)(ws + pl.lv[0].off_in), level_map(pl, 0, 1), f);
     });

@@ -77,7 +77,6 @@ inline int64_t state_stride(int64_t M, int C) {
 // them in reverse (rev = 1), chunk c sitting at scan position n - 1 - c.
 struct LevelMap {
   int64_t n;       // items
-  int64_t stride;  // padded item count (multiple of WG K): component stride
   int K;
   int WG;
   int rev;
@@ -165,11 +164,6 @@ PSM_DEV void traj_store(R* __restrict__ m_, R* __restrict__ L_, int inter, int64
     st_aos(L_, i, L);
   }
 }
-
-
-struct Lin {
-  int use_sigma;
-};
 
 // p[0..n) <- v (flag words and counters; a kernel rather than hipMemsetAsync,
 // so that a captured graph replays it like any other launch)
@@ -490,7 +484,7 @@ __global__ __launch_bounds__(kLaneWG) void k_linearize_states(
 // ============================================================================
 template <typename R, int NX, int NY, bool SQRT, typename FB = Fallback>
 __global__ __launch_bounds__(kLaneWG) void k_filter_reduce(
-    int64_t M, int64_t Mp, int chunk, int64_t nchunks, const int64_t* __restrict__ soff, int nseq,
+    int64_t M, int chunk, int64_t nchunks, const int64_t* __restrict__ soff, int nseq,
     const R* __restrict__ lin, const R* __restrict__ ys, const R* __restrict__ m0,
     const R* __restrict__ L0, const R* __restrict__ ref, R* __restrict__ agg, LevelMap lm, FB fb) {
   if (fb.skip()) return;
@@ -726,7 +720,7 @@ PSM_DEV void enter_chunk(int64_t c, const ScanLevels<R>& lv, R (&m)[NX], R (&L)[
 
 template <typename R, int NX, int NY, bool SQRT, typename FB = Fallback>
 __global__ __launch_bounds__(kLaneWG) void k_filter_apply(
-    int64_t M, int64_t Mp, int chunk, int64_t nchunks, const int64_t* __restrict__ soff, int nseq,
+    int64_t M, int chunk, int64_t nchunks, const int64_t* __restrict__ soff, int nseq,
     const R* __restrict__ lin, const R* __restrict__ ys, const R* __restrict__ m0,
     const R* __restrict__ L0, const R* __restrict__ ref, ScanLevels<R> lv, R* __restrict__ out_m,
     R* __restrict__ out_L, int out_inter, typename AccOf<R>::type* __restrict__ ell_state, FB fb) {
@@ -817,7 +811,7 @@ __global__ __launch_bounds__(BS) void k_ell_reduce(const Acc* __restrict__ ell_s
 // ============================================================================
 template <typename R, int NX, int NY, bool SQRT, typename FB = Fallback>
 __global__ __launch_bounds__(kLaneWG) void k_smoother_reduce(
-    int64_t M, int64_t Mp, int chunk, int64_t nchunks, const int64_t* __restrict__ soff, int nseq,
+    int64_t M, int chunk, int64_t nchunks, const int64_t* __restrict__ soff, int nseq,
     const R* __restrict__ lin, const R* __restrict__ fm, const R* __restrict__ fL, int f_inter,
     const R* __restrict__ ref, R* __restrict__ elems, R* __restrict__ agg, LevelMap lm, FB fb) {
   if (fb.skip()) return;
@@ -866,7 +860,7 @@ __global__ __launch_bounds__(kLaneWG) void k_smoother_reduce(
 
 template <typename R, int NX, bool SQRT, typename FB = Fallback>
 __global__ __launch_bounds__(kLaneWG) void k_smoother_apply(
-    int64_t M, int64_t Mp, int chunk, int64_t nchunks, const R* __restrict__ elems,
+    int64_t M, int chunk, int64_t nchunks, const R* __restrict__ elems,
     ScanLevels<R> lv, const R* __restrict__ ref, R* __restrict__ out_m, R* __restrict__ out_L, int out_inter,
     FB fb) {
   if (fb.skip()) return;

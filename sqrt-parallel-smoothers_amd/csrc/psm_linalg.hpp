@@ -21,9 +21,6 @@
 
 namespace psm {
 
-template <typename R> PSM_DEV R rsqrt_(R x);
-template <> PSM_DEV double rsqrt_<double>(double x) { return 1.0 / sqrt(x); }
-template <> PSM_DEV float rsqrt_<float>(float x) { return 1.0f / sqrtf(x); }
 // sqrt for the factorisations' non-negative, finite arguments: the hardware
 // reciprocal square-root estimate, one Goldschmidt step for sqrt(x) and
 // 1 / (2 sqrt(x)), and a final residual correction; it matched the correctly
@@ -88,20 +85,6 @@ PSM_DEV void mmT(const R (&a)[M][K], const R (&b)[N][K], R (&c)[M][N]) {
     }
 }
 
-// c = a^T * b
-template <typename R, int K, int M, int N>
-PSM_DEV void mTm(const R (&a)[K][M], const R (&b)[K][N], R (&c)[M][N]) {
-#pragma unroll
-  for (int i = 0; i < M; ++i)
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      R s = a[0][i] * b[0][j];
-#pragma unroll
-      for (int k = 1; k < K; ++k) s = fma(a[k][i], b[k][j], s);
-      c[i][j] = s;
-    }
-}
-
 template <typename R, int M, int N>
 PSM_DEV void mv(const R (&a)[M][N], const R (&x)[N], R (&y)[M]) {
 #pragma unroll
@@ -110,18 +93,6 @@ PSM_DEV void mv(const R (&a)[M][N], const R (&x)[N], R (&y)[M]) {
 #pragma unroll
     for (int k = 1; k < N; ++k) s = fma(a[i][k], x[k], s);
     y[i] = s;
-  }
-}
-
-// y = a^T x
-template <typename R, int M, int N>
-PSM_DEV void mTv(const R (&a)[M][N], const R (&x)[M], R (&y)[N]) {
-#pragma unroll
-  for (int j = 0; j < N; ++j) {
-    R s = a[0][j] * x[0];
-#pragma unroll
-    for (int k = 1; k < M; ++k) s = fma(a[k][j], x[k], s);
-    y[j] = s;
   }
 }
 
