@@ -51,7 +51,10 @@ struct SampleItem {
       set_zero(eps);
     }
   }
-  // x <- E x [+ g + D eps]; D is a factor, or its covariance
+  // x <- E x [+ g + D eps]; D is a factor, or its covariance.  A sequence's last
+  // factor is the caller's, any square root; the others are lower triangular (their
+  // zeros cost less than a branch on the flag: 16,384 states and 64 samples 173 us,
+  // 189 with one, 161 with the lower triangle alone).
   PSM_DEV void step(bool off, R (&x)[NX]) const {
     R L[NX][NX], y[NX];
     if constexpr (SQRT) copy(a.D, L);
@@ -60,14 +63,7 @@ struct SampleItem {
     for (int i = 0; i < NX; ++i) {
       R s = a.g[i];
 #pragma unroll
-      for (int j = 0; j <= i; ++j) s = fma(L[i][j], eps[j], s);
-      if constexpr (SQRT) {
-        // the last state's is the caller's filtered factor, any square root
-        if (a.flag == FLAG_HEAD) {
-#pragma unroll
-          for (int j = i + 1; j < NX; ++j) s = fma(L[i][j], eps[j], s);
-        }
-      }
+      for (int j = 0; j < (SQRT ? NX : i + 1); ++j) s = fma(L[i][j], eps[j], s);
       y[i] = off ? s : R(0);
 #pragma unroll
       for (int j = 0; j < NX; ++j) y[i] = fma(a.E[i][j], x[j], y[i]);
