@@ -65,8 +65,8 @@ FP32_BAR = 1e-4   # smoothed-mean relative error of the FP32 path the metric req
 PMC_NAMES = {
     "k_fscan_up_l0": "psm::k_scan_up<psm::FAgg<double, 5>, double, true, {wg}>",
     "k_sscan_up_l0": "psm::k_scan_up<psm::SAgg<double, 5>, double, true, {wg}>",
-    "k_fscan_up_l0_quad": "psm::k_scan_up_quad<psm::FAgg<double, 5>, double, {wg}>",
-    "k_sscan_up_l0_quad": "psm::k_scan_up_quad<psm::SAgg<double, 5>, double, {wg}>",
+    "k_fscan_up_l0_quad": "psm::k_scan_up_coop<psm::FAgg<double, 5>, double, true, 4, {wg}>",
+    "k_sscan_up_l0_quad": "psm::k_scan_up_coop<psm::SAgg<double, 5>, double, true, 4, {wg}>",
     "k_filter_reduce": "psm::k_filter_reduce<double, 5, 2, true>",
     "k_filter_apply": "psm::k_filter_apply<double, 5, 2, true>",
     "k_smoother_reduce": "psm::k_smoother_reduce<double, 5, 2, true>",
