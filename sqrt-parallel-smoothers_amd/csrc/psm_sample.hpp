@@ -22,7 +22,7 @@
 //   5. k_sample_apply   lane (chunk, sample): the recursion through the chunk
 // (one chunk takes 5 alone, one group 1, 4 and 5).  With Cs about the cube root of
 // the states the chain is at most 5 Cs steps: T = 16,384 and 64 samples take 144, on
-// 512 x 69 lanes in 1 and 512 x 64 in 5, and 45, 16, 7, 24 and 43 us (one level of 128 chunks, where every sample's lane formed P_c too:
+// 512 x 69 lanes in 1 and 512 x 64 in 5, and 48, 16, 8, 22 and 44 us (one level of 128 chunks, where every sample's lane formed P_c too:
 // 656, 25 and 201 us).  Each lane loads the next item before it uses the current
 // one: kernels 1 and 5 read every element once per column, from cache.  The
 // standard normals eps (n_states, n_samples, nx) are drawn by the caller.
@@ -42,8 +42,10 @@ template <typename R, int NX, bool SQRT>
 struct SampleItem {
   SAgg<R, NX> a;
   R eps[NX];
+  int64_t at;
   PSM_DEV void load(const R* __restrict__ elems, int64_t pos, const R* __restrict__ e) {
     load_agg(elems, pos, a);
+    at = pos;
     if (e != nullptr) {
 #pragma unroll
       for (int i = 0; i < NX; ++i) eps[i] = e[i];
@@ -51,11 +53,11 @@ struct SampleItem {
       set_zero(eps);
     }
   }
-  // x <- E x [+ g + D eps]; D is a factor, or its covariance.  A sequence's last
-  // factor is the caller's, any square root; the others are lower triangular (their
-  // zeros cost less than a branch on the flag: 16,384 states and 64 samples 173 us,
-  // 189 with one, 161 with the lower triangle alone).
-  PSM_DEV void step(bool off, R (&x)[NX]) const {
+  // x <- E x [+ g + D eps]; D is a factor, or its covariance.  The factors are lower
+  // triangular, but for a sequence's last one, which is the caller's: what it has above
+  // the diagonal is loaded there alone (16,384 states and 64 samples: 166 us, 173 with
+  // the whole of every factor).
+  PSM_DEV void step(bool off, const R* __restrict__ elems, R (&x)[NX]) const {
     R L[NX][NX], y[NX];
     if constexpr (SQRT) copy(a.D, L);
     else cholesky(a.D, L);
@@ -63,10 +65,19 @@ struct SampleItem {
     for (int i = 0; i < NX; ++i) {
       R s = a.g[i];
 #pragma unroll
-      for (int j = 0; j < (SQRT ? NX : i + 1); ++j) s = fma(L[i][j], eps[j], s);
+      for (int j = 0; j <= i; ++j) s = fma(L[i][j], eps[j], s);
       y[i] = off ? s : R(0);
 #pragma unroll
       for (int j = 0; j < NX; ++j) y[i] = fma(a.E[i][j], x[j], y[i]);
+    }
+    if constexpr (SQRT) {
+      if (a.flag == FLAG_HEAD && off) {
+        const R* p = blk<SAgg<R, NX>::NQ>(elems, at) + (NX + NX * NX) * kBlk;
+#pragma unroll
+        for (int i = 0; i < NX; ++i)
+#pragma unroll
+          for (int j = i + 1; j < NX; ++j) y[i] = fma(p[(i * NX + j) * kBlk], eps[j], y[i]);
+      }
     }
     copy(y, x);
   }
@@ -109,7 +120,7 @@ __global__ __launch_bounds__(kLaneWG) void k_sample_reduce(
   cur.load(elems, sm(i1 - 1), noise(i1 - 1));
   for (int64_t k = i1 - 1; k >= i0; --k) {
     if (k > i0) next.load(elems, sm(k - 1), noise(k - 1));
-    cur.step(off, x);
+    cur.step(off, elems, x);
     cur = next;
   }
   sample_map_store(c, q, S, x, P, o);
@@ -197,7 +208,7 @@ __global__ __launch_bounds__(kLaneWG) void k_sample_apply(
   cur.load(elems, sm(i1 - 1), eps + ((i1 - 1) * S + s) * NX);
   for (int64_t k = i1 - 1; k >= i0; --k) {
     if (k > i0) next.load(elems, sm(k - 1), eps + ((k - 1) * S + s) * NX);
-    cur.step(true, x);
+    cur.step(true, elems, x);
     R xn[NX];
     copy(x, xn);
     if constexpr (kCentred<R, SQRT>) from_centred(ref, sm(k), xn);
